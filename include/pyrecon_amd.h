@@ -270,6 +270,34 @@ int prh_rsd_update_f32(float *delta, const float *t, const size_t *nmesh, const 
 int prh_rsd_update_f64(double *delta, const double *t, const size_t *nmesh, const double *boxsize,
                        const double *boxcenter, double factor, int a, int b, void *stream);
 
+/* The field-level FFT reconstructions on half spectra (the real meshes' kz <= n2 / 2), in few
+ * passes over memory.  Axes of 2 to 1024 cells with factors 2, 3, 5 and 7; *bytes = 0 from
+ * prh_spectral_scratch says that a shape is outside that, and prh_fft3d_* with prh_spectral_* cover it.
+ * prh_spectral_scratch: bytes of device scratch of one call of a kind.
+ * prh_spectral_iterate_*: one iteration of iterative_fft.py:30-67 with the 1 / (1 + beta) of the
+ *   first one in factor: out = delta - factor * IFFT((k . los)^2 / k^2 FFT(src)) (los), or
+ *   delta - factor * sum_ab x_a x_b / |x|^2 IFFT(k_a k_b / k^2 FFT(src)) (los == NULL, over all
+ *   nine a, b), the real part of numpy's c2c transforms.  out may be src or delta.
+ * prh_spectral_displacements_*: psi_a = IFFT(i k_a / k^2 FFT(delta)) (los == NULL,
+ *   iterative_fft.py:69-82), divided by 1 + beta (k . los)^2 / k^2 in Fourier space with a line of
+ *   sight (plane_parallel_fft.py:41-55).                                                        */
+#define PRH_SPECTRAL_LOCAL 0
+#define PRH_SPECTRAL_GLOBAL 1
+#define PRH_SPECTRAL_DISPLACEMENTS 2
+int prh_spectral_scratch(const size_t *nmesh, int dtype, int kind, size_t *bytes);
+int prh_spectral_iterate_f32(prh_workspace *ws, const float *src, const float *delta, float *out, const size_t *nmesh,
+                             const float *boxsize, const float *boxcenter, const double *los, double factor,
+                             void *scratch, size_t nscratch, void *stream);
+int prh_spectral_iterate_f64(prh_workspace *ws, const double *src, const double *delta, double *out, const size_t *nmesh,
+                             const double *boxsize, const double *boxcenter, const double *los, double factor,
+                             void *scratch, size_t nscratch, void *stream);
+int prh_spectral_displacements_f32(prh_workspace *ws, const float *delta, float *psi0, float *psi1, float *psi2,
+                                   const size_t *nmesh, const float *boxsize, const double *los, double beta,
+                                   void *scratch, size_t nscratch, void *stream);
+int prh_spectral_displacements_f64(prh_workspace *ws, const double *delta, double *psi0, double *psi1, double *psi2,
+                                   const size_t *nmesh, const double *boxsize, const double *los, double beta,
+                                   void *scratch, size_t nscratch, void *stream);
+
 /* Deterministic FP64 sums of one or two meshes (recon.py:227 np.sum calls).
  * sums: host double[2]; synchronizes stream.                               */
 int prh_mesh_sums_f32(prh_workspace *ws, const float *a, const float *b, size_t size,

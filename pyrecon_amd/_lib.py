@@ -33,6 +33,8 @@ TUNE_PAIRED_SWEEPS = 0
 FFT_COMPLEX, FFT_REAL_IN, FFT_REAL_OUT = 0, 1, 2
 SPEC_PLANE_PARALLEL, SPEC_INV_K2, SPEC_LOS_SQ, SPEC_KA_KB, SPEC_GRAD, SPEC_I_KA = 0, 1, 2, 3, 4, 5
 
+SPECTRAL_LOCAL, SPECTRAL_GLOBAL, SPECTRAL_DISPLACEMENTS = 0, 1, 2
+
 WS_MULTIGRID, WS_PAINT, WS_FFT, WS_MIXED = 1, 2, 4, 8
 OP_MUL, OP_DIV, OP_RDIV = 0, 1, 2
 WS_ALL = 15
@@ -105,6 +107,7 @@ def _signatures():
         'prh_synth_points': (_i, [_vp, _vp, _i, _sz, ctypes.c_uint64, _vp, _vp, _vp, _i, _d, _d, _d, _vp]),
         'prh_fmg_mixed_group': (_i, [_vp, _i, _vp, _vp, _szp, _vp, _vp, _vp, _d, _i, _i, _vp, _i, _i, _vp]),
         'prh_residual_norm_f64': (_i, [_vp, _vp, _vp, _szp, _vp, _vp, _d, _vp, ctypes.POINTER(_d), _vp]),
+        'prh_spectral_scratch': (_i, [_szp, _i, _i, _szp]),
         'prh_paint_mixed_f64': (_i, [_vp, _vp, _szp, _vp, _vp, _vp, _i, _vp, _i, _sz, _i, _vp]),
         'prh_fmg_noalloc_f64': (_i, [_vp, _vp, _szp, _vp, _vp, _d, _d, _i, _i, _vp, _vp]),
     }
@@ -130,6 +133,8 @@ def _signatures():
             'prh_mesh_scalar_op_' + suffix: (_i, [_vp, _vp, _sz, _i, _d, _vp]),
             'prh_fft3d_' + suffix: (_i, [_vp, _vp, _vp, _szp, _i, _i, _vp]),
             'prh_spectral_' + suffix: (_i, [_vp, _i, _vp, _vp, _szp, _vp, _vp, _d, _d, _i, _i, _vp]),
+            'prh_spectral_iterate_' + suffix: (_i, [_vp, _vp, _vp, _vp, _szp, _vp, _vp, _vp, _d, _vp, _sz, _vp]),
+            'prh_spectral_displacements_' + suffix: (_i, [_vp, _vp, _vp, _vp, _vp, _szp, _vp, _vp, _d, _vp, _sz, _vp]),
             'prh_rsd_update_' + suffix: (_i, [_vp, _vp, _szp, _vp, _vp, _d, _i, _i, _vp]),
             'prh_read_shifts_' + suffix: (_i, [_vp, _vp, _szp, _vp, _vp, _vp, _i, _sz, _d, _vp, _i, _i, _i,
                                                 _vp, _i, ctypes.POINTER(_i), _vp]),

@@ -20,7 +20,7 @@
 #include <type_traits>
 #include <vector>
 
-#include "prh_workspace.hpp"
+#include "prh_fft.hpp"
 
 namespace prh {
 
@@ -31,16 +31,6 @@ constexpr int kSmoothThreads = 512;
 constexpr int kMaxFly = 2;  // butterflies per thread and pass (held in registers)
 constexpr size_t kSmoothLds = 81920;      // target LDS bytes of a block (2 blocks per CU)
 constexpr size_t kSmoothLdsMax = 163840;  // upper limit (one line per block)
-
-template <typename R>
-struct Cx {
-  R re, im;
-};
-
-template <typename R>
-__device__ __forceinline__ Cx<R> cmul(Cx<R> a, Cx<R> b) {
-  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
 
 // Parameters of one Stockham pass: radix, span Ns of the sub-transforms done
 // so far (a power of two except after a second odd radix), butterflies per

@@ -6,6 +6,8 @@ redshift-space density, with a global line of sight as beta IFFT((k.los)^2 delta
 a local one as beta sum_ij x_i x_j / |x|^2 IFFT(k_i k_j delta_k / k^2) (6 inverse transforms).
 Transforms, Fourier-space operators and the real-space updates run in the HIP library.
 """
+import ctypes
+
 from . import _lib
 from .device import stream_handle
 from .recon import SpectralReconstruction, ReconstructionError, _suffix
@@ -19,12 +21,36 @@ class IterativeFFTReconstruction(SpectralReconstruction):
         if getattr(self, 'mesh_delta', None) is None or self.mesh_delta.buffer is None:
             raise ReconstructionError('set the density contrast before running')
         self._iter = 0
-        self.mesh_delta_real = self.mesh_delta.deepcopy()
+        scratch = self._scratch(_lib.SPECTRAL_LOCAL if self.los is None else _lib.SPECTRAL_GLOBAL,
+                                _lib.SPECTRAL_DISPLACEMENTS)
+        # the half-spectrum iteration reads the current density and writes the next one
+        self.mesh_delta_real = self.mesh_delta if scratch is not None else self.mesh_delta.deepcopy()
         for _ in range(niterations):
-            self._iterate()
+            if scratch is not None: self._iterate_half_spectrum(scratch)
+            else: self._iterate()
         self.mesh_delta = None
-        self.mesh_psi = self._compute_psi()
+        self.mesh_psi = self._half_spectrum_psi(self.mesh_delta_real, scratch) if scratch is not None \
+            else self._compute_psi()
         self.mesh_delta_real = None
+
+    def _factor(self):
+        """beta, reduced in the first iteration (Burden et al. 2015, eq. 12, flat-sky approximation)."""
+        return self.beta / (1. + self.beta) if self._iter == 0 else self.beta
+
+    def _iterate_half_spectrum(self, scratch):
+        """One iteration (iterative_fft.py:30-67) on half spectra."""
+        self.logger.info('Running iteration {:d}.'.format(self._iter))
+        source = self.mesh_delta_real
+        if source is self.mesh_delta: self.mesh_delta_real = self._new_mesh()
+        nm, nm_ptr = _lib.size3(self.info.shape)
+        bs, bs_ptr = _lib.vec3(self.info.boxsize, self.info.dtype)
+        bc, bc_ptr = _lib.vec3(self.info.boxcenter, self.info.dtype)
+        los_arr = None if self.los is None else (ctypes.c_double * 3)(*[float(x) for x in self.los])
+        fn = getattr(_lib.lib, 'prh_spectral_iterate_' + _suffix(self.info.dtype))
+        _lib.check(fn(self.workspace.handle, source.buffer.ptr, self.mesh_delta.buffer.ptr,
+                      self.mesh_delta_real.buffer.ptr, nm_ptr, bs_ptr, bc_ptr, los_arr, float(self._factor()),
+                      scratch.ptr, scratch.nbytes, stream_handle(self.stream)), 'iteration')
+        self._iter += 1
 
     def _rsd_update(self, t, factor, a=-1, b=-1):
         nm, nm_ptr = _lib.size3(self.info.shape)
@@ -46,21 +72,14 @@ class IterativeFFTReconstruction(SpectralReconstruction):
         if self.los is not None:
             self._spectral(_lib.SPEC_LOS_SQ, delta_k, work, norm=norm, los=self.los)
             self._to_real(work, out=t)
-            factor = self.beta
-            if self._iter == 0:
-                # Burden et al. 2015, eq. 12 (flat-sky approximation)
-                factor /= (1. + self.beta)
-            self._rsd_update(t, factor)
+            self._rsd_update(t, self._factor())
         else:
             for i in range(3):
                 for j in range(i, 3):
                     self._spectral(_lib.SPEC_KA_KB, delta_k, work, a=i, b=j, norm=norm)
                     self._to_real(work, out=t)
                     # j > i counted twice for j < i
-                    factor = (1. + (i != j)) * self.beta
-                    if self._iter == 0:
-                        factor /= (1. + self.beta)
-                    self._rsd_update(t, factor, a=i, b=j)
+                    self._rsd_update(t, (1. + (i != j)) * self._factor(), a=i, b=j)
         self._iter += 1
 
     def _compute_psi(self):

@@ -88,21 +88,29 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
             self.mesh_data.smooth_gaussian(self.smoothing_radius)
         self.set_density_contrast(ran_min=self.ran_min, smoothing_radius=self.smoothing_radius)
         self.mesh_data = None
-        delta_k = self._spectrum(self.mesh_delta)
-        self.mesh_delta = None
-        self._spectral(_lib.SPEC_INV_K2, delta_k, delta_k)
+        scratch = self._scratch(_lib.SPECTRAL_DISPLACEMENTS)
+        if scratch is not None:
+            meshes = self._half_spectrum_psi(self.mesh_delta, scratch)
+            self.mesh_delta = None
+        else:
+            delta_k = self._spectrum(self.mesh_delta)
+            self.mesh_delta = None
+            self._spectral(_lib.SPEC_INV_K2, delta_k, delta_k)
+            norm = 1. / self.info.size
+            work = self._complex()
         shifts = np.empty_like(self._positions_rec_data)
         pos, _ = as_device(self._positions_rec_data, stream=self.stream)
-        norm = 1. / self.info.size
-        work = self._complex()
         psis = []
         for iaxis in range(3):
             # no displacement is needed along an axis the line of sight does not touch
             if not return_psi and self.los is not None and self.los[iaxis] == 0:
                 shifts[:, iaxis] = 0.
                 continue
-            self._spectral(_lib.SPEC_I_KA, delta_k, work, a=iaxis, norm=norm)
-            psi = self._to_real(work)
+            if scratch is not None:
+                psi = meshes[iaxis]
+            else:
+                self._spectral(_lib.SPEC_I_KA, delta_k, work, a=iaxis, norm=norm)
+                psi = self._to_real(work)
             shifts[:, iaxis] = psi.read_cic(pos, wrap=True).numpy(stream=self.stream)
             if return_psi: psis.append(psi)
         if self.los is None:

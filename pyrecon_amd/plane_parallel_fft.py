@@ -25,6 +25,11 @@ class PlaneParallelFFTReconstruction(SpectralReconstruction):
         """Compute the Zel'dovich displacement meshes :attr:`mesh_psi` (plane_parallel_fft.py:41-55)."""
         if getattr(self, 'mesh_delta', None) is None or self.mesh_delta.buffer is None:
             raise ReconstructionError('set the density contrast before running')
+        scratch = self._scratch(_lib.SPECTRAL_DISPLACEMENTS)
+        if scratch is not None:
+            self.mesh_psi = self._half_spectrum_psi(self.mesh_delta, scratch, los=self.los, beta=self.beta)
+            self.mesh_delta = None
+            return
         delta_k = self._spectrum(self.mesh_delta)
         self.mesh_delta = None
         norm = 1. / self.info.size

@@ -294,6 +294,29 @@ class SpectralReconstruction(BaseReconstruction):
         self._fft(spectrum, out.buffer, True, _lib.FFT_REAL_OUT)
         return out
 
+    def _scratch(self, *kinds):
+        """Device scratch for half-spectrum calls of the given kinds, or None for a mesh outside what they
+        take (the c2c transforms and operators above cover those)."""
+        nm, nm_ptr = _lib.size3(self.info.shape)
+        nbytes, need = ctypes.c_size_t(), 0
+        for kind in kinds:
+            check(lib.prh_spectral_scratch(nm_ptr, _lib.dtype_code(self.info.dtype), int(kind), ctypes.byref(nbytes)),
+                  'spectral scratch')
+            if not nbytes.value: return None
+            need = max(need, nbytes.value)
+        return DeviceArray((need,), np.uint8, stream=self.stream)
+
+    def _half_spectrum_psi(self, delta, scratch, los=None, beta=0.):
+        """Displacement meshes IFFT(i k_a / k^2 FFT(delta)), over 1 + beta mu^2 in Fourier space with ``los``."""
+        psis = [self._new_mesh() for _ in range(3)]
+        nm, nm_ptr = _lib.size3(self.info.shape)
+        bs, bs_ptr = _lib.vec3(self.info.boxsize, self.info.dtype)
+        los_arr = None if los is None else (ctypes.c_double * 3)(*[float(x) for x in los])
+        fn = getattr(lib, 'prh_spectral_displacements_' + _suffix(self.info.dtype))
+        check(fn(self.workspace.handle, delta.buffer.ptr, *[psi.buffer.ptr for psi in psis], nm_ptr, bs_ptr, los_arr,
+                 float(beta), scratch.ptr, scratch.nbytes, stream_handle(self.stream)), 'displacements')
+        return psis
+
     _FIELDS = {'disp': _lib.FIELD_DISP, 'rsd': _lib.FIELD_RSD, 'disp+rsd': _lib.FIELD_DISP_RSD}
 
     def _check_field(self, field):
