@@ -32,16 +32,19 @@ __device__ __forceinline__ Cx<R> cmul(Cx<R> a, Cx<R> b) {
 constexpr int kLineMax = 1024;
 constexpr int kLinePasses = 10;
 
-// One pass: radix, span ns of the sub-transforms done so far, butterflies m = n / rad of a line,
-// twiddle step, and the multipliers that divide by ns and m (floor(2^32 / d) + 1; exact for the
-// small numerators used here).
+// One pass: radix, span ns of the sub-transforms done so far, butterflies m = n / rad of a line, start
+// of its twiddles, and the multipliers that divide by ns and m (floor(2^32 / d) + 1; exact for the
+// small numerators used here).  The twiddles of a pass, exp(-2 pi i r k / (ns rad)) for r = 1 .. rad - 1,
+// k < ns, lie k first: neighbouring butterflies read neighbouring values.  (One table of the n-th roots
+// read with a stride r n / (ns rad) puts them on a few LDS banks: 646 instead of 523 us for 512-cell
+// rows along z of 512^3 in FP64.)
 struct LinePass {
-  int rad, ns, m, span;
+  int rad, ns, m, tw;
   unsigned div_ns, div_m;
 };
 
 struct LinePlan {
-  int n, npass;
+  int n, npass, ntw;
   LinePass pass[kLinePasses];
 };
 
@@ -224,7 +227,7 @@ struct LineFft {
   __device__ __forceinline__ int slot(int line, int e) const {
     if (ACROSS) return ((e ^ (((e >> 2) ^ (e >> 3)) & 1)) << lw) + line;
     const int i = line * n + e;
-    return i ^ ((i >> 4) & 15);
+    return i ^ ((i >> 4) & 15) ^ ((i >> 3) & 8);
   }
 
   // Butterfly f of this thread.
@@ -285,10 +288,10 @@ struct LineFft {
           int line, j;
           if (!where(P, f, line, j)) continue;
           if (P.ns > 1) {
-            const int step = (j - quotient(j, P.div_ns) * P.ns) * P.span;
+            const Cx<R>* root = tw + P.tw + (j - quotient(j, P.div_ns) * P.ns);
 #pragma unroll
             for (int r = 1; r < RAD; r++) {
-              Cx<R> w = tw[r * step];
+              Cx<R> w = root[(r - 1) * P.ns];
               if (INV) w.im = -w.im;
               v[f * RAD + r] = cmul(v[f * RAD + r], w);
             }
@@ -320,5 +323,47 @@ struct LineFft {
     }
   }
 };
+
+// Threads for a tile of `lines` lines: every pass's butterflies, kFlies a thread, and the elements.
+template <typename R>
+inline int line_threads(const LinePlan& P, int lines) {
+  int need = (lines * P.n + LineTile<R>::held - 1) / LineTile<R>::held;
+  for (int i = 0; i < P.npass; i++) {
+    const int rad = P.pass[i].rad;
+    const int flies = rad >= 5 ? kFlies<R, 5> : rad >= 3 ? kFlies<R, 3> : kFlies<R, 2>;
+    const int t = (lines * P.pass[i].m + flies - 1) / flies;
+    need = t > need ? t : need;
+  }
+  return (need + 63) / 64 * 64;
+}
+
+struct LineCols {
+  int lw, threads;
+  size_t lds;
+};
+
+// Tile of kAcross lines: 128-byte rows, 64-byte ones for lines that would need more than 1024 threads.
+template <typename R>
+LineCols line_cols(const LinePlan& P) {
+  int lw = sizeof(R) == 8 ? 3 : 4;
+  if (line_threads<R>(P, 1 << lw) > 1024) lw--;
+  return {lw, line_threads<R>(P, 1 << lw),
+          sizeof(Cx<R>) * ((static_cast<size_t>(P.n + 1) << lw) + static_cast<size_t>(P.ntw))};
+}
+
+struct LineRows {
+  int nl, threads;
+  size_t lds;
+};
+// Pairs of rows: as many as 256 threads take.  Blocks of a multiple of four wavefronts share the
+// four SIMDs evenly; five pairs of 384 elements on five wavefronts left half of the slots empty
+// (2.2 against 1.35 ms for the six fields of 384^3).
+template <typename R>
+LineRows line_rows(const LinePlan& P) {
+  int nl = 256 * LineTile<R>::held / P.n;
+  if (nl < 1) nl = 1;
+  while (nl > 1 && line_threads<R>(P, nl) > 256) nl--;
+  return {nl, line_threads<R>(P, nl), sizeof(Cx<R>) * (((nl * P.n + 15) & ~15) + static_cast<size_t>(P.ntw))};
+}
 
 }  // namespace prh

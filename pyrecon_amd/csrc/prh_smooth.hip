@@ -12,9 +12,9 @@
 // lines are filtered at once as the real and imaginary parts of one complex
 // line.
 //
-// The 1-D transforms are mixed-radix Stockham FFTs (radix 2, 3, 4, 5, 7) on
-// lines held in LDS, ping-ponging between two buffers; twiddles come from a
-// per-axis table exp(-2 pi i k / n) built on the host in double precision.
+// The 1-D transforms are those of prh_fft.hpp for lines of up to 1024 cells, register forms for some
+// power-of-two lengths, and for longer lines mixed-radix Stockham FFTs (radix 2, 3, 4, 5, 7, 8) in LDS;
+// twiddles come from per-axis tables built on the host in double precision.
 #include <cmath>
 #include <cstdint>
 #include <type_traits>
@@ -25,9 +25,6 @@
 namespace prh {
 
 constexpr int kSmoothThreads = 512;
-#ifndef PRH_SMOOTH_REG512
-#define PRH_SMOOTH_REG512 1
-#endif
 constexpr int kMaxFly = 2;  // butterflies per thread and pass (held in registers)
 constexpr size_t kSmoothLds = 81920;      // target LDS bytes of a block (2 blocks per CU)
 constexpr size_t kSmoothLdsMax = 163840;  // upper limit (one line per block)
@@ -274,6 +271,123 @@ __global__ __launch_bounds__(kSmoothThreads) void k_smooth_axis(
   }
 }
 
+// Lines of up to kLineMax cells (LineFft): forward, gain, inverse in one tile, read and written once.
+// Bound: HBM, with the LDS passes of two transforms close behind.  A smoothing of 256^3 in FP64 takes
+// 0.21 ms (3.8 TB/s) and of 384 x 320 x 448 0.74 ms; the Stockham kernel below, which splits every
+// element's index with 64-bit divisions, took 0.42 and 1.70.
+// kAcross: a complex line is two lines adjacent along z (PAIRED: loaded as one value, which needs an
+// even row length and an aligned mesh); blockIdx.x counts tiles of a plane of `width` lines, blockIdx.y
+// the planes.  Otherwise (z): two rows, `nl` pairs a block.
+template <typename R, bool PAIRED>
+__global__ __launch_bounds__(1024) void k_smooth_across(R* __restrict__ mesh, LinePlan P, int lw, int width,
+                                                        size_t plane, size_t es, const Cx<R>* __restrict__ tw,
+                                                        const R* __restrict__ gain) {
+  extern __shared__ double smem[];
+  const int n = P.n, W = 1 << lw;
+  Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
+  Cx<R>* stw = buf + (n + 1) * W;
+  R* sgain = reinterpret_cast<R*>(stw + P.ntw);
+  for (int k = threadIdx.x; k < P.ntw; k += blockDim.x) stw[k] = tw[k];
+  for (int k = threadIdx.x; k < n; k += blockDim.x) sgain[k] = gain[k];
+  LineFft<R, true> L{buf, stw, n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
+  const int q0 = blockIdx.x * 2 * W;
+  R* base = mesh + blockIdx.y * plane + q0;
+  L.template run<false, false, true>(
+      P,
+      [&](int line, int e) {
+        const int q = q0 + 2 * line;
+        const R* at = base + e * es + 2 * line;
+        if (PAIRED) return q < width ? *reinterpret_cast<const Cx<R>*>(at) : Cx<R>{R(0), R(0)};
+        return Cx<R>{q < width ? at[0] : R(0), q + 1 < width ? at[1] : R(0)};
+      },
+      [](int, int, Cx<R>) {});
+  L.template run<true, false, false>(
+      P,
+      [&](int line, int e) {
+        const Cx<R> v = buf[L.slot(line, e)];
+        const R g = sgain[e];
+        return Cx<R>{v.re * g, v.im * g};
+      },
+      [&](int line, int e, Cx<R> v) {
+        const int q = q0 + 2 * line;
+        R* at = base + e * es + 2 * line;
+        if (PAIRED) {
+          if (q < width) *reinterpret_cast<Cx<R>*>(at) = v;
+        } else {
+          if (q < width) at[0] = v.re;
+          if (q + 1 < width) at[1] = v.im;
+        }
+      });
+}
+
+template <typename R>
+__global__ __launch_bounds__(256) void k_smooth_along(R* __restrict__ mesh, LinePlan P, int nl, long long nrows,
+                                                      const Cx<R>* __restrict__ tw, const R* __restrict__ gain) {
+  extern __shared__ double smem[];
+  const int n = P.n;
+  Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
+  Cx<R>* stw = buf + ((nl * n + 15) & ~15);
+  R* sgain = reinterpret_cast<R*>(stw + P.ntw);
+  for (int k = threadIdx.x; k < P.ntw; k += blockDim.x) stw[k] = tw[k];
+  for (int k = threadIdx.x; k < n; k += blockDim.x) sgain[k] = gain[k];
+  LineFft<R, false> L{buf, stw, n, nl, 0, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
+  const long long row0 = 2LL * blockIdx.x * nl;
+  L.template run<false, false, true>(
+      P,
+      [&](int line, int e) {
+        const long long row = row0 + 2 * line;
+        const R* at = mesh + row * n + e;
+        return Cx<R>{row < nrows ? at[0] : R(0), row + 1 < nrows ? at[n] : R(0)};
+      },
+      [](int, int, Cx<R>) {});
+  L.template run<true, false, false>(
+      P,
+      [&](int line, int e) {
+        const Cx<R> v = buf[L.slot(line, e)];
+        const R g = sgain[e];
+        return Cx<R>{v.re * g, v.im * g};
+      },
+      [&](int line, int e, Cx<R> v) {
+        const long long row = row0 + 2 * line;
+        R* at = mesh + row * n + e;
+        if (row < nrows) at[0] = v.re;
+        if (row + 1 < nrows) at[n] = v.im;
+      });
+}
+
+// One axis of the smoothing through LineFft.
+template <typename R>
+static int smooth_lines(const LinePlan& P, R* mesh, int d, const size_t* n, const Cx<R>* tw, const R* gain,
+                        hipStream_t s) {
+  const auto lds_limit = [](const void* fn, size_t bytes) {
+    if (bytes > 65536)
+      PRH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+    return static_cast<int>(PRH_OK);
+  };
+  if (d == 2) {
+    const LineRows B = line_rows<R>(P);
+    const size_t lds = B.lds + sizeof(R) * P.n;
+    const long long nrows = static_cast<long long>(n[0]) * static_cast<long long>(n[1]);
+    PRH_TRY(lds_limit(reinterpret_cast<const void*>(&k_smooth_along<R>), lds));
+    k_smooth_along<R><<<ceil_div((nrows + 1) / 2, B.nl), B.threads, lds, s>>>(mesh, P, B.nl, nrows, tw, gain);
+  } else {
+    const LineCols B = line_cols<R>(P);
+    const size_t lds = B.lds + sizeof(R) * P.n;
+    const size_t plane = d == 1 ? n[1] * n[2] : 0, es = d == 1 ? n[2] : n[1] * n[2];
+    const int width = static_cast<int>(es);
+    const dim3 grid(ceil_div(es, size_t(2) << B.lw), d == 1 ? static_cast<unsigned>(n[0]) : 1);
+    if (es % 2 == 0 && reinterpret_cast<uintptr_t>(mesh) % sizeof(Cx<R>) == 0) {
+      PRH_TRY(lds_limit(reinterpret_cast<const void*>(&k_smooth_across<R, true>), lds));
+      k_smooth_across<R, true><<<grid, B.threads, lds, s>>>(mesh, P, B.lw, width, plane, es, tw, gain);
+    } else {
+      PRH_TRY(lds_limit(reinterpret_cast<const void*>(&k_smooth_across<R, false>), lds));
+      k_smooth_across<R, false><<<grid, B.threads, lds, s>>>(mesh, P, B.lw, width, plane, es, tw, gain);
+    }
+  }
+  PRH_LAUNCHED();
+  return PRH_OK;
+}
+
 // Lines of 512 cells along z (contiguous), with the transforms in registers:
 // one wavefront per complex line (two real rows), lane L holding elements
 // L + 64 r, r = 0..7.  A 512-point DFT is 8 x 64 and the 64 is 8 x 8:
@@ -398,69 +512,8 @@ __global__ __launch_bounds__(64 * kReg512Waves) void k_smooth_reg512(
   }
 }
 
-// Lines of 512 cells along x or y (stride `es`), transforms as in
-// k_smooth_reg512.  A block takes 16 adjacent real lines (consecutive z, one
-// 128-byte row of FP64 per element index): coalesced loads into an LDS tile
-// [element][line] (row stride 17 against bank conflicts), each of the 8
-// wavefronts reads its complex line (real lines 2w, 2w + 1) into registers,
-// the tile memory then serves as the transposition buffers, and the results
-// go back through the tile to coalesced stores.  Requires I % 16 == 0 and
-// consecutive lines adjacent (istride 1).
 constexpr int kReg512SWaves = 8;
-constexpr int kTileRow = 17;  // LDS row stride of the [element][16 lines] tile
-
-template <typename R>
-__global__ __launch_bounds__(64 * kReg512SWaves) void k_smooth_reg512s(
-    R* __restrict__ mesh, long long nreal, int I, long long ostride, long long es,
-    const Cx<R>* __restrict__ tw_global, const R* __restrict__ gain) {
-  constexpr int NT = 64 * kReg512SWaves;
-  __shared__ Cx<R> stw[512];
-  __shared__ R tile[512 * kTileRow];  // also 8 transposition buffers of 512 Cx<R>
-  static_assert(sizeof(R) * 512 * kTileRow >= sizeof(Cx<R>) * 512 * kReg512SWaves, "tile");
-  for (int k = threadIdx.x; k < 512; k += NT) stw[k] = tw_global[k];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  Cx<R>* xb = reinterpret_cast<Cx<R>*>(tile) + 512 * w;
-  const int c = threadIdx.x & 15, e0 = threadIdx.x >> 4;  // load/store: line c, elements e0 + 32 k
-  const long long ngroups = nreal / 16;
-  for (long long g = blockIdx.x; g < ngroups; g += gridDim.x) {
-    const long long q0 = 16 * g;
-    R* base = mesh + (q0 / I) * ostride + (q0 % I);
-    __syncthreads();  // the tile is free (previous group stored, twiddles staged)
-#pragma unroll 4
-    for (int k = 0; k < 16; k++) {
-      const int e = e0 + 32 * k;
-      tile[e * kTileRow + c] = base[static_cast<long long>(e) * es + c];
-    }
-    __syncthreads();
-    Cx<R> v[8];
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-      const R* t = tile + (lane + 64 * r) * kTileRow + 2 * w;
-      v[r] = {t[0], t[1]};
-    }
-    __syncthreads();  // the tile becomes the transposition buffers
-    fft512_lane(v, xb, stw, lane, false);
-#pragma unroll
-    for (int m2 = 0; m2 < 8; m2++) {
-      const R gg = gain[lane + 64 * m2];
-      v[m2].re *= gg;
-      v[m2].im *= gg;
-    }
-    fft512_lane(v, xb, stw, lane, true);  // ends with a barrier
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-      R* t = tile + (lane + 64 * r) * kTileRow + 2 * w;
-      t[0] = v[r].re;
-      t[1] = v[r].im;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int k = 0; k < 16; k++) {
-      const int e = e0 + 32 * k;
-      base[static_cast<long long>(e) * es + c] = tile[e * kTileRow + c];
-    }
-  }
-}
+constexpr int kTileRow = 17;  // LDS row stride of the [element][16 lines] tile of k_smooth_reg1024s
 
 // Lines of 1024 cells in registers: lane L holds elements L + 64 r, r = 0..15.
 // Forward: one radix-2 step in the lane (a = x_n + x_{n+512}, b = (x_n -
@@ -543,9 +596,13 @@ __global__ __launch_bounds__(64 * kReg512Waves) void k_smooth_reg1024(
   }
 }
 
-// Lines of 1024 cells along x or y, as k_smooth_reg512s: 16 adjacent real
-// lines staged through an LDS tile [element][line] (139 KB in FP64), which
-// then serves as the 8 wavefronts' transposition buffers.
+// Lines of 1024 cells along x or y (stride `es`) in FP64.  A block takes 16
+// adjacent real lines (consecutive z): coalesced loads into an LDS tile
+// [element][line] (row stride 17 against bank conflicts, 139 KB), each of the 8
+// wavefronts reads its complex line (real lines 2w, 2w + 1) into registers, the
+// tile memory then serves as the transposition buffers, and the results go
+// back through the tile to coalesced stores.  Requires I % 16 == 0 and
+// consecutive lines adjacent (istride 1).
 template <typename R>
 __global__ __launch_bounds__(64 * kReg512SWaves) void k_smooth_reg1024s(
     R* __restrict__ mesh, long long nreal, int I, long long ostride, long long es,
@@ -682,16 +739,23 @@ static int launch_dft_axis(const void* src, void* dst, int n, long long nlines, 
 }
 
 // gain[k] = exp(-(r k_phys)^2 / 2) / n with k_phys = 2 pi fftfreq(n, L / n)[k]
-// (numpy's ordering: k < (n - 1) / 2 + 1 -> k, else k - n), in double.
+// (numpy's ordering: k < (n - 1) / 2 + 1 -> k, else k - n), in double, for the three axes at once.
 template <typename R>
-__global__ void k_axis_gain(R* __restrict__ gain, int n, double val, double rad) {
+struct GainArgs {
+  R* gain[3];
+  int n[3];
+  double val[3], rad[3];
+};
+template <typename R>
+__global__ void k_axis_gain(GainArgs<R> A) {
+  const int d = blockIdx.y, n = A.n[d];
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const int f = k < (n - 1) / 2 + 1 ? k : k - n;
   constexpr double twopi = 2 * 3.141592653589793;
-  const double kp = twopi * (static_cast<double>(f) * val);
-  const double a = rad * kp;
-  gain[k] = static_cast<R>(exp(-0.5 * (a * a)) / static_cast<double>(n));
+  const double kp = twopi * (static_cast<double>(f) * A.val[d]);
+  const double a = A.rad[d] * kp;
+  A.gain[d][k] = static_cast<R>(exp(-0.5 * (a * a)) / static_cast<double>(n));
 }
 
 static int ceil_log2(int v) {
@@ -776,11 +840,31 @@ int smooth_setup(prh_workspace* ws) {
       S.tw64[d] = static_cast<double*>(p);
       PRH_HIP(hipMemcpy(S.tw64[d], tw.data(), 2 * sizeof(double) * n, hipMemcpyHostToDevice));
     }
-    if (ws->dtype == PRH_F64) {
-      PRH_HIP(hipMemcpy(S.tw[d], tw.data(), 2 * w * n, hipMemcpyHostToDevice));
-    } else {
-      std::vector<float> tf(tw.begin(), tw.end());
-      PRH_HIP(hipMemcpy(S.tw[d], tf.data(), 2 * w * n, hipMemcpyHostToDevice));
+    const auto upload = [&](void* to, const std::vector<double>& v) -> int {
+      if (ws->dtype == PRH_F64) {
+        PRH_HIP(hipMemcpy(to, v.data(), w * v.size(), hipMemcpyHostToDevice));
+      } else {
+        std::vector<float> vf(v.begin(), v.end());
+        PRH_HIP(hipMemcpy(to, vf.data(), w * vf.size(), hipMemcpyHostToDevice));
+      }
+      return PRH_OK;
+    };
+    PRH_TRY(upload(S.tw[d], tw));
+    LinePlan L;
+    if (line_plan(n, L) && L.ntw > 0) {
+      std::vector<double> pt(2 * static_cast<size_t>(L.ntw));
+      for (int p = 0; p < L.npass; p++) {
+        const LinePass& Q = L.pass[p];
+        for (int r = 1; Q.ns > 1 && r < Q.rad; r++)
+          for (int k = 0; k < Q.ns; k++) {
+            const size_t from = 2 * static_cast<size_t>(r * k * (n / (Q.ns * Q.rad)));
+            const size_t at = 2 * static_cast<size_t>(Q.tw + (r - 1) * Q.ns + k);
+            pt[at] = tw[from];
+            pt[at + 1] = tw[from + 1];
+          }
+      }
+      PRH_TRY(ws_alloc(ws, &S.pass_tw[d], 2 * w * L.ntw));
+      PRH_TRY(upload(S.pass_tw[d], pt));
     }
   }
   return PRH_OK;
@@ -795,6 +879,8 @@ size_t smooth_bytes(const size_t* n, int dtype) {
                         (padded_len(n[d]) + n[d]) * 2 * static_cast<size_t>(dtype) > kSmoothLdsMax ||
                         plan_max_lm(P) > fly_log2();
     if (direct) b += 2 * sizeof(double) * n[d];
+    LinePlan L;
+    if (line_plan(n[d], L)) b += 2 * static_cast<size_t>(dtype) * L.ntw;
   }
   return b;
 }
@@ -824,16 +910,20 @@ static int do_smooth(prh_workspace* ws, R* mesh, const size_t* nmesh, const R* b
   hipStream_t s = as_stream(stream);
   const long long n0 = static_cast<long long>(nmesh[0]), n1 = static_cast<long long>(nmesh[1]),
                   n2 = static_cast<long long>(nmesh[2]);
+  GainArgs<R> G;
+  int longest = 0;
   for (int d = 0; d < 3; d++) {
     // d_i = boxsize / nmesh (float64), val = 1 / (n d) as in numpy.fft.fftfreq; the radius is
     // held in the mesh dtype (mesh.py:664-666)
     const double cell = static_cast<double>(boxsize[d]) / static_cast<double>(static_cast<int>(nmesh[d]));
-    const double val = 1.0 / (static_cast<double>(nmesh[d]) * cell);
-    const double rad = static_cast<double>(static_cast<R>(radius[d]));
-    const int n = static_cast<int>(nmesh[d]);
-    k_axis_gain<R><<<ceil_div(n, 256), 256, 0, s>>>(static_cast<R*>(ws->smooth.gain[d]), n, val, rad);
-    PRH_LAUNCHED();
+    G.val[d] = 1.0 / (static_cast<double>(nmesh[d]) * cell);
+    G.rad[d] = static_cast<double>(static_cast<R>(radius[d]));
+    G.n[d] = static_cast<int>(nmesh[d]);
+    G.gain[d] = static_cast<R*>(ws->smooth.gain[d]);
+    longest = G.n[d] > longest ? G.n[d] : longest;
   }
+  k_axis_gain<R><<<dim3(ceil_div(longest, 256), 3), 256, 0, s>>>(G);
+  PRH_LAUNCHED();
   // axis order z, y, x: the z pass reads whole rows
   for (int d = 2; d >= 0; d--) {
     AxisPlan P;
@@ -862,27 +952,36 @@ static int do_smooth(prh_workspace* ws, R* mesh, const size_t* nmesh, const R* b
                                                  static_cast<const R*>(ws->smooth.gain[d]), s)));
       continue;
     }
+    const Cx<R>* tw = static_cast<const Cx<R>*>(ws->smooth.tw[d]);
+    const R* gain = static_cast<const R*>(ws->smooth.gain[d]);
+    // Which kernel: lines of 512 and 1024 along z stay in registers with one wavefront each, which
+    // needs no index arithmetic (512^3 FP64: 377 against 523 us, FP32 193 against 287; 1024^3: 3.4
+    // against 7.1 ms), and so do lines of 1024 in FP64 across (5.5 and 8.0 against 7.0 and 9.5 ms, where
+    // LineFft's tile leaves one block a CU).  Every other length that LineFft takes goes through it,
+    // 512 across included (527 and 599 us a pass against 543 and 613 for the register form, FP32 311
+    // and 311 against 351 and 386).
+    LinePlan lines;
+    const bool reg = (d == 2 && (n == 512 || n == 1024)) ||
+                     (d != 2 && n == 1024 && sizeof(R) == 8 && I % 16 == 0);
+    if (!reg && line_plan(nmesh[d], lines)) {
+      PRH_TRY(smooth_lines<R>(lines, mesh, d, nmesh, static_cast<const Cx<R>*>(ws->smooth.pass_tw[d]), gain, s));
+      continue;
+    }
     const long long ncomplex = (nreal + 1) / 2;
     const unsigned grid = static_cast<unsigned>((ncomplex + LP - 1) / LP);
     const size_t lds = bytes(llp);
-    const Cx<R>* tw = static_cast<const Cx<R>*>(ws->smooth.tw[d]);
-    const R* gain = static_cast<const R*>(ws->smooth.gain[d]);
     if (lds > 65536) {
       PRH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_smooth_axis<R, true>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
       PRH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_smooth_axis<R, false>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
     }
-    if (d == 2 && n == 1024 && PRH_SMOOTH_REG512) {
+    if (d == 2 && n == 1024) {
       const long long ncx = (nreal + 1) / 2;
       const long long nb = (ncx + kReg512Waves - 1) / kReg512Waves;
       const unsigned g1024 = static_cast<unsigned>(nb < 8192 ? nb : 8192);
       k_smooth_reg1024<R><<<g1024, 64 * kReg512Waves, 0, s>>>(mesh, nreal, tw, gain);
-    } else if (n == 1024 && PRH_SMOOTH_REG512 && I % 16 == 0 && istride == 1) {
-      const long long ngroups = nreal / 16;
-      const unsigned g1024 = static_cast<unsigned>(ngroups < 8192 ? ngroups : 8192);
-      k_smooth_reg1024s<R><<<g1024, 64 * kReg512SWaves, 0, s>>>(mesh, nreal, I, ostride, es, tw, gain);
-    } else if (d == 2 && n == 512 && PRH_SMOOTH_REG512) {
+    } else if (d == 2 && n == 512) {
       const long long ncx = (nreal + 1) / 2;
       const long long nb = (ncx + kReg512Waves - 1) / kReg512Waves;
       const unsigned g512 = static_cast<unsigned>(nb < 8192 ? nb : 8192);
@@ -890,14 +989,16 @@ static int do_smooth(prh_workspace* ws, R* mesh, const size_t* nmesh, const R* b
     } else if (d == 2) {
       k_smooth_axis<R, true><<<grid, kSmoothThreads, lds, s>>>(mesh, P, nreal, I, ostride, istride,
                                                                es, llp, tw, gain);
-    } else if (n == 512 && PRH_SMOOTH_REG512 && I % 16 == 0 && istride == 1) {
-      const long long ngroups = nreal / 16;
-      const unsigned g512 = static_cast<unsigned>(ngroups < 8192 ? ngroups : 8192);
-      k_smooth_reg512s<R><<<g512, 64 * kReg512SWaves, 0, s>>>(mesh, nreal, I, ostride, es, tw, gain);
-    }
-    else
+    } else if (reg) {
+      if constexpr (sizeof(R) == 8) {
+        const long long ngroups = nreal / 16;
+        const unsigned g1024 = static_cast<unsigned>(ngroups < 8192 ? ngroups : 8192);
+        k_smooth_reg1024s<R><<<g1024, 64 * kReg512SWaves, 0, s>>>(mesh, nreal, I, ostride, es, tw, gain);
+      }
+    } else {
       k_smooth_axis<R, false><<<grid, kSmoothThreads, lds, s>>>(mesh, P, nreal, I, ostride,
                                                                 istride, es, llp, tw, gain);
+    }
     PRH_LAUNCHED();
   }
   return PRH_OK;

@@ -54,6 +54,7 @@ bool line_plan(size_t n, LinePlan& P) {
   if (nr > kLinePasses) return false;
   P.n = static_cast<int>(n);
   P.npass = nr;
+  P.ntw = 0;
   auto magic = [](int d) { return d > 1 ? static_cast<unsigned>((1ULL << 32) / d + 1) : 0u; };
   int ns = 1;
   for (int i = 0; i < nr; i++) {
@@ -61,7 +62,8 @@ bool line_plan(size_t n, LinePlan& P) {
     S.rad = rads[i];
     S.ns = ns;
     S.m = P.n / S.rad;
-    S.span = P.n / (ns * S.rad);
+    S.tw = P.ntw;
+    if (ns > 1) P.ntw += (S.rad - 1) * ns;
     S.div_ns = magic(ns);
     S.div_m = magic(S.m);
     ns *= S.rad;
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(1024) void k_rows_forward(const R* __restrict__ mes
   Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
   const int n = P.n;
   const int held = (nl * n + 15) & ~15;
-  LineFft<R, false> L{buf, stage_twiddles(buf + held, tw, n), n, nl, 0, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
+  LineFft<R, false> L{buf, stage_twiddles(buf + held, tw, P.ntw), n, nl, 0, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
   const int pair0 = blockIdx.x * nl;
   L.template run<false, false, true>(
       P,
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
   Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
   const int n = P.n;
   const int held = (nl * n + 15) & ~15;
-  LineFft<R, false> L{buf, stage_twiddles(buf + held, tw, n), n, nl, 0, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
+  LineFft<R, false> L{buf, stage_twiddles(buf + held, tw, P.ntw), n, nl, 0, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
   const int pair0 = blockIdx.x * nl;
   constexpr int NF = MODE == kRowsMinusLocal ? kTerms : 1;
   constexpr int kSum = MODE == kRowsMinusLocal ? LineTile<R>::held : 1;
@@ -302,7 +304,7 @@ __global__ __launch_bounds__(1024) void k_columns(Cx<R>* s0, Cx<R>* s1, Cx<R>* s
   Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
   const int n = P.n;
   const int W = 1 << lw;
-  LineFft<R, true> L{buf, stage_twiddles(buf + (n + 1) * W, tw, n), n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
+  LineFft<R, true> L{buf, stage_twiddles(buf + (n + 1) * W, tw, P.ntw), n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
   Cx<R>* spec = blockIdx.y == 0 ? s0 : blockIdx.y == 1 ? s1 : s2;
   Cx<R>* base = spec + static_cast<size_t>(blockIdx.z) * n * pitch + blockIdx.x * W;
   L.template run<INV, false, false>(
@@ -326,7 +328,7 @@ __global__ __launch_bounds__(1024) void k_columns_local(const Cx<R>* __restrict_
   Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
   const int n = P.n;
   const int W = 1 << lw;
-  LineFft<R, true> L{buf, stage_twiddles(buf + (n + 1) * W, tw, n), n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
+  LineFft<R, true> L{buf, stage_twiddles(buf + (n + 1) * W, tw, P.ntw), n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
   const int power = blockIdx.y, ix = plane0 + blockIdx.z, kz0 = blockIdx.x * W;
   const size_t row = static_cast<size_t>(S.pitch);
   const Cx<R>* in = (power == 0 ? x0 : power == 1 ? x1 : x2) + static_cast<size_t>(ix) * n * row + kz0;
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(1024) void k_pencils(const Cx<R>* spec, Cx<R>* out0
   Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
   const int n = P.n;
   const int W = 1 << lw;
-  LineFft<R, true> L{buf, stage_twiddles(buf + (n + 1) * W, tw, n), n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
+  LineFft<R, true> L{buf, stage_twiddles(buf + (n + 1) * W, tw, P.ntw), n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
   const int iy = blockIdx.y, kz0 = blockIdx.x * W;
   const size_t es = static_cast<size_t>(S.n[1]) * S.pitch;
   const size_t base = static_cast<size_t>(iy) * S.pitch + kz0;
@@ -532,48 +534,6 @@ int allow_lds(K kernel, size_t bytes) {
   return PRH_OK;
 }
 
-// Threads for a tile of `lines` lines: every pass's butterflies, kFlies a thread, and the elements.
-template <typename R>
-int line_threads(const LinePlan& P, int lines) {
-  int need = (lines * P.n + LineTile<R>::held - 1) / LineTile<R>::held;
-  for (int i = 0; i < P.npass; i++) {
-    const int rad = P.pass[i].rad;
-    const int flies = rad >= 5 ? kFlies<R, 5> : rad >= 3 ? kFlies<R, 3> : kFlies<R, 2>;
-    const int t = (lines * P.pass[i].m + flies - 1) / flies;
-    need = t > need ? t : need;
-  }
-  return (need + 63) / 64 * 64;
-}
-
-struct Tile {
-  int lw, threads;
-  size_t lds;
-};
-
-// Tile of kAcross lines: 128-byte rows, 64-byte ones for lines that would need more than 1024 threads.
-template <typename R>
-Tile across_tile(const LinePlan& P) {
-  int lw = sizeof(R) == 8 ? 3 : 4;
-  if (line_threads<R>(P, 1 << lw) > 1024) lw--;
-  return {lw, line_threads<R>(P, 1 << lw),
-          sizeof(Cx<R>) * ((static_cast<size_t>(P.n + 1) << lw) + static_cast<size_t>(P.n))};
-}
-
-struct Rows {
-  int nl, threads;
-  size_t lds;
-};
-// Pairs of rows: as many as 256 threads take.  Blocks of a multiple of four wavefronts share the
-// four SIMDs evenly; five pairs of 384 elements on five wavefronts left half of the slots empty
-// (2.2 against 1.35 ms for the six fields of 384^3).
-template <typename R>
-Rows rows_block(const LinePlan& P) {
-  int nl = 256 * LineTile<R>::held / P.n;
-  if (nl < 1) nl = 1;
-  while (nl > 1 && line_threads<R>(P, nl) > 256) nl--;
-  return {nl, line_threads<R>(P, nl), sizeof(Cx<R>) * (((nl * P.n + 15) & ~15) + static_cast<size_t>(P.n))};
-}
-
 unsigned magic_of(int d) { return d > 1 ? static_cast<unsigned>((1ULL << 32) / d + 1) : 0u; }
 
 template <typename R>
@@ -582,7 +542,7 @@ struct Call {
   Layout L;
   SpecShape S;
   hipStream_t s;
-  const Cx<R>* tw(int d) const { return static_cast<const Cx<R>*>(ws->smooth.tw[d]); }
+  const Cx<R>* tw(int d) const { return static_cast<const Cx<R>*>(ws->smooth.pass_tw[d]); }
 
   // a launch that moves `meshes` half spectra (or real meshes), under the transform timer
   template <class F>
@@ -598,7 +558,7 @@ struct Call {
   // mesh -> half spectrum, transformed along z and y
   int forward_zy(const R* mesh, Cx<R>* spec) const {
     PRH_TRY(timed(2, [&]() {
-      const Rows B = rows_block<R>(L.P[2]);
+      const LineRows B = line_rows<R>(L.P[2]);
       const int nrows = S.n[0] * S.n[1];
       auto* k = &k_rows_forward<R>;
       PRH_TRY(allow_lds(k, B.lds));
@@ -612,7 +572,7 @@ struct Call {
   template <bool INV>
   int columns(int count, Cx<R>* s0, Cx<R>* s1, Cx<R>* s2) const {
     return timed(2. * count, [&]() {
-      const Tile B = across_tile<R>(L.P[1]);
+      const LineCols B = line_cols<R>(L.P[1]);
       const dim3 grid(S.pitch >> B.lw, count, S.n[0]);
       auto* k = &k_columns<R, INV>;
       PRH_TRY(allow_lds(k, B.lds));
@@ -624,7 +584,7 @@ struct Call {
   template <int MODE>
   int pencils(const Cx<R>* spec, Cx<R>* o0, Cx<R>* o1, Cx<R>* o2, Cx<R>* edge_y, Cx<R>* edge_z) const {
     return timed(MODE == kXGlobal ? 2 : 4, [&]() {
-      const Tile B = across_tile<R>(L.P[0]);
+      const LineCols B = line_cols<R>(L.P[0]);
       const dim3 grid(S.pitch >> B.lw, S.n[1]);
       auto* k = &k_pencils<R, MODE>;
       PRH_TRY(allow_lds(k, B.lds));
@@ -638,7 +598,7 @@ struct Call {
     const double part = static_cast<double>(A.nrows) / (static_cast<double>(S.n[0]) * S.n[1]);
     const double meshes = MODE == kRowsStore ? 2. * fields : MODE == kRowsMinus ? 3. : kTerms + 2.;
     return timed(meshes * part, [&]() {
-      const Rows B = rows_block<R>(L.P[2]);
+      const LineRows B = line_rows<R>(L.P[2]);
       auto* k = &k_rows_inverse<R, MODE>;
       PRH_TRY(allow_lds(k, B.lds));
       const dim3 grid(ceil_div((A.nrows + 1) / 2, B.nl), MODE == kRowsStore ? fields : 1);
@@ -724,7 +684,7 @@ int do_iterate(prh_workspace* ws, const R* src, const R* delta, R* out, const si
   for (int x0 = 0; x0 < S.n[0]; x0 += L.slab) {
     const int px = S.n[0] - x0 < L.slab ? S.n[0] - x0 : L.slab;
     PRH_TRY(C.timed((3. + kTerms) * px / S.n[0], [&]() {
-      const Tile B = across_tile<R>(L.P[1]);
+      const LineCols B = line_cols<R>(L.P[1]);
       const dim3 grid(S.pitch >> B.lw, 3, px);
       auto* k = &k_columns_local<R>;
       PRH_TRY(allow_lds(k, B.lds));

@@ -99,6 +99,7 @@ struct SmoothState {
   bool have = false;  // false when a dimension is longer than the direct transform allows
   bool direct[3] = {};  // axis transformed by the direct DFT (a prime factor > 7, or too long for the radix passes)
   void* tw[3] = {};
+  void* pass_tw[3] = {};  // the same roots in the order of the passes of LinePlan (axes that have one)
   void* gain[3] = {};
   double* tw64[3] = {};  // exp(-2 pi i k / n), k < n, in double (direct DFT axes)
 };
