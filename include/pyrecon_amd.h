@@ -424,6 +424,46 @@ int prh_shift_algebra_f64(const void *positions, int pos_dtype, const void *s0, 
                           size_t npositions, double f, const double *los, int field, int shifted, void *out,
                           int out_dtype, void *stream);
 
+/* The three displacement meshes of an FFT reconstruction read by CIC at n positions in one pass:
+ * field PRH_FIELD_VALUE gives the (N, 3) displacements in the positions dtype (RealMesh.read_cic,
+ * mesh.py:570-610, of each mesh; wrap as there), the others the shifts or, with shifted, the shifted
+ * positions of prh_shift_algebra_* (wrap 0).  Status and nonfinite as prh_read_shifts_*.        */
+int prh_read_psi_f32(prh_workspace *ws, const float *psi0, const float *psi1, const float *psi2, const size_t *nmesh,
+                     const float *boxsize, const float *boxcenter, const void *positions, int pos_dtype,
+                     size_t npositions, double f, const float *los, int field, int wrap, int shifted, void *out,
+                     int out_dtype, int *nonfinite, void *stream);
+int prh_read_psi_f64(prh_workspace *ws, const double *psi0, const double *psi1, const double *psi2, const size_t *nmesh,
+                     const double *boxsize, const double *boxcenter, const void *positions, int pos_dtype,
+                     size_t npositions, double f, const double *los, int field, int wrap, int shifted, void *out,
+                     int out_dtype, int *nonfinite, void *stream);
+
+/* Per-point algebra in the positions dtype, with numpy's expressions and order, for reads that wrap
+ * positions first (recon.py:255-325 with wrap) and for the particle reconstruction
+ * (iterative_fft_particle.py:104-239).  Arrays are (n, 3); with l the line of sight (x / |x| if local,
+ * else los), rsd = f (s . l) l and component d of s taken as 0 where bit d of skip is set:
+ *   PRH_POINT_WRAP      out = (x - offset) % boxsize + offset
+ *   PRH_POINT_ITERATE   s -= first (s . l) l if first != 0; out = x - f (s . l) l
+ *   PRH_POINT_REAL      out = x - rsd
+ *   PRH_POINT_SHIFT     h = s, rsd or s + rsd (field); out = h, or a - h if shifted (wrapped if wrap)
+ *   PRH_POINT_PARTICLE  the same with h = t + rsd for PRH_FIELD_DISP_RSD
+ *   PRH_POINT_DATA      h = s, x - a or s + (x - a); out = h, or x - h if shifted (wrapped if wrap)
+ * *outside (host, ITERATE and REAL, may be NULL; reading it synchronizes): some out - offset lies
+ * below 0 or above top.  ws holds the status flags.                                              */
+#define PRH_POINT_WRAP 0
+#define PRH_POINT_ITERATE 1
+#define PRH_POINT_REAL 2
+#define PRH_POINT_SHIFT 3
+#define PRH_POINT_PARTICLE 4
+#define PRH_POINT_DATA 5
+typedef struct {
+  double f, first, los[3], offset[3], boxsize[3], top[3];
+  int local, field, shifted, wrap, skip;
+} prh_point_args;
+int prh_point_algebra_f32(prh_workspace *ws, int op, const float *x, const float *a, const float *s, const float *t,
+                          size_t n, const prh_point_args *args, float *out, int *outside, void *stream);
+int prh_point_algebra_f64(prh_workspace *ws, int op, const double *x, const double *a, const double *s, const double *t,
+                          size_t n, const prh_point_args *args, double *out, int *outside, void *stream);
+
 /* Mixed-precision solve (no reference counterpart; same contract as
  * prh_fmg_f64, which it tracks).  The coarse stages of the full multigrid
  * (levels below the finest) run in FP32; the vcycle_niterations

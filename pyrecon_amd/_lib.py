@@ -33,6 +33,7 @@ TUNE_PAIRED_SWEEPS = 0
 FFT_COMPLEX, FFT_REAL_IN, FFT_REAL_OUT = 0, 1, 2
 SPEC_PLANE_PARALLEL, SPEC_INV_K2, SPEC_LOS_SQ, SPEC_KA_KB, SPEC_GRAD, SPEC_I_KA = 0, 1, 2, 3, 4, 5
 
+POINT_WRAP, POINT_ITERATE, POINT_REAL, POINT_SHIFT, POINT_PARTICLE, POINT_DATA = 0, 1, 2, 3, 4, 5
 SPECTRAL_LOCAL, SPECTRAL_GLOBAL, SPECTRAL_DISPLACEMENTS = 0, 1, 2
 
 WS_MULTIGRID, WS_PAINT, WS_FFT, WS_MIXED = 1, 2, 4, 8
@@ -61,6 +62,12 @@ _i = ctypes.c_int
 _d = ctypes.c_double
 _f = ctypes.c_float
 _szp = ctypes.POINTER(ctypes.c_size_t)
+
+
+class PointArgs(ctypes.Structure):
+    """prh_point_args."""
+    _fields_ = [('f', _d), ('first', _d), ('los', _d * 3), ('offset', _d * 3), ('boxsize', _d * 3), ('top', _d * 3),
+                ('local', _i), ('field', _i), ('shifted', _i), ('wrap', _i), ('skip', _i)]
 
 
 def _signatures():
@@ -135,6 +142,10 @@ def _signatures():
             'prh_spectral_' + suffix: (_i, [_vp, _i, _vp, _vp, _szp, _vp, _vp, _d, _d, _i, _i, _vp]),
             'prh_spectral_iterate_' + suffix: (_i, [_vp, _vp, _vp, _vp, _szp, _vp, _vp, _vp, _d, _vp, _sz, _vp]),
             'prh_spectral_displacements_' + suffix: (_i, [_vp, _vp, _vp, _vp, _vp, _szp, _vp, _vp, _d, _vp, _sz, _vp]),
+            'prh_read_psi_' + suffix: (_i, [_vp, _vp, _vp, _vp, _szp, _vp, _vp, _vp, _i, _sz, _d, _vp, _i, _i, _i,
+                                            _vp, _i, ctypes.POINTER(_i), _vp]),
+            'prh_point_algebra_' + suffix: (_i, [_vp, _i, _vp, _vp, _vp, _vp, _sz, ctypes.POINTER(PointArgs), _vp,
+                                                 ctypes.POINTER(_i), _vp]),
             'prh_rsd_update_' + suffix: (_i, [_vp, _vp, _szp, _vp, _vp, _d, _i, _i, _vp]),
             'prh_read_shifts_' + suffix: (_i, [_vp, _vp, _szp, _vp, _vp, _vp, _i, _sz, _d, _vp, _i, _i, _i,
                                                 _vp, _i, ctypes.POINTER(_i), _vp]),

@@ -1503,6 +1503,38 @@ __global__ __launch_bounds__(kCicThreads) void k_read_sorted(const R* __restrict
   flag_errors(err, misc);
 }
 
+// The three displacement meshes of an FFT reconstruction read by CIC at each point at once: one base
+// cell, one set of weights and one read of the position for the three.  The displacement itself
+// (PRH_FIELD_VALUE), or the shift or shifted position it gives, as the fused reads above.  `order`:
+// the points' binned order, or null.  Bound: the 24 mesh values of
+// a point from L2 and the scattered results.  4e6 + 2e7 points at 384^3 in FP64: 4.1 ms as three reads
+// and the algebra apart, 2.3 together.
+template <typename R, typename P, typename O>
+__global__ __launch_bounds__(kCicThreads) void k_read_psi(const R* __restrict__ psi0, const R* __restrict__ psi1,
+                                                          const R* __restrict__ psi2, ReadArgs<R> A,
+                                                          const P* __restrict__ pos, size_t m, O* __restrict__ out,
+                                                          uint32_t* __restrict__ misc,
+                                                          const uint32_t* __restrict__ order) {
+  const size_t t = blockIdx.x * static_cast<size_t>(kCicThreads) + threadIdx.x;
+  uint32_t err = 0;
+  if (t < m) {
+    const size_t i = order ? order[t] : t;
+    const Frame<R>& F = A.F;
+    const P x[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
+    R p[3];
+    to_mesh_units<R, P>(x, F, A.wrap, p, err);
+    const P s[3] = {static_cast<P>(cic_value(psi0, F.n[0], F.n[1], F.n[2], p)),
+                    static_cast<P>(cic_value(psi1, F.n[0], F.n[1], F.n[2], p)),
+                    static_cast<P>(cic_value(psi2, F.n[0], F.n[1], F.n[2], p))};
+    if (A.field == PRH_FIELD_VALUE) {
+      for (int d = 0; d < 3; d++) out[3 * i + d] = static_cast<O>(s[d]);
+    } else {
+      shift_out<R, P, O>(i, x, s, A, A.field, A.shifted, A.local, 0, out);
+    }
+  }
+  flag_errors(err, misc);
+}
+
 // The painted positions tile by tile (one workgroup per tile of the tile
 // paint, tiles dealt to the XCDs in contiguous ranges): the tile's potential is
 // staged in LDS once and each point's 32 mesh reads come from there; results
@@ -2040,6 +2072,42 @@ static int do_read_fd(const R* mesh, const size_t* nmesh, const R* boxsize, cons
   return PRH_OK;
 }
 
+// Bins the points by 8^3 tile (a counting sort, in chunks of the paint scratch) and calls
+// read(offset, count, order) for each chunk.  The order lies in the paint's point-order payload, and is
+// kept for later reads of the same positions when one chunk holds them all.
+template <typename R, typename P, class Read>
+static int read_in_bins(prh_workspace* ws, const ReadArgs<R>& A, const P* pos, size_t n, hipStream_t s, Read&& read) {
+  const Frame<R>& F = A.F;
+  PaintScratch& S = ws->paint;
+  uint32_t* order = static_cast<uint32_t*>(S.payload);
+  S.bins = PaintScratch::Bins();
+  const int t0 = (F.n[0] + kRT - 1) / kRT, t1 = (F.n[1] + kRT - 1) / kRT, t2 = (F.n[2] + kRT - 1) / kRT;
+  const size_t ntile = static_cast<size_t>(t0) * t1 * t2;
+  const unsigned nscan = ceil_div(ntile, kScanBlock);
+  if (n <= S.chunk) {
+    S.bins.pos = pos;
+    S.bins.n = n;
+    S.bins.pdt = Tag<P>::code;
+  }
+  for (size_t o = 0; o < n; o += S.chunk) {
+    const size_t m = n - o < S.chunk ? n - o : S.chunk;
+    const unsigned grid = ceil_div(m, kCicThreads);
+    k_bin_key<R, P><<<grid, kCicThreads, 0, s>>>(pos + 3 * o, m, F, A.wrap, t1, t2, S.key, S.rank, S.count);
+    PRH_LAUNCHED();
+    k_scan_reduce<<<nscan, kCicThreads, 0, s>>>(S.count, ntile, S.partial);
+    PRH_LAUNCHED();
+    k_scan_partials<<<1, kCicThreads, 0, s>>>(S.partial, static_cast<int>(nscan));
+    PRH_LAUNCHED();
+    k_scan_final<<<nscan, kCicThreads, 0, s>>>(S.count, ntile, S.partial, S.start);
+    PRH_LAUNCHED();
+    k_group_scatter<<<grid, kCicThreads, 0, s>>>(S.key, S.rank, m, S.start, order);
+    PRH_LAUNCHED();
+    read(o, m, order);
+    PRH_LAUNCHED();
+  }
+  return PRH_OK;
+}
+
 // Shifts of n points.  With a workspace holding paint scratch for this mesh,
 // the points are binned by 8^3 tile (a counting sort, in chunks of the paint
 // scratch size) and read in binned order; otherwise in input order.
@@ -2129,36 +2197,43 @@ static int read_shifts_all(prh_workspace* ws, const R* phi, const ReadArgs<R>& A
     PRH_LAUNCHED();
     return PRH_OK;
   }
-  S.bins = PaintScratch::Bins();
-  const int t0 = (F.n[0] + kRT - 1) / kRT, t1 = (F.n[1] + kRT - 1) / kRT, t2 = (F.n[2] + kRT - 1) / kRT;
-  const size_t ntile = static_cast<size_t>(t0) * t1 * t2;
-  const unsigned nscan = ceil_div(ntile, kScanBlock);
-  if (n <= S.chunk) {
-    S.bins.pos = pos;
-    S.bins.n = n;
-    S.bins.pdt = Tag<P>::code;
-  }
-  for (size_t o = 0; o < n; o += S.chunk) {
-    const size_t m = n - o < S.chunk ? n - o : S.chunk;
-    const unsigned grid = ceil_div(m, kCicThreads);
-    k_bin_key<R, P><<<grid, kCicThreads, 0, s>>>(pos + 3 * o, m, F, A.wrap, t1, t2, S.key, S.rank, S.count);
-    PRH_LAUNCHED();
-    k_scan_reduce<<<nscan, kCicThreads, 0, s>>>(S.count, ntile, S.partial);
-    PRH_LAUNCHED();
-    k_scan_partials<<<1, kCicThreads, 0, s>>>(S.partial, static_cast<int>(nscan));
-    PRH_LAUNCHED();
-    k_scan_final<<<nscan, kCicThreads, 0, s>>>(S.count, ntile, S.partial, S.start);
-    PRH_LAUNCHED();
-    k_group_scatter<<<grid, kCicThreads, 0, s>>>(S.key, S.rank, m, S.start, order);
-    PRH_LAUNCHED();
+  return read_in_bins<R, P>(ws, A, pos, n, s, [&](size_t o, size_t m, const uint32_t* bins) {
     timer_before(PRH_TIMER_READ_SHIFTS, s);
-    k_read_binned<R, P, O><<<grid, kCicThreads, 0, s>>>(phi, A, pos + 3 * o, m, out + ostride * o,
-                                                        misc, order);
+    k_read_binned<R, P, O><<<ceil_div(m, kCicThreads), kCicThreads, 0, s>>>(phi, A, pos + 3 * o, m,
+                                                                            out + ostride * o, misc, bins);
     timer_after(PRH_TIMER_READ_SHIFTS, s,
                 static_cast<double>(m) * (3 * sizeof(P) + ostride * sizeof(O)) +
                     static_cast<double>(F.n[0]) * F.n[1] * F.n[2] * sizeof(R));
-    PRH_LAUNCHED();
+  });
+}
+
+// The three meshes of k_read_psi, the points visited as read_shifts_all visits them.
+template <typename R, typename P, typename O>
+static int read_psi_all(prh_workspace* ws, const R* const* psi, const ReadArgs<R>& A, const P* pos, size_t n,
+                        O* out, uint32_t* misc, hipStream_t s) {
+  const Frame<R>& F = A.F;
+  const auto read = [&](size_t o, size_t m, const uint32_t* order) {
+    timer_before(PRH_TIMER_READ_SHIFTS, s);
+    k_read_psi<R, P, O><<<ceil_div(m, kCicThreads), kCicThreads, 0, s>>>(psi[0], psi[1], psi[2], A, pos + 3 * o, m,
+                                                                         out + 3 * o, misc, order);
+    timer_after(PRH_TIMER_READ_SHIFTS, s,
+                static_cast<double>(m) * 3 * (sizeof(P) + sizeof(O)) +
+                    3. * F.n[0] * F.n[1] * F.n[2] * sizeof(R));
+  };
+  const bool binned = (ws->flags & PRH_WS_PAINT) && n >= 65536 && ws->n[0] == size_t(F.n[0]) &&
+                      ws->n[1] == size_t(F.n[1]) && ws->n[2] == size_t(F.n[2]);
+  const uint32_t* order = nullptr;
+  if (binned) {
+    PaintScratch& S = ws->paint;
+    auto covers = [&](const auto& o) {
+      return o.pos == static_cast<const void*>(pos) && o.n == n && o.pdt == Tag<P>::code;
+    };
+    order = covers(S.order) ? S.sorted : covers(S.order_prev) ? S.sorted_prev
+            : n <= S.chunk && covers(S.bins) ? static_cast<const uint32_t*>(S.payload) : nullptr;
+    if (!order) return read_in_bins<R, P>(ws, A, pos, n, s, read);
   }
+  read(0, n, order);
+  PRH_LAUNCHED();
   return PRH_OK;
 }
 
@@ -2219,6 +2294,207 @@ static int do_shift_algebra(const void* pos, int pdt, const void* s0, const void
   return PRH_OK;
 }
 
+// The status flags of a read: out-of-box positions (an error without wrap) and non-finite ones.
+static int read_status(prh_workspace* ws, int wrap, int* nonfinite, hipStream_t s) {
+  uint32_t* host = ws->flag_host;
+  PRH_HIP(hipMemcpyAsync(host, ws->misc, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  PRH_HIP(hipStreamSynchronize(s));
+  if (nonfinite && (host[0] & kErrNonFinite)) *nonfinite = 1;
+  if (!wrap && (host[0] & kErrRange)) {
+    set_error("positions not in box range");
+    return PRH_ERR_RANGE;
+  }
+  return PRH_OK;
+}
+
+// ---- per-point algebra of the reads that wrap positions first, and of the particle reconstruction ----
+// numpy's expressions in the positions dtype P, in numpy's order (pyrecon/recon.py:255-325,
+// pyrecon/iterative_fft_particle.py:104-239): callers use these where every promotion is to P.  Bound:
+// HBM, one pass over the (n, 3) arrays; on the host, numpy took 60 of the 65 ms of a plane-parallel
+// reconstruction of 1e6 points (4.4 ms now, host copies included) and 150 of the 166 ms of a particle
+// reconstruction of 3e5 + 2e6 points at 128^3 (10.3 ms now).
+template <typename P>
+struct PointArgs {
+  P f, first;    // growth rate; the first iteration's beta / (1 + beta), 0 otherwise
+  P los[3];
+  P off[3], bs[3], top[3];  // box corner, size, and size minus a cell (numpy's out-of-bounds test)
+  int local, field, shifted, wrap, skip;  // skip: bit d set where component d of s counts as 0
+};
+
+template <typename P>
+__device__ __forceinline__ P np_wrap(P x, P off, P bs) { return np_mod(x - off, bs) + off; }
+
+// Direction of the line of sight and (s . l) at x.
+template <typename P>
+__device__ __forceinline__ P along_los(const P x[3], const P s[3], const PointArgs<P>& A, P l[3]) {
+  if (A.local) {
+    const P dist = sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
+    for (int d = 0; d < 3; d++) l[d] = x[d] / dist;
+  } else {
+    for (int d = 0; d < 3; d++) l[d] = A.los[d];
+  }
+  return ((P(0) + s[0] * l[0]) + s[1] * l[1]) + s[2] * l[2];
+}
+
+// OP (PRH_POINT_*): see the header.  a, s, t: (n, 3) arrays; out may be one of them.
+template <typename P, int OP>
+__global__ __launch_bounds__(kCicThreads) void k_point_algebra(const P* x, const P* a, const P* s, const P* t,
+                                                               size_t n, PointArgs<P> A, P* out,
+                                                               uint32_t* __restrict__ misc) {
+  const size_t i = blockIdx.x * static_cast<size_t>(kCicThreads) + threadIdx.x;
+  uint32_t err = 0;
+  if (i < n) {
+    const P p[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
+    P r[3];
+    if constexpr (OP == PRH_POINT_WRAP) {
+      for (int d = 0; d < 3; d++) r[d] = np_wrap(p[d], A.off[d], A.bs[d]);
+    } else {
+      P q[3], l[3];
+      for (int d = 0; d < 3; d++) q[d] = (A.skip >> d) & 1 ? P(0) : s[3 * i + d];
+      if constexpr (OP == PRH_POINT_ITERATE || OP == PRH_POINT_REAL) {
+        P dot = along_los(p, q, A, l);
+        if (OP == PRH_POINT_ITERATE && A.first != P(0)) {
+          const P fd = A.first * dot;
+          for (int d = 0; d < 3; d++) q[d] = q[d] - fd * l[d];
+          dot = ((P(0) + q[0] * l[0]) + q[1] * l[1]) + q[2] * l[2];
+        }
+        const P fd = A.f * dot;
+        bool outside = false;
+        for (int d = 0; d < 3; d++) {
+          r[d] = p[d] - fd * l[d];
+          const P diff = r[d] - A.off[d];
+          outside = outside || diff < P(0) || diff > A.top[d];
+        }
+        if (outside) err = kErrRange;
+      } else {
+        P sh[3], from[3];
+        if constexpr (OP == PRH_POINT_DATA) {
+          // x the data, a their reconstructed positions
+          for (int d = 0; d < 3; d++) {
+            const P rsd = p[d] - a[3 * i + d];
+            sh[d] = A.field == PRH_FIELD_DISP ? q[d] : A.field == PRH_FIELD_RSD ? rsd : q[d] + rsd;
+            from[d] = p[d];
+          }
+        } else {
+          // x the (wrapped) positions the line of sight is taken at, a the positions as given
+          const P fd = A.f * along_los(p, q, A, l);
+          for (int d = 0; d < 3; d++) {
+            const P rsd = fd * l[d];
+            const P disp = OP == PRH_POINT_PARTICLE && A.field == PRH_FIELD_DISP_RSD ? t[3 * i + d] : q[d];
+            sh[d] = A.field == PRH_FIELD_DISP ? q[d] : A.field == PRH_FIELD_RSD ? rsd : disp + rsd;
+            from[d] = a[3 * i + d];
+          }
+        }
+        for (int d = 0; d < 3; d++) {
+          r[d] = A.shifted ? from[d] - sh[d] : sh[d];
+          if (A.shifted && A.wrap) r[d] = np_wrap(r[d], A.off[d], A.bs[d]);
+        }
+      }
+    }
+    for (int d = 0; d < 3; d++) out[3 * i + d] = r[d];
+  }
+  if (OP == PRH_POINT_ITERATE || OP == PRH_POINT_REAL) flag_errors(err, misc);
+}
+
+template <typename P>
+static int do_point_algebra(prh_workspace* ws, int op, const P* x, const P* a, const P* s, const P* t, size_t n,
+                            const prh_point_args* g, P* out, int* outside, void* stream) {
+  if (!ws || !g || (n && (!x || !out))) return PRH_ERR_ARG;
+  const bool flagged = op == PRH_POINT_ITERATE || op == PRH_POINT_REAL;
+  const bool disp_rsd = g->field == PRH_FIELD_DISP_RSD;
+  if (op < PRH_POINT_WRAP || op > PRH_POINT_DATA || (n && op != PRH_POINT_WRAP && !s) ||
+      (n && op >= PRH_POINT_SHIFT && !a) || (n && op == PRH_POINT_PARTICLE && disp_rsd && !t)) {
+    set_error("point algebra %d: unknown operation or missing array", op);
+    return PRH_ERR_ARG;
+  }
+  if (outside) *outside = 0;
+  if (n == 0) return PRH_OK;
+  PointArgs<P> A;
+  A.f = static_cast<P>(g->f);
+  A.first = static_cast<P>(g->first);
+  for (int d = 0; d < 3; d++) {
+    A.los[d] = static_cast<P>(g->los[d]);
+    A.off[d] = static_cast<P>(g->offset[d]);
+    A.bs[d] = static_cast<P>(g->boxsize[d]);
+    A.top[d] = static_cast<P>(g->top[d]);
+  }
+  A.local = g->local;
+  A.field = g->field;
+  A.shifted = g->shifted;
+  A.wrap = g->wrap;
+  A.skip = g->skip;
+  hipStream_t st = as_stream(stream);
+  uint32_t* misc = ws->misc;
+  if (flagged) {
+    k_zero_misc<<<1, 64, 0, st>>>(misc);
+    PRH_LAUNCHED();
+  }
+  const unsigned grid = ceil_div(n, static_cast<size_t>(kCicThreads));
+  switch (op) {
+    case PRH_POINT_WRAP: k_point_algebra<P, PRH_POINT_WRAP><<<grid, kCicThreads, 0, st>>>(x, a, s, t, n, A, out, misc); break;
+    case PRH_POINT_ITERATE: k_point_algebra<P, PRH_POINT_ITERATE><<<grid, kCicThreads, 0, st>>>(x, a, s, t, n, A, out, misc); break;
+    case PRH_POINT_REAL: k_point_algebra<P, PRH_POINT_REAL><<<grid, kCicThreads, 0, st>>>(x, a, s, t, n, A, out, misc); break;
+    case PRH_POINT_SHIFT: k_point_algebra<P, PRH_POINT_SHIFT><<<grid, kCicThreads, 0, st>>>(x, a, s, t, n, A, out, misc); break;
+    case PRH_POINT_PARTICLE: k_point_algebra<P, PRH_POINT_PARTICLE><<<grid, kCicThreads, 0, st>>>(x, a, s, t, n, A, out, misc); break;
+    default: k_point_algebra<P, PRH_POINT_DATA><<<grid, kCicThreads, 0, st>>>(x, a, s, t, n, A, out, misc); break;
+  }
+  PRH_LAUNCHED();
+  if (flagged && outside) {
+    PRH_HIP(hipMemcpyAsync(ws->flag_host, misc, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    PRH_HIP(hipStreamSynchronize(st));
+    *outside = ws->flag_host[0] & kErrRange ? 1 : 0;
+  }
+  return PRH_OK;
+}
+
+template <typename R>
+static int do_read_psi(prh_workspace* ws, const R* const* psi, const size_t* nmesh, const R* boxsize,
+                       const R* boxcenter, const void* pos, int pdt, size_t n, double f, const R* los, int field,
+                       int wrap, int shifted, void* out, int odt, int* nonfinite, void* stream) {
+  if (!ws || !nmesh || !boxsize || !boxcenter || (n && (!psi[0] || !psi[1] || !psi[2] || !pos || !out)))
+    return PRH_ERR_ARG;
+  if (field < PRH_FIELD_DISP || field > PRH_FIELD_VALUE || (field == PRH_FIELD_VALUE && shifted) ||
+      (wrap && field != PRH_FIELD_VALUE)) {
+    set_error("unknown field %d, or one that this read does not shift or wrap", field);
+    return PRH_ERR_ARG;
+  }
+  if ((pdt != PRH_F32 && pdt != PRH_F64) || (odt != PRH_F32 && odt != PRH_F64)) {
+    set_error("positions/output dtype must be PRH_F32 or PRH_F64");
+    return PRH_ERR_ARG;
+  }
+  const int q = pdt > Tag<R>::code ? pdt : Tag<R>::code;
+  const int expect = (field == PRH_FIELD_RSD && los) ? q : pdt;
+  if (odt != expect) {
+    set_error("output dtype %d does not follow numpy promotion (expected %d)", odt, expect);
+    return PRH_ERR_ARG;
+  }
+  if (nonfinite) *nonfinite = 0;
+  if (n == 0) return PRH_OK;
+  hipStream_t s = as_stream(stream);
+  k_zero_misc<<<1, 64, 0, s>>>(ws->misc);
+  PRH_LAUNCHED();
+  ReadArgs<R> A{};
+  A.F = make_frame<R>(nmesh, boxsize, boxcenter);
+  A.fgrowth = f;
+  for (int d = 0; d < 3; d++) A.los[d] = los ? los[d] : R(0);
+  A.local = los ? 0 : 1;
+  A.field = field;
+  A.wrap = wrap;
+  A.shifted = shifted;
+  int st;
+  if (pdt == PRH_F64)
+    st = read_psi_all<R, double, double>(ws, psi, A, static_cast<const double*>(pos), n, static_cast<double*>(out),
+                                         ws->misc, s);
+  else if (odt == PRH_F32)
+    st = read_psi_all<R, float, float>(ws, psi, A, static_cast<const float*>(pos), n, static_cast<float*>(out),
+                                       ws->misc, s);
+  else
+    st = read_psi_all<R, float, double>(ws, psi, A, static_cast<const float*>(pos), n, static_cast<double*>(out),
+                                        ws->misc, s);
+  PRH_TRY(st);
+  return read_status(ws, wrap, nonfinite, s);
+}
+
 template <typename R>
 static int do_read_shifts(prh_workspace* ws, const R* phi, const size_t* nmesh, const R* boxsize, const R* boxcenter,
                           const void* pos, int pdt, size_t n, double f, const R* los, int field,
@@ -2274,15 +2550,7 @@ static int do_read_shifts(prh_workspace* ws, const R* phi, const size_t* nmesh, 
                                            static_cast<double*>(out), misc, s);
   }
   PRH_TRY(st);
-  uint32_t* host = ws->flag_host;
-  PRH_HIP(hipMemcpyAsync(host, misc, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  PRH_HIP(hipStreamSynchronize(s));
-  if (nonfinite && (host[0] & kErrNonFinite)) *nonfinite = 1;
-  if (!wrap && (host[0] & kErrRange)) {
-    set_error("positions not in box range");
-    return PRH_ERR_RANGE;
-  }
-  return PRH_OK;
+  return read_status(ws, wrap, nonfinite, s);
 }
 
 }  // namespace prh
@@ -2354,6 +2622,31 @@ int prh_shift_algebra_f64(const void* positions, int pos_dtype, const void* s0, 
                           int out_dtype, void* stream) {
   return do_shift_algebra<double>(positions, pos_dtype, s0, s1, s2, npositions, f, los, field, shifted, out,
                                   out_dtype, stream);
+}
+
+int prh_read_psi_f32(prh_workspace* ws, const float* psi0, const float* psi1, const float* psi2, const size_t* nmesh,
+                     const float* boxsize, const float* boxcenter, const void* positions, int pos_dtype,
+                     size_t npositions, double f, const float* los, int field, int wrap, int shifted, void* out,
+                     int out_dtype, int* nonfinite, void* stream) {
+  const float* const psi[3] = {psi0, psi1, psi2};
+  return do_read_psi<float>(ws, psi, nmesh, boxsize, boxcenter, positions, pos_dtype, npositions, f, los, field, wrap,
+                            shifted, out, out_dtype, nonfinite, stream);
+}
+int prh_point_algebra_f32(prh_workspace* ws, int op, const float* x, const float* a, const float* s, const float* t,
+                          size_t n, const prh_point_args* args, float* out, int* outside, void* stream) {
+  return do_point_algebra<float>(ws, op, x, a, s, t, n, args, out, outside, stream);
+}
+int prh_read_psi_f64(prh_workspace* ws, const double* psi0, const double* psi1, const double* psi2, const size_t* nmesh,
+                     const double* boxsize, const double* boxcenter, const void* positions, int pos_dtype,
+                     size_t npositions, double f, const double* los, int field, int wrap, int shifted, void* out,
+                     int out_dtype, int* nonfinite, void* stream) {
+  const double* const psi[3] = {psi0, psi1, psi2};
+  return do_read_psi<double>(ws, psi, nmesh, boxsize, boxcenter, positions, pos_dtype, npositions, f, los, field, wrap,
+                            shifted, out, out_dtype, nonfinite, stream);
+}
+int prh_point_algebra_f64(prh_workspace* ws, int op, const double* x, const double* a, const double* s, const double* t,
+                          size_t n, const prh_point_args* args, double* out, int* outside, void* stream) {
+  return do_point_algebra<double>(ws, op, x, a, s, t, n, args, out, outside, stream);
 }
 
 int prh_read_shifts_f32(prh_workspace* ws, const float* phi, const size_t* nmesh, const float* boxsize,

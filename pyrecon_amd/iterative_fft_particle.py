@@ -4,8 +4,9 @@
 Each iteration repaints the data at their current real-space estimate (wrapped), smooths, forms the
 density contrast, transforms, divides by k^2 and reads the displacement at the data; the RSD part
 of the displacement (reduced by beta / (1 + beta) in the first iteration) is then removed from the
-original positions.  Paint, smoothing, density contrast, transforms, Fourier-space operators and
-CIC reads run in the HIP library; the per-point RSD algebra is the reference's numpy.
+original positions.  All of it runs in the HIP library, the per-point algebra with numpy's expressions
+in the positions dtype; where numpy would promote beyond that dtype (f4 positions with a f8 mesh and a
+global line of sight or wrap), or for other dtypes, the algebra is the reference's numpy on the host.
 """
 import numpy as np
 
@@ -62,6 +63,17 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
         check(status, 'density contrast')
         self.mesh_delta = delta
 
+    def _on_device(self, dtype):
+        """Whether numpy's algebra of positions of ``dtype`` stays in that dtype, as the device's does."""
+        if np.dtype(dtype) not in (np.dtype('f4'), np.dtype('f8')): return False
+        return self._device_dtype(dtype) or (self.los is None and not self.wrap)
+
+    @property
+    def _positions_rec_data(self):
+        """Reconstructed real-space positions of the data, on the host."""
+        rec = self._rec_data
+        return rec.numpy(stream=self.stream) if isinstance(rec, DeviceArray) else rec
+
     def run(self, niterations=3):
         """Reconstructed real-space data positions and the displacement meshes :attr:`mesh_psi`
         (iterative_fft_particle.py:61-78)."""
@@ -70,9 +82,17 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
         self._iter = 0
         self.mesh_data.smooth_gaussian(self.smoothing_radius)
         if self.has_randoms: self.mesh_randoms.smooth_gaussian(self.smoothing_radius)
-        self._positions_rec_data = self._positions_data.copy()
+        dtype = self._positions_data.dtype
+        if self._on_device(dtype):
+            self._data, _ = as_device(self._positions_data, stream=self.stream)
+            self._rec_data = self._data
+            self._data_weights, _ = as_device(self._weights_data, stream=self.stream)
+        else:
+            self._data = self._data_weights = None
+            self._rec_data = self._positions_data.copy()
         for it in range(niterations):
             self.mesh_psi = self._iterate(return_psi=it == niterations - 1)
+        self._data_weights = None
         self.mesh_randoms = None
 
     def _iterate(self, return_psi=False):
@@ -83,51 +103,63 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
             # paint the reconstructed real-space data positions, wrapped
             wrap = self.wrap
             self.wrap = True
-            BaseReconstruction.assign_data(self, self._positions_rec_data, weights=self._weights_data)
+            BaseReconstruction.assign_data(self, self._rec_data, weights=self._weights_data if self._data is None
+                                           else self._data_weights)
             self.wrap = wrap
             self.mesh_data.smooth_gaussian(self.smoothing_radius)
         self.set_density_contrast(ran_min=self.ran_min, smoothing_radius=self.smoothing_radius)
         self.mesh_data = None
-        scratch = self._scratch(_lib.SPECTRAL_DISPLACEMENTS)
-        if scratch is not None:
-            meshes = self._half_spectrum_psi(self.mesh_delta, scratch)
-            self.mesh_delta = None
+        # no displacement is needed along an axis the line of sight does not touch
+        skipped = [not return_psi and self.los is not None and self.los[iaxis] == 0 for iaxis in range(3)]
+        psis = self._compute_psi(skipped)
+        self.mesh_delta = None
+        first = self.beta / (1 + self.beta) if self._iter == 0 else 0.
+        outside = False
+        if self._data is not None:
+            shifts = self._read_psi_device(self._rec_data, wrap=True, psis=psis)
+            # the RSD is removed from the original positions; the next iteration paints these
+            self._rec_data = self._point_algebra(_lib.POINT_ITERATE, self._data, s=shifts, first=first, out=shifts,
+                                                 skip=sum(skip << iaxis for iaxis, skip in enumerate(skipped)),
+                                                 outside=not self.wrap)
+            if not self.wrap: self._rec_data, outside = self._rec_data
         else:
-            delta_k = self._spectrum(self.mesh_delta)
-            self.mesh_delta = None
-            self._spectral(_lib.SPEC_INV_K2, delta_k, delta_k)
-            norm = 1. / self.info.size
-            work = self._complex()
-        shifts = np.empty_like(self._positions_rec_data)
-        pos, _ = as_device(self._positions_rec_data, stream=self.stream)
-        psis = []
-        for iaxis in range(3):
-            # no displacement is needed along an axis the line of sight does not touch
-            if not return_psi and self.los is not None and self.los[iaxis] == 0:
-                shifts[:, iaxis] = 0.
-                continue
-            if scratch is not None:
-                psi = meshes[iaxis]
+            shifts = np.zeros_like(self._rec_data)
+            pos, _ = as_device(self._rec_data, stream=self.stream)
+            for iaxis, psi in enumerate(psis):
+                if not skipped[iaxis]: shifts[:, iaxis] = psi.read_cic(pos, wrap=True).numpy(stream=self.stream)
+            if self.los is None:
+                los = self._positions_data / distance(self._positions_data)[:, None]
             else:
-                self._spectral(_lib.SPEC_I_KA, delta_k, work, a=iaxis, norm=norm)
-                psi = self._to_real(work)
-            shifts[:, iaxis] = psi.read_cic(pos, wrap=True).numpy(stream=self.stream)
-            if return_psi: psis.append(psi)
-        if self.los is None:
-            los = self._positions_data / distance(self._positions_data)[:, None]
-        else:
-            los = self.los
-        if self._iter == 0:
-            # first iteration: remove the RSD part approximately (Burden et al. 2015, eq. 12)
-            shifts -= self.beta / (1 + self.beta) * np.sum(shifts * los, axis=-1)[:, None] * los
-        # the RSD is removed from the original positions; the next iteration paints these
-        self._positions_rec_data = self._positions_data - self.f * np.sum(shifts * los, axis=-1)[:, None] * los
-        diff = self._positions_rec_data - self.info.offset
-        if (not self.wrap) and np.any((diff < 0) | (diff > self.info.boxsize - self.info.cellsize)):
-            self.logger.warning('Some particles are out-of-bounds.')
+                los = self.los
+            if self._iter == 0:
+                # first iteration: remove the RSD part approximately (Burden et al. 2015, eq. 12)
+                shifts -= first * np.sum(shifts * los, axis=-1)[:, None] * los
+            self._rec_data = self._positions_data - self.f * np.sum(shifts * los, axis=-1)[:, None] * los
+            outside = self._out_of_bounds(self._rec_data)
+        if outside: self.logger.warning('Some particles are out-of-bounds.')
         self._iter += 1
         if return_psi:
             return psis
+
+    def _out_of_bounds(self, positions):
+        diff = positions - self.info.offset
+        return (not self.wrap) and np.any((diff < 0) | (diff > self.info.boxsize - self.info.cellsize))
+
+    def _compute_psi(self, skipped):
+        """The displacement meshes of :attr:`mesh_delta`; any mesh stands in for a skipped axis."""
+        scratch = self._scratch(_lib.SPECTRAL_DISPLACEMENTS)
+        if scratch is not None:
+            return self._half_spectrum_psi(self.mesh_delta, scratch)
+        delta_k = self._spectrum(self.mesh_delta)
+        self._spectral(_lib.SPEC_INV_K2, delta_k, delta_k)
+        work = self._complex()
+        psis = [None] * 3
+        for iaxis in range(3):
+            if skipped[iaxis]: continue
+            self._spectral(_lib.SPEC_I_KA, delta_k, work, a=iaxis, norm=1. / self.info.size)
+            psis[iaxis] = self._to_real(work)
+        done = next(psi for psi in psis if psi is not None)
+        return [done if psi is None else psi for psi in psis]
 
     def _read_psi(self, positions, wrap=False):
         shifts = np.empty_like(positions)
@@ -139,23 +171,58 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
     def read_shifts(self, positions, field='disp+rsd'):
         """Displacements at ``positions``, or with ``positions='data'`` at the reconstructed data
         (iterative_fft_particle.py:141-212)."""
-        field = field.lower()
-        allowed_fields = ['disp', 'rsd', 'disp+rsd']
-        if field not in allowed_fields:
-            raise ReconstructionError('Unknown field {}. Choices are {}'.format(field, allowed_fields))
-        if getattr(self, 'mesh_psi', None) is None:
-            raise ReconstructionError('run the reconstruction before reading shifts')
-        if isinstance(positions, str) and positions == 'data':
-            shifts = self._read_psi(self._positions_rec_data, wrap=True)
+        return self._shifts(positions, self._check_field(field), False)
+
+    def read_shifted_positions(self, positions, field='disp+rsd'):
+        """``positions - read_shifts(positions)`` (``'data'``: the data given to :meth:`assign_data`), wrapped
+        if :attr:`wrap` (iterative_fft_particle.py:214-239)."""
+        return self._shifts(positions, self._check_field(field), True)
+
+    def _shifts(self, positions, field, shifted):
+        """Shifts or shifted positions (host arrays out)."""
+        data = isinstance(positions, str) and positions == 'data'
+        if not data and not isinstance(positions, DeviceArray): positions = np.asarray(positions)
+        if self._data is not None if data else \
+                positions.ndim == 2 and positions.shape[1] == 3 and self._on_device(positions.dtype):
+            return self._device_shifts(None if data else positions, field, shifted).numpy(stream=self.stream)
+        if not data and isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
+        shifts = self._host_shifts(positions, field)
+        if not shifted: return shifts
+        positions = (self._positions_data if data else positions) - shifts
+        if self.wrap: positions = self.info.wrap(positions)
+        return positions
+
+    def _device_shifts(self, positions, field, shifted):
+        """On the device, as a device array; ``None`` stands for the data."""
+        code = self._FIELDS[field]
+        if positions is None:
+            psi = self._read_psi_device(self._rec_data, wrap=True) if field != 'rsd' else self._rec_data
+            return self._point_algebra(_lib.POINT_DATA, self._data, a=self._rec_data, s=psi, field=code, shifted=shifted)
+        pos, _ = as_device(positions, stream=self.stream)
+        inside = self._point_algebra(_lib.POINT_WRAP, pos) if self.wrap else pos
+        psi = self._read_psi_device(inside)
+        moved = None
+        if field == 'disp+rsd':
+            # the original algorithm's convention: RSD removed first, then the displacement read there
+            real = self._point_algebra(_lib.POINT_REAL, inside, s=psi, outside=not self.wrap)
+            if not self.wrap:
+                real, outside = real
+                if outside: self.logger.warning('Some particles are out-of-bounds.')
+            moved = self._read_psi_device(real, wrap=True)
+        return self._point_algebra(_lib.POINT_PARTICLE, inside, a=pos, s=psi, t=moved, field=code, shifted=shifted,
+                                   out=psi)
+
+    def _host_shifts(self, positions, field):
+        """The shifts with the reference's numpy algebra on the host."""
+        if isinstance(positions, str):
+            shifts = self._read_psi(self._rec_data, wrap=True)
             if field == 'disp':
                 return shifts
-            rsd = self._positions_data - self._positions_rec_data
+            rsd = self._positions_data - self._rec_data
             if field == 'rsd':
                 return rsd
             shifts += rsd
             return shifts
-        if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
-        positions = np.asarray(positions)
         if self.wrap: positions = self.info.wrap(positions)
         shifts = self._read_psi(positions, wrap=False)
         if field == 'disp':
@@ -167,24 +234,10 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
         rsd = self.f * np.sum(shifts * los, axis=-1)[:, None] * los
         if field == 'rsd':
             return rsd
-        # the original algorithm's convention: RSD removed first, then the displacement read there
         real_positions = positions - rsd
-        diff = real_positions - self.info.offset
-        if (not self.wrap) and np.any((diff < 0) | (diff > self.info.boxsize - self.info.cellsize)):
-            self.logger.warning('Some particles are out-of-bounds.')
+        if self._out_of_bounds(real_positions): self.logger.warning('Some particles are out-of-bounds.')
         shifts = self._read_psi(real_positions, wrap=True)
         return shifts + rsd
-
-    def read_shifted_positions(self, positions, field='disp+rsd'):
-        """``positions - read_shifts(positions)`` (``'data'``: the data given to :meth:`assign_data`), wrapped
-        if :attr:`wrap` (iterative_fft_particle.py:214-239)."""
-        if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
-        shifts = self.read_shifts(positions, field=field)
-        if isinstance(positions, str) and positions == 'data':
-            positions = self._positions_data
-        positions = positions - shifts
-        if self.wrap: positions = self.info.wrap(positions)
-        return positions
 
 
 class IterativeFFTParticleReconstruction(OriginalIterativeFFTParticleReconstruction):

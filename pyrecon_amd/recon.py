@@ -7,6 +7,7 @@ arrays (:class:`~pyrecon_amd.device.DeviceArray`, or a tensor exposing
 """
 import ctypes
 import logging
+import warnings
 
 import numpy as np
 
@@ -226,7 +227,6 @@ class BaseReconstruction(object):
                  int(bool(shifted)), out.ptr, _lib.dtype_code(odtype), ctypes.byref(nonfinite),
                  stream_handle(self.stream)), 'read_shifts')
         if nonfinite.value:
-            import warnings
             warnings.warn('Some positions are NaN/inf')
         return out.numpy(stream=self.stream) if is_host else out
 
@@ -327,40 +327,91 @@ class SpectralReconstruction(BaseReconstruction):
             raise ReconstructionError('run the reconstruction before reading shifts')
         return field
 
+    def _read_psi_device(self, pos, field=_lib.FIELD_VALUE, wrap=False, shifted=False, odtype=None, psis=None):
+        """:attr:`mesh_psi` (or ``psis``) read by CIC at the device positions: the (N, 3) displacements, or the
+        shifts or shifted positions they give (pyrecon/recon.py:255-325, without wrap)."""
+        if odtype is None: odtype = pos.dtype
+        if psis is None: psis = self.mesh_psi
+        if any(psi.buffer is None for psi in psis): raise MeshError('mesh has no value')
+        out = DeviceArray((len(pos), 3), odtype, stream=self.stream)
+        nm, nm_ptr = _lib.size3(self.info.shape)
+        bs, bs_ptr = _lib.vec3(self.info.boxsize, self.info.dtype)
+        bc, bc_ptr = _lib.vec3(self.info.boxcenter, self.info.dtype)
+        los = None if self.los is None else np.ascontiguousarray(self.los, dtype=self.info.dtype)
+        nonfinite = ctypes.c_int(0)
+        fn = getattr(lib, 'prh_read_psi_' + _suffix(self.info.dtype))
+        status = fn(self.workspace.handle, *[psi.buffer.ptr for psi in psis], nm_ptr, bs_ptr, bc_ptr, pos.ptr,
+                    _lib.dtype_code(pos.dtype), len(pos), float(self.f), los.ctypes.data if los is not None else None,
+                    int(field), int(bool(wrap)), int(bool(shifted)), out.ptr, _lib.dtype_code(odtype),
+                    ctypes.byref(nonfinite), stream_handle(self.stream))
+        if status == _lib.ERR_RANGE:
+            low, high = self.boxcenter - self.boxsize / 2., self.boxcenter + self.boxsize / 2.
+            raise MeshError('positions not in box range {} - {}'.format(low, high))
+        check(status, 'read')
+        if nonfinite.value: warnings.warn('Some positions are NaN/inf')
+        return out
+
+    def _device_dtype(self, dtype):
+        """Whether numpy's promotions of positions of ``dtype`` with the box and a global line of sight (both in
+        the mesh dtype) all stay in ``dtype``, as the device's per-point algebra has it."""
+        dtype = np.dtype(dtype)
+        return dtype in (np.dtype('f4'), np.dtype('f8')) and np.promote_types(dtype, self.info.dtype) == dtype
+
+    def _point_algebra(self, op, x, a=None, s=None, t=None, out=None, field=_lib.FIELD_DISP_RSD, first=0., shifted=False,
+                       skip=0, outside=False):
+        """prh_point_algebra over (N, 3) device arrays; with ``outside``, also whether a result is out of bounds."""
+        info = self.info
+        if out is None: out = DeviceArray(x.shape, x.dtype, stream=self.stream)
+        vec = lambda v: (ctypes.c_double * 3)(*[float(c) for c in v])
+        args = _lib.PointArgs(f=float(self.f), first=float(first), los=vec(self.los if self.los is not None else [0.] * 3),
+                              offset=vec(info.offset), boxsize=vec(info.boxsize), top=vec(info.boxsize - info.cellsize),
+                              local=int(self.los is None), field=int(field), shifted=int(bool(shifted)),
+                              wrap=int(bool(self.wrap)), skip=int(skip))
+        flag = ctypes.c_int(0)
+        ptr = lambda array: array.ptr if array is not None else None
+        fn = getattr(lib, 'prh_point_algebra_' + _suffix(x.dtype))
+        check(fn(self.workspace.handle, int(op), x.ptr, ptr(a), ptr(s), ptr(t), len(x), ctypes.byref(args), out.ptr,
+                 ctypes.byref(flag) if outside else None, stream_handle(self.stream)), 'point algebra')
+        return (out, bool(flag.value)) if outside else out
+
     def _device_shifts(self, positions, field, shifted):
-        """Shifts (or, ``shifted``, shifted positions) without wrap, on the device: the three CIC reads
-        of :attr:`mesh_psi`, then the RSD algebra of pyrecon/recon.py:255-325 in numpy's dtypes and
-        order (``prh_shift_algebra_*``).  Host in -> host out, device in -> device out."""
+        """Shifts (or, ``shifted``, shifted positions) without wrap, on the device: the CIC reads of
+        :attr:`mesh_psi` and the RSD algebra of pyrecon/recon.py:255-325 in numpy's dtypes and order, in one
+        pass over the points.  Host in -> host out, device in -> device out."""
         pos, is_host = as_device(positions, stream=self.stream)
         if pos.ndim != 2 or pos.shape[1] != 3:
             raise ValueError('positions must have shape (N, 3)')
         if pos.dtype not in (np.dtype('f4'), np.dtype('f8')):
             pos, is_host = as_device(np.asarray(positions, dtype='f8'), stream=self.stream)
-        comps = [psi.read_cic(pos, wrap=False) for psi in self.mesh_psi]
-        los = None if self.los is None else np.ascontiguousarray(self.los, dtype=self.info.dtype)
         odt = pos.dtype
-        if field == 'rsd' and los is not None: odt = np.promote_types(pos.dtype, self.info.dtype)
-        out = DeviceArray((len(pos), 3), odt, stream=self.stream)
-        fn = getattr(lib, 'prh_shift_algebra_' + _suffix(self.info.dtype))
-        check(fn(pos.ptr, _lib.dtype_code(pos.dtype), comps[0].ptr, comps[1].ptr, comps[2].ptr, len(pos),
-                 float(self.f), los.ctypes.data if los is not None else None, self._FIELDS[field], int(bool(shifted)),
-                 out.ptr, _lib.dtype_code(odt), stream_handle(self.stream)), 'shift algebra')
+        if field == 'rsd' and self.los is not None: odt = np.promote_types(pos.dtype, self.info.dtype)
+        out = self._read_psi_device(pos, field=self._FIELDS[field], shifted=shifted, odtype=odt)
         return out.numpy(stream=self.stream) if is_host else out
+
+    def _wrapped_shifts(self, positions, field, shifted):
+        """The same with the positions wrapped first, on the device; host arrays out."""
+        if not isinstance(positions, DeviceArray): positions = np.asarray(positions)
+        if positions.ndim != 2 or positions.shape[1] != 3 or not self._device_dtype(positions.dtype):
+            # other dtypes take numpy's promotions on the host
+            if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
+            shifts = self._host_shifts(positions, field)
+            return self.info.wrap(positions - shifts) if shifted else shifts
+        pos, _ = as_device(positions, stream=self.stream)
+        inside = self._point_algebra(_lib.POINT_WRAP, pos)
+        psi = self._read_psi_device(inside)
+        out = self._point_algebra(_lib.POINT_SHIFT, inside, a=pos, s=psi, field=self._FIELDS[field], shifted=shifted,
+                                  out=psi)
+        return out.numpy(stream=self.stream)
 
     def read_shifts(self, positions, field='disp+rsd'):
         """Displacements at ``positions`` (pyrecon/recon.py:255-302): each component read by CIC from
-        :attr:`mesh_psi` on the device.  Without :attr:`wrap` the RSD algebra runs on the device
-        (host in -> host out, device in -> device out); with it, positions are wrapped first and the
-        algebra is the reference's numpy on the host (host arrays out)."""
+        :attr:`mesh_psi`, then the RSD algebra, on the device.  Without :attr:`wrap` host in -> host out,
+        device in -> device out; with it, positions are wrapped first and host arrays come out."""
         field = self._check_field(field)
-        if not self.wrap: return self._device_shifts(positions, field, False)
-        return self._host_shifts(positions, field)
+        return self._wrapped_shifts(positions, field, False) if self.wrap else self._device_shifts(positions, field, False)
 
     def _host_shifts(self, positions, field):
-        """The shifts with the reference's numpy RSD algebra on the host, positions wrapped first if
-        :attr:`wrap` (host arrays out)."""
-        if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
-        positions = np.asarray(positions)
+        """The shifts of host positions with the reference's numpy RSD algebra, wrapped first if :attr:`wrap`."""
         shifts = np.empty_like(positions)
         if self.wrap: positions = self.info.wrap(positions)
         pos, _ = as_device(positions, stream=self.stream)
@@ -381,9 +432,4 @@ class SpectralReconstruction(BaseReconstruction):
     def read_shifted_positions(self, positions, field='disp+rsd'):
         """``positions - read_shifts(positions)``, wrapped if :attr:`wrap` (pyrecon/recon.py:304-325)."""
         field = self._check_field(field)
-        if not self.wrap: return self._device_shifts(positions, field, True)
-        if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
-        shifts = self._host_shifts(positions, field)
-        positions = positions - shifts
-        if self.wrap: positions = self.info.wrap(positions)
-        return positions
+        return self._wrapped_shifts(positions, field, True) if self.wrap else self._device_shifts(positions, field, True)
