@@ -48,23 +48,6 @@ __device__ __forceinline__ void unflatten(I i, int n1, int n2, int& ix, int& iy,
   }
 }
 
-// Generic kernels: one thread per cell on a 3D grid (x = blockIdx.z), for any
-// shape; used for the coarse levels and for shapes the tiled kernel does not
-// cover.
-template <typename R, bool ZERO_IN>
-__global__ __launch_bounds__(kThreads) void k_jacobi(const R* __restrict__ v,
-                                                     const R* __restrict__ f, R* __restrict__ out,
-                                                     LevelGeom<R> G, R omega, R keep) {
-  const int iz = blockIdx.x * blockDim.x + threadIdx.x;
-  const int iy = blockIdx.y * blockDim.y + threadIdx.y;
-  const int ix = blockIdx.z;
-  if (iz >= G.n[2] || iy >= G.n[1]) return;
-  const size_t i = (static_cast<size_t>(ix) * G.n[1] + iy) * G.n[2] + iz;
-  const Coef<R> k = cell_coef(G, ix, iy, iz);
-  const Hood<R> h = ZERO_IN ? zero_hood<R>() : gather_hood(v, G.n[0], G.n[1], G.n[2], ix, iy, iz);
-  out[i] = jacobi_update(k, h, f[i], omega, keep, G.local);
-}
-
 // A source read with its mean removed: each value f becomes f - sum[0] / n
 // (sum on the device, n the number of cells), the same FP64 subtraction as a
 // centred copy of f would hold.  sum == nullptr: the source as it is.
@@ -75,22 +58,6 @@ struct Centre {
 template <typename R>
 __device__ __forceinline__ R centre_mean(const Centre& C) {
   return C.sum ? static_cast<R>(*C.sum / C.n) : R(0);
-}
-
-template <typename R, typename O>
-__global__ __launch_bounds__(kThreads) void k_residual(const R* __restrict__ v,
-                                                       const R* __restrict__ f,
-                                                       O* __restrict__ r, LevelGeom<R> G,
-                                                       Centre C) {
-  const int iz = blockIdx.x * blockDim.x + threadIdx.x;
-  const int iy = blockIdx.y * blockDim.y + threadIdx.y;
-  const int ix = blockIdx.z;
-  if (iz >= G.n[2] || iy >= G.n[1]) return;
-  const size_t i = (static_cast<size_t>(ix) * G.n[1] + iy) * G.n[2] + iz;
-  const Coef<R> k = cell_coef(G, ix, iy, iz);
-  const Hood<R> h = gather_hood(v, G.n[0], G.n[1], G.n[2], ix, iy, iz);
-  const R fv = C.sum ? f[i] - centre_mean<R>(C) : f[i];
-  r[i] = static_cast<O>(residual_value(k, h, fv, G.local));
 }
 
 // 2.5D-blocked kernel for large levels (n2 % 64 == 0, n1 % TY == 0).  A block
@@ -123,7 +90,11 @@ struct TileCoef {
   double* acc = nullptr;
   // kOpResidual: the source's mean to remove (the mixed path's centred source)
   Centre C;
+  // FLEX tiles: tz x ty cells (at most kFlexCells), and their numbers along z and y
+  int tz = 0, ty = 0, ztiles = 0, ytiles = 0;
 };
+constexpr int kFlexCells = 512;   // cells of a FLEX tile: two per thread
+constexpr int kFlexPlane = 768;   // staged cells of one: (tz + 2) (ty + 2) at most
 
 // One cell of a blocked sweep: the coefficients at (px, py, pz) (A, B, C are
 // h2 * p^2 along x, y, z) and the Jacobi update or the residual.
@@ -191,13 +162,20 @@ constexpr int tiled_min_waves() {
   return std::is_same<R, double>::value && std::is_same<O, float>::value ? 4 : PRH_TILED_MIN_WAVES;
 }
 
-template <typename R, typename O, int OP, int TY, bool LOCAL, bool FAST>
+// FLEX: tiles of any extent, for levels whose rows are no multiple of 64 cells or
+// whose planes are no multiple of 8 rows: the level's (y, z) plane is cut evenly
+// into tiles of at most kFlexCells cells, the tile's cells are dealt to the
+// threads in order, and the last tiles may be partial.
+template <typename R, typename O, int OP, int TY, bool LOCAL, bool FAST, bool FLEX = false>
 __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tiled(const R* __restrict__ v,
                                                        const R* __restrict__ f,
                                                        O* __restrict__ out, TileCoef<R> T,
                                                        R omega, R keep, int xlen) {
-  constexpr int W = kTileZ + 2, H = TY + 2, PLANE = W * H, KY = TY / 4;
+  static_assert(!FLEX || TY == 8, "two cells per thread");
+  constexpr int KY = TY / 4, PLANE = FLEX ? kFlexPlane : (kTileZ + 2) * (TY + 2);
   constexpr int PER = (PLANE + 255) / 256;
+  const int W = FLEX ? T.tz + 2 : kTileZ + 2;
+  const int staged_cells = FLEX ? W * (T.ty + 2) : PLANE;
   __shared__ R lds[4 * PLANE];
   const LevelGeom<R>& G = T.G;
   const R fmean = OP == kOpResidual ? centre_mean<R>(T.C) : R(0);
@@ -207,12 +185,12 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
   // logical tiles are numbered z-tile fastest, then y-tile, then x-run, and each
   // XCD gets a contiguous range of them, so tiles that share halo rows and
   // columns run together on one L2
-  const int ztiles = n2 / kTileZ, ytiles = n1 / TY;
+  const int ztiles = FLEX ? T.ztiles : n2 / kTileZ, ytiles = FLEX ? T.ytiles : n1 / TY;
   const unsigned nb = gridDim.x, bid = blockIdx.x, per = nb / 8;
   const unsigned L = bid < per * 8 ? (bid % 8) * per + bid / 8 : bid;
   const int zt = static_cast<int>(L % ztiles), yt = static_cast<int>((L / ztiles) % ytiles);
   const int xr = static_cast<int>(L / (static_cast<unsigned>(ztiles) * ytiles));
-  const int z0 = zt * kTileZ, y0 = yt * TY;
+  const int z0 = zt * (FLEX ? T.tz : kTileZ), y0 = yt * (FLEX ? T.ty : TY);
   const int xb = xr * xlen;
   const int xe = xb + xlen < n0 ? xb + xlen : n0;
   const size_t s0 = static_cast<size_t>(n1) * n2;
@@ -221,7 +199,7 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
 #pragma unroll
   for (int q = 0; q < PER; q++) {
     const int e = tid + 256 * q;
-    has[q] = e < PLANE;
+    has[q] = e < staged_cells;
     const int row = e / W, col = e - (e / W) * W;
     int gy = y0 - 1 + row;
     gy += gy < 0 ? n1 : 0;
@@ -229,6 +207,8 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
     int gz = z0 - 1 + col;
     gz += gz < 0 ? n2 : 0;
     gz -= gz >= n2 ? n2 : 0;
+    // a partial tile stages cells past its end too (wrapped again, and not used)
+    if (FLEX) gy = min(gy, n1 - 1), gz = min(gz, n2 - 1);
     off[q] = gy * n2 + gz;
   }
   auto wrapx = [n0](int x) { return x < 0 ? x + n0 : (x >= n0 ? x - n0 : x); };
@@ -242,24 +222,35 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
     for (int q = 0; q < PER; q++)
       if (has[q]) dst[tid + 256 * q] = src[off[q]];
   }
-  // per-thread constants: rows iy_k = y0 + ty + 4k, column iz
-  const int iz = z0 + tz;
+  // per-thread constants: rows iy_k = y0 + ty + 4k, column iz; FLEX: cells tid and
+  // tid + 256 of the tile
+  constexpr int KZ = FLEX ? KY : 1;  // columns a thread has
   int rowoff[KY], lo[KY];
+  bool live[KY];
   R py[KY], B[KY], pypz[KY];
-  R pz = R(0), C = R(0);
-  if (LOCAL) {
-    pz = static_cast<R>(iz) + G.org[2];
-    C = G.h2[2] * pz * pz;
-  }
+  R pz[KZ], C[KZ];
 #pragma unroll
   for (int k = 0; k < KY; k++) {
-    const int iy = y0 + ty + 4 * k;
+    int row = ty + 4 * k, col = tz;
+    live[k] = true;
+    if (FLEX) {
+      const int e = tid + 256 * k;
+      row = e / T.tz;
+      col = e - row * T.tz;
+      live[k] = row < T.ty && y0 + row < n1 && z0 + col < n2;
+      if (!live[k]) row = col = 0;
+    }
+    const int iy = y0 + row, iz = z0 + col;
     rowoff[k] = iy * n2 + iz;
-    lo[k] = (ty + 4 * k + 1) * W + tz + 1;
+    lo[k] = (row + 1) * W + col + 1;
+    if (k < KZ) {
+      pz[k] = LOCAL ? static_cast<R>(iz) + G.org[2] : R(0);
+      C[k] = LOCAL ? G.h2[2] * pz[k] * pz[k] : R(0);
+    }
     if (LOCAL) {
       py[k] = static_cast<R>(iy) + G.org[1];
       B[k] = G.h2[1] * py[k] * py[k];
-      pypz[k] = py[k] * pz;
+      pypz[k] = py[k] * pz[FLEX ? k : 0];
     } else {
       py[k] = R(0);
       B[k] = R(0);
@@ -296,6 +287,7 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
     }
 #pragma unroll
     for (int k = 0; k < KY; k++) {
+      if (FLEX && !live[k]) continue;
       const int o = lo[k];
       Hood<R> h = zero_hood<R>();
       if (OP != kOpJacobiZero) {
@@ -320,7 +312,8 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
       h.ypzm = P[o + W - 1];
       }
       const R fv = (OP == kOpResidual && T.C.sum) ? fvs[k] - fmean : fvs[k];
-      const R res = stencil_cell<R, OP, LOCAL, FAST>(T, h, fv, px, A, py[k], B[k], pz, C, pypz[k],
+      const R res = stencil_cell<R, OP, LOCAL, FAST>(T, h, fv, px, A, py[k], B[k], pz[FLEX ? k : 0],
+                                                     C[FLEX ? k : 0], pypz[k],
                                                      omega, keep);
       if constexpr (OP == kOpJacobiAcc)
         T.acc[static_cast<size_t>(x) * s0 + rowoff[k]] += static_cast<double>(res);
@@ -871,7 +864,9 @@ __global__ __launch_bounds__(NT, 1) void k_stencil_pair(const float* __restrict_
 constexpr int kRowsY1024 = 4;
 inline int rows_ry(const int* n) { return n[2] == 1024 ? kRowsY1024 : kRowsY; }
 
-// row length in units of 64 cells (1, 2, 4, 8 or 16), 0 where the kernel does not apply
+// row length in units of 64 cells (1, 2, 4, 8 or 16), 0 where the kernel does not apply (rows of 192, 320
+// and 384 cells are slower here than in the 64-wide tiles: 5.94, 15.8 and 24.1 ms a solve of 192^3 (FP32
+// meshes), 320^3 and 384^3 (mixed) against 5.72, 15.1 and 22.0; rows of 448 spill)
 inline int rows_cz(const int* n) {
   if (n[2] % 64 != 0 || n[1] % rows_ry(n) != 0 || n[0] < 1) return 0;
   const int cz = n[2] / 64;
@@ -888,6 +883,28 @@ inline int rows_xlen(const int* n) {
 }
 
 inline bool tiled_ok(const int* n) { return n[2] % kTileZ == 0 && n[1] % kTileY == 0 && n[0] >= 1; }
+
+// Levels that the 64-wide tiles do not cover (rows no multiple of 64 cells, planes no multiple of 8
+// rows) and that fill the device by themselves.  FP64 ones go through FLEX tiles: a solve of 320 x 384 x
+// 224 takes 24.4 ms (29.5 with the columns below, 35.1 with a cell a thread).  FP32 ones, half the size
+// and mostly in cache, go through the columns: 21.4 ms for 384 x 320 x 448 against 22.9 with FLEX tiles.
+constexpr size_t kFlexMin = 500000;
+inline bool fills_alone(const int* n) {
+  return !tiled_ok(n) && static_cast<size_t>(n[0]) * n[1] * n[2] >= kFlexMin;
+}
+// The plane cut evenly: tiles along z of at most 64 cells, and along y of as many rows as two cells a
+// thread take.
+template <typename R>
+inline void flex_tiles(const int* n, TileCoef<R>& T) {
+  T.ztiles = (n[2] + kTileZ - 1) / kTileZ;
+  T.tz = (n[2] + T.ztiles - 1) / T.ztiles;
+  T.ztiles = (n[2] + T.tz - 1) / T.tz;
+  int rows = kFlexCells / T.tz;
+  while ((T.tz + 2) * (rows + 2) > kFlexPlane) rows--;
+  T.ytiles = (n[1] + rows - 1) / rows;
+  T.ty = (n[1] + T.ytiles - 1) / T.ytiles;
+  T.ytiles = (n[1] + T.ty - 1) / T.ty;
+}
 
 // PRH_TUNE_PAIRED_SWEEPS, off by default: on MI355X the fused pair is slower
 // than two single sweeps (0.69 against 2 x 0.31 ms at 512^3), because a sweep
@@ -1011,6 +1028,147 @@ static void launch_tiled(const R* v, const R* f, O* out, const LevelGeom<R>& G, 
       k_stencil_tiled<R, O, OP, kTileY, true, FAST><<<grid, 256, 0, s>>>(v, f, out, T, omega, keep, xlen);
     else
       k_stencil_tiled<R, O, OP, kTileY, false, FAST><<<grid, 256, 0, s>>>(v, f, out, T, omega, keep, xlen);
+  }
+}
+
+// Columns: each thread takes XL consecutive x of one (y, z), keeping the planes x - 1, x and x + 1 of
+// its neighbourhood in registers (11.5 loads a cell for XL = 4 instead of 19) and the parts of the
+// coefficients that do not change along x.  No LDS and no barrier: neighbouring threads' loads meet in
+// L1, and the levels lie in L2 or the last-level cache.
+template <typename R, typename O, int OP, bool LOCAL, int XL>
+__global__ __launch_bounds__(kThreads) void k_stencil_columns(const R* __restrict__ v, const R* __restrict__ f,
+                                                              O* __restrict__ out, TileCoef<R> T, R omega,
+                                                              R keep) {
+  const LevelGeom<R>& G = T.G;
+  const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
+  const int iz = blockIdx.x * blockDim.x + threadIdx.x;
+  const int iy = blockIdx.y * blockDim.y + threadIdx.y;
+  if (iz >= n2 || iy >= n1) return;
+  const R fmean = OP == kOpResidual ? centre_mean<R>(T.C) : R(0);
+  const int xb = blockIdx.z * XL, xe = min(xb + XL, n0);
+  const int s0 = n1 * n2;
+  const int yp = (iy + 1 == n1 ? 0 : iy + 1) * n2, ym = (iy == 0 ? n1 - 1 : iy - 1) * n2, y0 = iy * n2;
+  const int zp = iz + 1 == n2 ? 0 : iz + 1, zm = iz == 0 ? n2 - 1 : iz - 1;
+  R py = R(0), B = R(0), pz = R(0), C = R(0), pypz = T.K.pypz;
+  if (LOCAL) {
+    py = static_cast<R>(iy) + G.org[1];
+    B = G.h2[1] * py * py;
+    pz = static_cast<R>(iz) + G.org[2];
+    C = G.h2[2] * pz * pz;
+    pypz = py * pz;
+  }
+  struct Plane {
+    R c, yp, ym, zp, zm, pp, pm, mp, mm;  // last four: (y, z) = (+, +), (+, -), (-, +), (-, -)
+  };
+  auto cross = [&](Plane& P, const R* u) {
+    P.c = u[y0 + iz];
+    P.yp = u[yp + iz];
+    P.ym = u[ym + iz];
+    P.zp = u[y0 + zp];
+    P.zm = u[y0 + zm];
+  };
+  auto corners = [&](Plane& P, const R* u) {
+    P.pp = u[yp + zp];
+    P.pm = u[yp + zm];
+    P.mp = u[ym + zp];
+    P.mm = u[ym + zm];
+  };
+  auto plane = [&](int x) { return v + static_cast<size_t>(x) * s0; };
+  Plane a, b, c;
+  if (OP != kOpJacobiZero) {
+    cross(a, plane(xb == 0 ? n0 - 1 : xb - 1));
+    cross(b, plane(xb));
+    corners(b, plane(xb));
+  }
+#pragma unroll
+  for (int u = 0; u < XL; u++) {
+    const int x = xb + u;
+    if (u > 0 && x >= xe) break;
+    const size_t at = static_cast<size_t>(x) * s0 + y0 + iz;
+    Hood<R> h = zero_hood<R>();
+    if (OP != kOpJacobiZero) {
+      const R* next = plane(x + 1 == n0 ? 0 : x + 1);
+      cross(c, next);
+      if (u + 1 < XL) corners(c, next);
+      h.c = b.c;
+      h.xp = c.c;
+      h.xm = a.c;
+      h.yp = b.yp;
+      h.ym = b.ym;
+      h.zp = b.zp;
+      h.zm = b.zm;
+      h.xpyp = c.yp;
+      h.xmym = a.ym;
+      h.xmyp = a.yp;
+      h.xpym = c.ym;
+      h.xpzp = c.zp;
+      h.xmzm = a.zm;
+      h.xmzp = a.zp;
+      h.xpzm = c.zm;
+      h.ypzp = b.pp;
+      h.ymzm = b.mm;
+      h.ymzp = b.mp;
+      h.ypzm = b.pm;
+    }
+    R px = R(0), A = R(0);
+    if (LOCAL) {
+      px = static_cast<R>(x) + G.org[0];
+      A = G.h2[0] * px * px;
+    }
+    const R fv = (OP == kOpResidual && T.C.sum) ? f[at] - fmean : f[at];
+    const R res = stencil_cell<R, OP, LOCAL, false>(T, h, fv, px, A, py, B, pz, C, pypz, omega, keep);
+    if constexpr (OP == kOpJacobiAcc)
+      T.acc[at] += static_cast<double>(res);
+    else
+      out[at] = static_cast<O>(res);
+    a = b;
+    b = c;
+  }
+}
+
+template <typename R, typename O, int OP, int XL>
+static void launch_columns_xl(const R* v, const R* f, O* out, const TileCoef<R>& T, R omega, R keep, hipStream_t s) {
+  const int* n = T.G.n;
+  int bz = 1;
+  while (bz < n[2] && bz < 64) bz <<= 1;
+  const dim3 block(bz, kThreads / bz);
+  const dim3 grid(ceil_div(n[2], bz), ceil_div(n[1], kThreads / bz), ceil_div(n[0], XL));
+  if (T.G.local)
+    k_stencil_columns<R, O, OP, true, XL><<<grid, block, 0, s>>>(v, f, out, T, omega, keep);
+  else
+    k_stencil_columns<R, O, OP, false, XL><<<grid, block, 0, s>>>(v, f, out, T, omega, keep);
+}
+
+// A level outside the 64-wide tiles, with the exact arithmetic whatever the path.  Two cells a thread on
+// levels that fill the device (192^3, line of sight z: 7.3 against 7.5 ms a solve), one on smaller ones,
+// which are short of wavefronts (64^3: 2.34 against 2.44 ms; a cell a thread with 19 loads took 2.38).
+template <typename R, typename O, int OP>
+static void launch_uneven(const R* v, const R* f, O* out, const LevelGeom<R>& G, R omega, R keep, hipStream_t s,
+                          double* acc = nullptr, Centre C = {}) {
+  TileCoef<R> T;
+  T.G = G;
+  T.K = G.local ? GlobalCoef<R>() : GlobalCoef<R>::make(G);
+  T.dinv = R(0);
+  T.acc = acc;
+  T.C = C;
+  if (!fills_alone(G.n)) {
+    launch_columns_xl<R, O, OP, 1>(v, f, out, T, omega, keep, s);
+    return;
+  }
+  if constexpr (std::is_same<R, double>::value) {
+    flex_tiles(G.n, T);
+    const int tiles = T.ztiles * T.ytiles;
+    // about 4096 blocks, of two planes or more
+    int xlen = static_cast<int>(static_cast<long>(G.n[0]) * tiles / 4096);
+    xlen = xlen < 2 ? 2 : xlen;
+    if (xlen > G.n[0]) xlen = G.n[0];
+    const unsigned grid = static_cast<unsigned>(tiles * ((G.n[0] + xlen - 1) / xlen));
+    if (G.local)
+      k_stencil_tiled<R, O, OP, 8, true, false, true><<<grid, 256, 0, s>>>(v, f, out, T, omega, keep, xlen);
+    else
+      k_stencil_tiled<R, O, OP, 8, false, false, true><<<grid, 256, 0, s>>>(v, f, out, T, omega, keep, xlen);
+  } else {
+    launch_columns_xl<R, O, OP, 2>(v, f, out, T, omega, keep, s);
   }
 }
 
@@ -1735,28 +1893,32 @@ static int launch_jacobi(const R* v, const R* f, R* out, const LevelGeom<R>& G, 
                          bool zero_in, hipStream_t s, int timer = -1, bool fast = false,
                          double* acc = nullptr, bool* fused = nullptr) {
   const size_t total = static_cast<size_t>(G.n[0]) * G.n[1] * G.n[2];
-  dim3 block, grid;
-  generic_shape(G.n, block, grid);
   if (fused) *fused = false;
   // a sweep added into the FP64 iterate is another kernel (kOpJacobiAcc): not in the timer
-  const bool into_acc = acc && !zero_in && tiled_ok(G.n) && fast && std::is_same<R, float>::value;
+  const bool tiled = tiled_ok(G.n);
+  const bool into_acc = acc && !zero_in && (!tiled || fast) && std::is_same<R, float>::value;
   if (into_acc) timer = -1;
+  constexpr bool kFast = std::is_same<R, float>::value;
   timer_before(timer, s);
   if (into_acc) {
-    launch_tiled<R, R, kOpJacobiAcc, std::is_same<R, float>::value>(v, f, out, G, omega, keep, s, acc);
+    if (tiled)
+      launch_tiled<R, R, kOpJacobiAcc, kFast>(v, f, out, G, omega, keep, s, acc);
+    else
+      launch_uneven<R, R, kOpJacobiAcc>(v, f, out, G, omega, keep, s, acc);
     if (fused) *fused = true;
-  } else if (zero_in && tiled_ok(G.n) && fast)
-    launch_tiled<R, R, kOpJacobiZero, std::is_same<R, float>::value>(v, f, out, G, omega, keep, s);
-  else if (zero_in && tiled_ok(G.n))
+  } else if (!tiled && zero_in) {
+    launch_uneven<R, R, kOpJacobiZero>(v, f, out, G, omega, keep, s);
+  } else if (!tiled) {
+    launch_uneven<R, R, kOpJacobi>(v, f, out, G, omega, keep, s);
+  } else if (zero_in && fast) {
+    launch_tiled<R, R, kOpJacobiZero, kFast>(v, f, out, G, omega, keep, s);
+  } else if (zero_in) {
     launch_tiled<R, R, kOpJacobiZero, false>(v, f, out, G, omega, keep, s);
-  else if (zero_in)
-    k_jacobi<R, true><<<grid, block, 0, s>>>(v, f, out, G, omega, keep);
-  else if (tiled_ok(G.n) && fast)
-    launch_tiled<R, R, kOpJacobi, std::is_same<R, float>::value>(v, f, out, G, omega, keep, s);
-  else if (tiled_ok(G.n))
+  } else if (fast) {
+    launch_tiled<R, R, kOpJacobi, kFast>(v, f, out, G, omega, keep, s);
+  } else {
     launch_tiled<R, R, kOpJacobi, false>(v, f, out, G, omega, keep, s);
-  else
-    k_jacobi<R, false><<<grid, block, 0, s>>>(v, f, out, G, omega, keep);
+  }
   // algorithmic traffic: read v (unless zero) and f, write the new iterate
   timer_after(timer, s, static_cast<double>(total) * sizeof(R) * (zero_in ? 2 : 3));
   PRH_LAUNCHED();
@@ -1772,9 +1934,7 @@ static int launch_residual(const R* v, const R* f, O* r, const LevelGeom<R>& G, 
   } else if (tiled_ok(G.n)) {
     launch_tiled<R, O, kOpResidual, false>(v, f, r, G, R(0), R(0), s, nullptr, C);
   } else {
-    dim3 block, grid;
-    generic_shape(G.n, block, grid);
-    k_residual<R, O><<<grid, block, 0, s>>>(v, f, r, G, C);
+    launch_uneven<R, O, kOpResidual>(v, f, r, G, R(0), R(0), s, nullptr, C);
   }
   PRH_LAUNCHED();
   return PRH_OK;
@@ -1905,7 +2065,7 @@ struct Solver {
   }
   bool grouped(int l) const {
     int nn[3] = {static_cast<int>(n(l)[0]), static_cast<int>(n(l)[1]), static_cast<int>(n(l)[2])};
-    return count > 1 && !tiled_ok(nn);
+    return count > 1 && !tiled_ok(nn) && !fills_alone(nn);
   }
 
   void setup(Hierarchy* h, const R* boxsize, const R* boxcenter, R beta, R damping, int nit,
