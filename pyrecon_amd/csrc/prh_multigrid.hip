@@ -884,6 +884,13 @@ inline int rows_xlen(const int* n) {
 
 inline bool tiled_ok(const int* n) { return n[2] % kTileZ == 0 && n[1] % kTileY == 0 && n[0] >= 1; }
 
+// Levels of up to 64^3 cells give the blocks of the tiles a few planes each: a sweep there is a chain of
+// barriers.  A cell a thread without LDS is faster (FP64 solve of 64^3 with its 32^3: 1.99 against 2.17
+// ms, of 256^3 12.6 against 13.0; FP32 of 64^3 1.55
+// against 1.62); at 128^3 it is slower (256^3 then 13.4 ms).
+constexpr size_t kShortTiles = size_t(64) * 64 * 64;
+inline bool short_tiles(const int* n) { return static_cast<size_t>(n[0]) * n[1] * n[2] <= kShortTiles; }
+
 // Levels that the 64-wide tiles do not cover (rows no multiple of 64 cells, planes no multiple of 8
 // rows) and that fill the device by themselves.  FP64 ones go through FLEX tiles: a solve of 320 x 384 x
 // 224 takes 24.4 ms (29.5 with the columns below, 35.1 with a cell a thread).  FP32 ones, half the size
@@ -1035,7 +1042,7 @@ static void launch_tiled(const R* v, const R* f, O* out, const LevelGeom<R>& G, 
 // its neighbourhood in registers (11.5 loads a cell for XL = 4 instead of 19) and the parts of the
 // coefficients that do not change along x.  No LDS and no barrier: neighbouring threads' loads meet in
 // L1, and the levels lie in L2 or the last-level cache.
-template <typename R, typename O, int OP, bool LOCAL, int XL>
+template <typename R, typename O, int OP, bool LOCAL, int XL, bool FAST>
 __global__ __launch_bounds__(kThreads) void k_stencil_columns(const R* __restrict__ v, const R* __restrict__ f,
                                                               O* __restrict__ out, TileCoef<R> T, R omega,
                                                               R keep) {
@@ -1116,7 +1123,7 @@ __global__ __launch_bounds__(kThreads) void k_stencil_columns(const R* __restric
       A = G.h2[0] * px * px;
     }
     const R fv = (OP == kOpResidual && T.C.sum) ? f[at] - fmean : f[at];
-    const R res = stencil_cell<R, OP, LOCAL, false>(T, h, fv, px, A, py, B, pz, C, pypz, omega, keep);
+    const R res = stencil_cell<R, OP, LOCAL, FAST>(T, h, fv, px, A, py, B, pz, C, pypz, omega, keep);
     if constexpr (OP == kOpJacobiAcc)
       T.acc[at] += static_cast<double>(res);
     else
@@ -1126,7 +1133,7 @@ __global__ __launch_bounds__(kThreads) void k_stencil_columns(const R* __restric
   }
 }
 
-template <typename R, typename O, int OP, int XL>
+template <typename R, typename O, int OP, int XL, bool FAST = false>
 static void launch_columns_xl(const R* v, const R* f, O* out, const TileCoef<R>& T, R omega, R keep, hipStream_t s) {
   const int* n = T.G.n;
   int bz = 1;
@@ -1134,25 +1141,26 @@ static void launch_columns_xl(const R* v, const R* f, O* out, const TileCoef<R>&
   const dim3 block(bz, kThreads / bz);
   const dim3 grid(ceil_div(n[2], bz), ceil_div(n[1], kThreads / bz), ceil_div(n[0], XL));
   if (T.G.local)
-    k_stencil_columns<R, O, OP, true, XL><<<grid, block, 0, s>>>(v, f, out, T, omega, keep);
+    k_stencil_columns<R, O, OP, true, XL, FAST><<<grid, block, 0, s>>>(v, f, out, T, omega, keep);
   else
-    k_stencil_columns<R, O, OP, false, XL><<<grid, block, 0, s>>>(v, f, out, T, omega, keep);
+    k_stencil_columns<R, O, OP, false, XL, FAST><<<grid, block, 0, s>>>(v, f, out, T, omega, keep);
 }
 
-// A level outside the 64-wide tiles, with the exact arithmetic whatever the path.  Two cells a thread on
-// levels that fill the device (192^3, line of sight z: 7.3 against 7.5 ms a solve), one on smaller ones,
-// which are short of wavefronts (64^3: 2.34 against 2.44 ms; a cell a thread with 19 loads took 2.38).
-template <typename R, typename O, int OP>
+// A level outside the 64-wide tiles, or too small for them; FAST as the tiles would take it (the exact
+// arithmetic outside them).  Two cells a thread on levels that fill the device (192^3, line of sight z:
+// 7.3 against 7.5 ms a solve), one on smaller ones, which are short of wavefronts (64^3: 2.34 against
+// 2.44 ms; a cell a thread with 19 loads took 2.38).
+template <typename R, typename O, int OP, bool FAST = false>
 static void launch_uneven(const R* v, const R* f, O* out, const LevelGeom<R>& G, R omega, R keep, hipStream_t s,
                           double* acc = nullptr, Centre C = {}) {
   TileCoef<R> T;
   T.G = G;
   T.K = G.local ? GlobalCoef<R>() : GlobalCoef<R>::make(G);
-  T.dinv = R(0);
+  T.dinv = FAST && !G.local ? R(1) / T.K.d : R(0);
   T.acc = acc;
   T.C = C;
   if (!fills_alone(G.n)) {
-    launch_columns_xl<R, O, OP, 1>(v, f, out, T, omega, keep, s);
+    launch_columns_xl<R, O, OP, 1, FAST>(v, f, out, T, omega, keep, s);
     return;
   }
   if constexpr (std::is_same<R, double>::value) {
@@ -1375,12 +1383,8 @@ __global__ __launch_bounds__(kThreads) void k_restrict_quads(const float* __rest
 // Trilinear prolongation from the coarse mesh (c0, c1, c2) to the fine mesh,
 // one thread per fine cell (src/multigrid.c:177-205), either overwriting the
 // fine value or adding to it (the V-cycle correction, src/multigrid.c:296).
-template <typename RC, typename R, bool ADD, typename I>
-__device__ __forceinline__ void prolong_at(const RC* __restrict__ uc, R* __restrict__ fine,
-                                           int c0, int c1, int c2, I i) {
-  const int F1 = 2 * c1, F2 = 2 * c2;
-  int X, Y, Z;
-  unflatten(i, F1, F2, X, Y, Z);
+template <typename RC, typename R>
+__device__ __forceinline__ R prolong_value(const RC* __restrict__ uc, int c0, int c1, int c2, int X, int Y, int Z) {
   const int jx = X >> 1, jy = Y >> 1, jz = Z >> 1;
   const size_t s0 = static_cast<size_t>(c1) * c2, s1 = static_cast<size_t>(c2);
   const size_t x0 = jx * s0, xp = (jx + 1 == c0 ? 0 : jx + 1) * s0;
@@ -1403,6 +1407,15 @@ __device__ __forceinline__ void prolong_at(const RC* __restrict__ uc, R* __restr
             R(8);
       break;
   }
+  return val;
+}
+
+template <typename RC, typename R, bool ADD, typename I>
+__device__ __forceinline__ void prolong_at(const RC* __restrict__ uc, R* __restrict__ fine,
+                                           int c0, int c1, int c2, I i) {
+  int X, Y, Z;
+  unflatten(i, 2 * c1, 2 * c2, X, Y, Z);
+  const R val = prolong_value<RC, R>(uc, c0, c1, c2, X, Y, Z);
   if (ADD)
     fine[i] += val;
   else
@@ -1666,217 +1679,472 @@ struct CoarseArgs {
 };
 
 // All single-workgroup levels live in LDS during the call: iterate, its
-// ping-pong partner, source and the per-cell g of each level (at most
-// 4096 (1 + 1/8 + 1/64 + 1/512) cells: 150 KB in FP64).
+// ping-pong partner and source of each level (at most 4096 (1 + 1/8 + 1/64 +
+// 1/512) cells: 112 KB in FP64).
 constexpr int kCoarseLds = 4682;
 
-// The cells of one level that a thread visits (i = threadIdx.x + kCoarseThreads u),
-// with their coordinates and the offsets of their periodic neighbours, worked
-// out once per visit of the level rather than once per sweep.  Offsets are
-// below the level's size in magnitude, so they pack in pairs of 16 bits.
-constexpr int kCoarsePer = static_cast<int>((kCoarseCells + kCoarseThreads - 1) / kCoarseThreads);
-static_assert(kCoarseCells <= 32767, "neighbour offsets are packed in 16 bits");
-struct CoarseCells {
-  int total;
-  int xy[kCoarsePer];  // ix | iy << 16
-  int z[kCoarsePer];
-  int ox[kCoarsePer];  // offset of x + 1 in the low half, of x - 1 in the high half
-  int oy[kCoarsePer];
-  int oz[kCoarsePer];
+// a / d, correctly rounded, from y = 1 / d correctly rounded: two corrections by fused multiply-adds
+// (Markstein, IBM J. Res. Dev. 34, 1990: with y correctly rounded, d's significand not all ones and q
+// within one unit in the last place, q + y (a - q d) is the rounded quotient).  Quotients near the ends
+// of the exponent range, zeros, infinities and NaN take the division; `reciprocal` returns NaN for a d
+// outside the theorem.
+template <typename R>
+__device__ __forceinline__ R reciprocal(R d) {
+  if constexpr (sizeof(R) == 8) {
+    const bool ones = (__double_as_longlong(d) & 0xfffffffffffffll) == 0xfffffffffffffll;
+    return ones || !(fabs(d) > 0x1p-400 && fabs(d) < 0x1p400) ? static_cast<R>(__builtin_nan("")) : R(1) / d;
+  } else {
+    const bool ones = (__float_as_int(d) & 0x7fffff) == 0x7fffff;
+    return ones || !(fabsf(d) > 0x1p-50f && fabsf(d) < 0x1p50f) ? static_cast<R>(__builtin_nanf("")) : R(1) / d;
+  }
+}
+__device__ __forceinline__ double divided(double a, double d, double y) {
+  const double q0 = a * y;
+  if (!(fabs(q0) > 0x1p-500 && fabs(q0) < 0x1p500)) return a / d;
+  const double q1 = fma(fma(-q0, d, a), y, q0);
+  return fma(fma(-q1, d, a), y, q1);
+}
+__device__ __forceinline__ float divided(float a, float d, float y) {
+  const float q0 = a * y;
+  if (!(fabsf(q0) > 0x1p-50f && fabsf(q0) < 0x1p50f)) return a / d;
+  const float q1 = fmaf(fmaf(-q0, d, a), y, q0);
+  return fmaf(fmaf(-q1, d, a), y, q1);
+}
+
+// XL consecutive x of one (y, z) of a level in LDS, for one thread: offsets of the neighbours and the
+// operator's coefficients, worked out once per visit of the level (five sweeps, and the residual on the
+// way down).  The x neighbourhood moves through registers, 11.5 LDS reads a cell for XL = 4.
+template <typename R, int XL>
+struct CoarseColumn {
+  int live;                  // cells of this column, 0 for a thread without one
+  int c, yp, ym, zp, zm, s0; // (y, z) offset in a plane, those of its neighbours, plane size
+  int ix, x0, xm, xp;        // first x; offsets of its plane, the one before it and the one after the last
+  R py, pz, pypz, px0;
+  R g[XL], y[XL];            // g and 1 / d: the divisions; the rest is a few products
+
+  __device__ __forceinline__ void set(const LevelGeom<R>& G, int t) {
+    const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
+    s0 = n1 * n2;
+    int group, iy, iz;
+    unflatten(t, n1, n2, group, iy, iz);
+    x0 = group * XL;
+    live = x0 < n0 ? min(XL, n0 - x0) : 0;
+    if (!live) return;
+    c = iy * n2 + iz;
+    yp = (iy + 1 == n1 ? 0 : iy + 1) * n2 + iz;
+    ym = (iy == 0 ? n1 - 1 : iy - 1) * n2 + iz;
+    zp = (iz + 1 == n2 ? 0 : iz + 1) - iz;
+    zm = (iz == 0 ? n2 - 1 : iz - 1) - iz;
+    xm = (x0 == 0 ? n0 - 1 : x0 - 1) * s0;
+    xp = (x0 + live == n0 ? 0 : x0 + live) * s0;
+    x0 *= s0;
+#pragma unroll
+    for (int u = 0; u < XL; u++) {
+      const Coef<R> k = cell_coef(G, group * XL + u, iy, iz);
+      if (u == 0) px0 = k.px, py = k.py, pz = k.pz;
+      g[u] = k.g;
+      y[u] = reciprocal(R(2) * (k.cx + k.cy + k.cz));
+    }
+    ix = group * XL;
+    pypz = py * pz;
+  }
+
+  struct Plane {
+    R c, yp, ym, zp, zm, pp, pm, mp, mm;
+  };
+  __device__ __forceinline__ Plane plane(const R* u, bool corners) const {
+    Plane P;
+    P.c = u[c];
+    P.yp = u[yp];
+    P.ym = u[ym];
+    P.zp = u[c + zp];
+    P.zm = u[c + zm];
+    P.pp = P.pm = P.mp = P.mm = R(0);
+    if (corners) {
+      P.pp = u[yp + zp];
+      P.pm = u[yp + zm];
+      P.mp = u[ym + zp];
+      P.mm = u[ym + zm];
+    }
+    return P;
+  }
+
+  // One sweep (or, RESIDUAL, the residual) of the column from `in` to `out`, with the generic kernels'
+  // expressions in their order.
+  template <bool RESIDUAL>
+  __device__ __forceinline__ void apply(const LevelGeom<R>& G, const R* in, const R* src, R* out, R omega, R keep,
+                                        bool zero_in) const {
+    if (!live) return;
+    const int local = G.local;
+    Plane a{}, b{}, n{};
+    if (!zero_in) {
+      a = plane(in + xm, false);
+      b = plane(in + x0, true);
+    }
+#pragma unroll
+    for (int u = 0; u < XL; u++) {
+      if (u >= live) break;
+      if (!zero_in) n = plane(in + (u + 1 == live ? xp : x0 + (u + 1) * s0), u + 1 < XL);
+      const R px = local ? static_cast<R>(ix + u) + G.org[0] : px0;
+      const R cx = G.ih2[0] + g[u] * px * px, cy = G.ih2[1] + g[u] * py * py, cz = G.ih2[2] + g[u] * pz * pz;
+      const R d = R(2) * (cx + cy + cz);
+      const R t0 = cx * (n.c + a.c);
+      const R t1 = cy * (b.yp + b.ym);
+      const R t2 = cz * (b.zp + b.zm);
+      const R t3 = g[u] / R(2) *
+                   (px * py * (n.yp + a.ym - a.yp - n.ym) + px * pz * (n.zp + a.zm - a.zp - n.zm) +
+                    pypz * (b.pp + b.mm - b.mp - b.pm));
+      R drift = R(0);
+      if (local) drift = g[u] * (px * (n.c - a.c) + py * (b.yp - b.ym) + pz * (b.zp - b.zm));
+      const int at = x0 + u * s0 + c;
+      const R fv = src[at];
+      if constexpr (RESIDUAL) {
+        R av = d * b.c - (t0 + t1 + t2 + t3);
+        if (local) av -= drift;
+        out[at] = fv - av;
+      } else {
+        R jac = fv + t0 + t1 + t2 + t3;
+        if (local) jac += drift;
+        jac = divided(jac, d, y[u]);
+        out[at] = keep * b.c + omega * jac;
+      }
+      a = b;
+      b = n;
+    }
+  }
 };
 
-__device__ __forceinline__ int pack16(int lo, int hi) { return (lo & 0xffff) | (hi << 16); }
-__device__ __forceinline__ int lo16(int p) { return static_cast<int>(static_cast<int16_t>(p & 0xffff)); }
-__device__ __forceinline__ int hi16(int p) { return p >> 16; }
-
-template <typename R>
-__device__ __forceinline__ CoarseCells coarse_cells(const LevelGeom<R>& G) {
-  const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2], s0 = n1 * n2;
-  CoarseCells C;
-  C.total = n0 * s0;
-#pragma unroll
-  for (int u = 0; u < kCoarsePer; u++) {
-    const int i = threadIdx.x + kCoarseThreads * u;
-    int ix = 0, iy = 0, iz = 0;
-    if (i < C.total) unflatten(i, n1, n2, ix, iy, iz);
-    const int xp = ix + 1 == n0 ? 0 : ix + 1, xm = ix == 0 ? n0 - 1 : ix - 1;
-    const int yp = iy + 1 == n1 ? 0 : iy + 1, ym = iy == 0 ? n1 - 1 : iy - 1;
-    const int zp = iz + 1 == n2 ? 0 : iz + 1, zm = iz == 0 ? n2 - 1 : iz - 1;
-    C.xy[u] = ix | (iy << 16);
-    C.z[u] = iz;
-    C.ox[u] = pack16((xp - ix) * s0, (xm - ix) * s0);
-    C.oy[u] = pack16((yp - iy) * n2, (ym - iy) * n2);
-    C.oz[u] = pack16(zp - iz, zm - iz);
-  }
-  return C;
-}
-
-// gather_hood() of cell u of C (the same neighbours)
-template <typename R>
-__device__ __forceinline__ Hood<R> coarse_hood(const R* v, const CoarseCells& C, int u, int i) {
-  const int xp = lo16(C.ox[u]), xm = hi16(C.ox[u]), yp = lo16(C.oy[u]), ym = hi16(C.oy[u]);
-  const int zp = lo16(C.oz[u]), zm = hi16(C.oz[u]);
-  const R* c = v + i;
-  Hood<R> h;
-  h.c = c[0];
-  h.xp = c[xp];
-  h.xm = c[xm];
-  h.yp = c[yp];
-  h.ym = c[ym];
-  h.zp = c[zp];
-  h.zm = c[zm];
-  h.xpyp = c[xp + yp];
-  h.xmym = c[xm + ym];
-  h.xmyp = c[xm + yp];
-  h.xpym = c[xp + ym];
-  h.xpzp = c[xp + zp];
-  h.xmzm = c[xm + zm];
-  h.xmzp = c[xm + zp];
-  h.xpzm = c[xp + zm];
-  h.ypzp = c[yp + zp];
-  h.ymzm = c[ym + zm];
-  h.ymzp = c[ym + zp];
-  h.ypzm = c[yp + zm];
-  return h;
-}
-
-template <typename R>
-__device__ __forceinline__ Coef<R> coarse_coef(const LevelGeom<R>& G, const CoarseCells& C, int u,
-                                               const R* gtab, int i) {
-  return cell_coef_g(G, C.xy[u] & 0xffff, C.xy[u] >> 16, C.z[u], gtab[i]);
-}
-
-template <typename R>
-__device__ __forceinline__ void cw_jacobi(const LevelGeom<R>& G, const CoarseCells& C, const R* in,
-                                          const R* src, R* out, const R* gtab, R omega, R keep,
-                                          bool zero_in) {
-#pragma unroll
-  for (int u = 0; u < kCoarsePer; u++) {
-    const int i = threadIdx.x + kCoarseThreads * u;
-    if (i < C.total) {
-      const Coef<R> k = coarse_coef(G, C, u, gtab, i);
-      const Hood<R> h = zero_in ? zero_hood<R>() : coarse_hood(in, C, u, i);
-      out[i] = jacobi_update(k, h, src[i], omega, keep, G.local);
-    }
-  }
-  __syncthreads();
-}
-
-template <typename R>
-__device__ __forceinline__ void cw_smooth(const LevelGeom<R>& G, const CoarseCells& C, R*& cur,
-                                          R*& alt, const R* src, const R* gtab, int niter,
-                                          R omega, R keep, bool zero_start) {
-  if (niter <= 0) {
-    if (zero_start) {
-      for (int i = threadIdx.x; i < C.total; i += kCoarseThreads) cur[i] = R(0);
-      __syncthreads();
-    }
-    return;
-  }
+// One visit of a level: `niter` sweeps, the iterate moving between cur and alt, then the residual into
+// the spare of the two if `residual`.  HELD: every column has a thread of its own, which keeps the
+// coefficients; otherwise the threads go round and work them out again.
+template <typename R, int XL, bool HELD>
+__device__ void coarse_visit(const LevelGeom<R>& G, R* cur, R* alt, const R* src, int niter, R omega, R keep,
+                             bool zero_start, bool residual) {
+  CoarseColumn<R, XL> C;
+  const int columns = G.n[1] * G.n[2] * ((G.n[0] + XL - 1) / XL);
+  if (HELD) C.set(G, threadIdx.x);
   for (int it = 0; it < niter; it++) {
-    cw_jacobi(G, C, cur, src, alt, gtab, omega, keep, zero_start && it == 0);
-    R* t = cur;
+    for (int t = threadIdx.x; t < columns; t += kCoarseThreads) {
+      if (!HELD) C.set(G, t);
+      C.template apply<false>(G, cur, src, alt, omega, keep, zero_start && it == 0);
+    }
+    __syncthreads();
+    R* s = cur;
     cur = alt;
-    alt = t;
+    alt = s;
+  }
+  if (residual) {
+    for (int t = threadIdx.x; t < columns; t += kCoarseThreads) {
+      if (!HELD) C.set(G, t);
+      C.template apply<true>(G, cur, src, alt, omega, keep, false);
+    }
+    __syncthreads();
   }
 }
 
-// src/multigrid.c:270-300 from relative level 0 to the coarsest, unrolled over
-// the (at most kMaxCoarse) levels.  Level 0's iterate and source are read from
-// global memory at the start and its iterate written back at the end; every
-// other step stays in LDS.  Per cell the arithmetic is the generic kernels'
-// (g computed once per call by cell_coef() itself), so the bits are the same.
+// The longest columns that still give every thread its own: small levels take one cell a thread.
+template <typename R>
+__device__ __forceinline__ void coarse_level(const LevelGeom<R>& G, R* cur, R* alt, const R* src, int niter,
+                                             R omega, R keep, bool zero_start, bool residual) {
+  const int plane = G.n[1] * G.n[2];
+  if (plane * G.n[0] <= kCoarseThreads)
+    coarse_visit<R, 1, true>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
+  else if (plane * ((G.n[0] + 1) / 2) <= kCoarseThreads)
+    coarse_visit<R, 2, true>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
+  else if (plane * ((G.n[0] + 3) / 4) <= kCoarseThreads)
+    coarse_visit<R, 4, true>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
+  else
+    coarse_visit<R, 2, false>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
+}
+
+// src/multigrid.c:270-300 from relative level 0 to the coarsest.  Level 0's
+// iterate and source are read from global memory at the start and its iterate
+// written back at the end; every other step stays in LDS.  Per cell the
+// expressions are the generic kernels', so the bits are the same.
+// Bound: one CU's arithmetic on a top level of 4096 cells (22 evaluations of 64
+// wavefronts of cells at 58 instructions are 34 us in FP64; 60 us a call, 42 in
+// FP32), latency on one of 512 (14.5 us a call), where the legs above leave it.
 template <typename R>
 __global__ __launch_bounds__(kCoarseThreads) void k_vcycle_coarse(CoarseArgs<R> A) {
-  __shared__ R sv[kCoarseLds], st[kCoarseLds], sf[kCoarseLds], sg[kCoarseLds];
+  __shared__ R sv[kCoarseLds], st[kCoarseLds], sf[kCoarseLds];
   const int job = blockIdx.x;
   const int nl = A.nlev;
-  int off[kMaxCoarse];
+  const auto cells = [&](int m) {
+    const LevelGeom<R>& G = A.L[job][m].G;
+    return G.n[0] * G.n[1] * G.n[2];
+  };
   {
-    int o = 0;
-#pragma unroll
-    for (int m = 0; m < kMaxCoarse; m++) {
-      off[m] = o;
-      if (m < nl) {
-        const LevelGeom<R>& G = A.L[job][m].G;
-        o += G.n[0] * G.n[1] * G.n[2];
-      }
-    }
-  }
-  {
-    const LevelGeom<R>& G = A.L[job][0].G;
-    const int total = G.n[0] * G.n[1] * G.n[2];
+    const int total = cells(0);
     const R* c0 = A.cur0[job];
     const R* f0 = A.src0[job];
     for (int i = threadIdx.x; i < total; i += kCoarseThreads) {
       sf[i] = f0[i];
-      if (!A.zero_start) sv[i] = c0[i];
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < kMaxCoarse; m++) {
-    if (m >= nl) break;
-    const LevelGeom<R>& G = A.L[job][m].G;
-    const int total = G.n[0] * G.n[1] * G.n[2];
-    for (int i = threadIdx.x; i < total; i += kCoarseThreads) {
-      int ix, iy, iz;
-      unflatten(i, G.n[1], G.n[2], ix, iy, iz);
-      sg[off[m] + i] = cell_coef(G, ix, iy, iz).g;
+      sv[i] = !A.zero_start || A.niter <= 0 ? c0[i] : R(0);
     }
   }
   __syncthreads();
-  R* cur[kMaxCoarse];
-  R* alt[kMaxCoarse];
-#pragma unroll
-  for (int m = 0; m < kMaxCoarse; m++) {
-    cur[m] = sv + off[m];
-    alt[m] = st + off[m];
-  }
-#pragma unroll
-  for (int m = 0; m < kMaxCoarse; m++) {
-    if (m >= nl) break;
+  // after the sweeps of a visit the iterate is in st if niter is odd; after the way down and up, in sv
+  const bool odd = A.niter > 0 && (A.niter & 1);
+  int off = 0;
+  for (int m = 0; m < nl; m++) {
     const LevelGeom<R>& G = A.L[job][m].G;
-    const R* src = sf + off[m];
-    const R* gt = sg + off[m];
-    const CoarseCells C = coarse_cells(G);
-    cw_smooth(G, C, cur[m], alt[m], src, gt, A.niter, A.omega, A.keep, m > 0 || A.zero_start);
-    if (m + 1 < nl) {
-#pragma unroll
-      for (int u = 0; u < kCoarsePer; u++) {
-        const int i = threadIdx.x + kCoarseThreads * u;
-        if (i < C.total) {
-          const Coef<R> k = coarse_coef(G, C, u, gt, i);
-          const Hood<R> h = coarse_hood(cur[m], C, u, i);
-          alt[m][i] = residual_value(k, h, src[i], G.local);
-        }
-      }
-      __syncthreads();
-      const int ctotal = (G.n[0] / 2) * (G.n[1] / 2) * (G.n[2] / 2);
-      R* fc = sf + off[m + 1];
-      for (int j = threadIdx.x; j < ctotal; j += kCoarseThreads)
-        restrict_at<R, R>(alt[m], fc, G.n[0], G.n[1], G.n[2], j);
+    const bool down = m + 1 < nl, zero = m > 0 || A.zero_start;
+    const int total = cells(m);
+    if (zero && A.niter <= 0) {
+      for (int i = threadIdx.x; i < total; i += kCoarseThreads) sv[off + i] = R(0);
       __syncthreads();
     }
+    coarse_level(G, sv + off, st + off, sf + off, A.niter, A.omega, A.keep, zero, down);
+    if (!down) break;
+    const R* r = (odd ? sv : st) + off;
+    const int ctotal = cells(m + 1);
+    for (int j = threadIdx.x; j < ctotal; j += kCoarseThreads)
+      restrict_at<R, R>(r, sf + off + total, G.n[0], G.n[1], G.n[2], j);
+    __syncthreads();
+    off += total;
   }
-#pragma unroll
-  for (int m = kMaxCoarse - 1; m >= 0; m--) {
-    if (m >= nl) continue;
+  for (int m = nl - 1; m >= 0; m--) {
     const LevelGeom<R>& G = A.L[job][m].G;
+    const int total = cells(m);
+    R* cur = (odd ? st : sv) + off;
     if (m + 1 < nl) {
       const LevelGeom<R>& Gc = A.L[job][m + 1].G;
-      const int ftotal = 8 * Gc.n[0] * Gc.n[1] * Gc.n[2];
+      // the coarser level's iterate went there and back: niter sweeps down and up
+      const int ftotal = 8 * cells(m + 1);
       for (int i = threadIdx.x; i < ftotal; i += kCoarseThreads)
-        prolong_at<R, R, true>(cur[m + 1], cur[m], Gc.n[0], Gc.n[1], Gc.n[2], i);
+        prolong_at<R, R, true>(sv + off + total, cur, Gc.n[0], Gc.n[1], Gc.n[2], i);
       __syncthreads();
     }
-    cw_smooth(G, coarse_cells(G), cur[m], alt[m], sf + off[m], sg + off[m], A.niter, A.omega, A.keep,
-              false);
+    coarse_level(G, cur, (odd ? sv : st) + off, sf + off, A.niter, A.omega, A.keep, false, false);
+    if (m > 0) off -= cells(m - 1);
   }
   {
-    const LevelGeom<R>& G = A.L[job][0].G;
-    const int total = G.n[0] * G.n[1] * G.n[2];
+    const int total = cells(0);
     R* c0 = A.cur0[job];
-    for (int i = threadIdx.x; i < total; i += kCoarseThreads) c0[i] = cur[0][i];
+    for (int i = threadIdx.x; i < total; i += kCoarseThreads) c0[i] = sv[i];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Small levels a V-cycle leg at a time.  A sweep of 64^3 cells is 0.4 us of
+// arithmetic in a launch of 4 to 8 us, so here one launch takes a whole leg:
+//   down: up to five sweeps (from zero or from the iterate), the residual and
+//         its restriction;
+//   up:   the coarser level's correction and up to five sweeps.
+// A workgroup owns a tile of BT^3 cells and keeps in LDS the iterate (twice) and
+// the source of every cell its results depend on (a sweep looks one cell
+// further): the region it sweeps shrinks by one cell a side per sweep, and
+// neighbouring workgroups repeat each other's halo.  Same expressions per cell,
+// same bits.  The sweeps share one loop: code that is run once per launch is
+// bound by the instruction fetch (unrolled, a leg on 16^3 took 16 us up and 25 us
+// down instead of 12 and 16).  Bound: latency, that of one trip to memory, then of
+// the passes (FP64 divisions).  A V-cycle's 16^3 level took 45 us of one workgroup
+// (below) or 28 us of launches.  Solves with and without legs: 64^3 FP64 1.79 and
+// 1.97 ms (one workgroup from 16^3 down: 2.09), 128^3 mixed 2.89 and 3.08.
+// ---------------------------------------------------------------------------
+constexpr int kLegSweeps = 5;
+// Levels of up to kLegCells cells (27^3; with 32^3 the repeated halos cost more than the launches: FP64
+// solve of 64^3 2.17 ms against 1.98), and in one workgroup below kCoarseOne.
+constexpr size_t kLegCells = 20000, kCoarseOne = 1024;
+constexpr int kLegTile = 4;
+
+template <typename R>
+struct LegJob {
+  TileCoef<R> T;
+  const R* in;    // iterate (not read when it starts from zero)
+  const R* src;
+  R* out;         // iterate after the leg (not `in`)
+  R* coarse;      // down: the coarser level's source; up: its correction
+};
+template <typename R>
+struct LegArgs {
+  int niter, zero_start;
+  int tx, ty, tz;  // tiles
+  R omega, keep;
+  LegJob<R> job[kMaxGroup];
+};
+
+template <typename R, bool DOWN>
+struct LegTile {
+  static constexpr int BT = kLegTile;
+  // cells around the tile: the residual's restriction looks one cell below the tile, the residual one
+  // further on both sides, and each sweep one more
+  static constexpr int kLo = DOWN ? 2 : 0, kHi = DOWN ? 1 : 0;
+  static constexpr int kPadLo = kLo + kLegSweeps, kPadHi = kHi + kLegSweeps;
+  static constexpr int kV = BT + kPadLo + kPadHi;  // staged extent of the iterate
+  static constexpr int kF = kV - 2;                // and of the source
+  static constexpr int kC = DOWN ? 0 : BT / 2 + 7;  // and of the correction on the coarser level
+  static constexpr size_t lds = sizeof(R) * (2 * static_cast<size_t>(kV) * kV * kV + static_cast<size_t>(kF) * kF * kF +
+                                             static_cast<size_t>(kC) * kC * kC);
+};
+constexpr int kLegThreads = 1024;
+
+__device__ __forceinline__ int wrap_once(int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; }
+
+// One sweep (OP kOpJacobi, kOpJacobiZero) or the residual from v to w, over the tile and lo cells below,
+// hi above: two cells along x a thread and round.
+template <typename R, bool DOWN, int OP, bool LOCAL, bool FAST>
+__device__ __forceinline__ void leg_pass(const TileCoef<R>& T, const R* v, const R* f, R* w, int lo, int hi, int x0,
+                                         int y0, int z0, R omega, R keep) {
+  using L = LegTile<R, DOWN>;
+  constexpr int BT = kLegTile, NV = L::kV, NF = L::kF;
+  const LevelGeom<R>& G = T.G;
+  const int E = BT + lo + hi, dv = L::kPadLo - lo;
+  const int columns = E * E * ((E + 1) / 2);
+  const float inv = 1.f / static_cast<float>(E);
+#pragma unroll 1
+  for (int t = threadIdx.x; t < columns; t += kLegThreads) {
+    // t / E and its quotient by E, exact below 2^22 with the half added
+    const int tj = static_cast<int>((static_cast<float>(t) + 0.5f) * inv), k = t - tj * E;
+    const int ti = static_cast<int>((static_cast<float>(tj) + 0.5f) * inv), j = tj - ti * E, i = 2 * ti;
+    R py = R(0), B = R(0), pz = R(0), C = R(0), pypz = T.K.pypz;
+    if (LOCAL) {
+      py = static_cast<R>(wrap_once(y0 - lo + j, G.n[1])) + G.org[1];
+      B = G.h2[1] * py * py;
+      pz = static_cast<R>(wrap_once(z0 - lo + k, G.n[2])) + G.org[2];
+      C = G.h2[2] * pz * pz;
+      pypz = py * pz;
+    }
+    const int at = ((i + dv) * NV + j + dv) * NV + k + dv;
+    const R* c = v + at;
+    const R* fc = f + ((i + dv - 1) * NF + j + dv - 1) * NF + k + dv - 1;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      if (u == 1 && i + 1 >= E) break;
+      const R *b = c + u * NV * NV, *a = b - NV * NV, *n = b + NV * NV;
+      Hood<R> h = zero_hood<R>();
+      if (OP != kOpJacobiZero) {
+        h.c = b[0];
+        h.xp = n[0], h.xm = a[0], h.yp = b[NV], h.ym = b[-NV], h.zp = b[1], h.zm = b[-1];
+        h.xpyp = n[NV], h.xmym = a[-NV], h.xmyp = a[NV], h.xpym = n[-NV];
+        h.xpzp = n[1], h.xmzm = a[-1], h.xmzp = a[1], h.xpzm = n[-1];
+        h.ypzp = b[NV + 1], h.ymzm = b[-NV - 1], h.ymzp = b[1 - NV], h.ypzm = b[NV - 1];
+      }
+      R px = R(0), A = R(0);
+      if (LOCAL) {
+        px = static_cast<R>(wrap_once(x0 - lo + i + u, G.n[0])) + G.org[0];
+        A = G.h2[0] * px * px;
+      }
+      w[at + u * NV * NV] =
+          stencil_cell<R, OP, LOCAL, FAST>(T, h, fc[u * NF * NF], px, A, py, B, pz, C, pypz, omega, keep);
+    }
+  }
+  __syncthreads();
+}
+
+template <typename R, bool DOWN, bool LOCAL, bool FAST>
+__global__ __launch_bounds__(kLegThreads) void k_vcycle_leg(LegArgs<R> A) {
+  using L = LegTile<R, DOWN>;
+  constexpr int BT = kLegTile, NV = L::kV, NF = L::kF, NT = kLegThreads;
+  extern __shared__ double smem[];
+  R* v = reinterpret_cast<R*>(smem);
+  R* w = v + NV * NV * NV;
+  R* f = w + NV * NV * NV;
+  const LegJob<R>& J = A.job[blockIdx.y];
+  const TileCoef<R>& T = J.T;
+  const int n0 = T.G.n[0], n1 = T.G.n[1], n2 = T.G.n[2];
+  const int bz = blockIdx.x % A.tz, by = blockIdx.x / A.tz % A.ty, bx = blockIdx.x / A.tz / A.ty;
+  const int x0 = bx * BT, y0 = by * BT, z0 = bz * BT;
+  const int tid = threadIdx.x;
+  // stage the source, the iterate and the correction: all loads of a thread first, so that one trip to
+  // the cache that holds the previous launch's results serves them all
+  const auto cell = [&](int t, int n, int pad) {
+    const int k = t % n, j = t / n % n, i = min(t / (n * n), n - 1);
+    return (wrap_once(x0 - pad + i, n0) * n1 + wrap_once(y0 - pad + j, n1)) * n2 + wrap_once(z0 - pad + k, n2);
+  };
+  constexpr int LV = (NV * NV * NV + NT - 1) / NT, LF = (NF * NF * NF + NT - 1) / NT;
+  constexpr int NC = DOWN ? 1 : L::kC, LC = (NC * NC * NC + NT - 1) / NT;
+  const bool with_v = !DOWN || !A.zero_start;
+  R sf[LF], sv[LV], sc[LC];
+#pragma unroll
+  for (int q = 0; q < LF; q++) sf[q] = J.src[cell(tid + q * NT, NF, L::kPadLo - 1)];
+  if (with_v) {
+#pragma unroll
+    for (int q = 0; q < LV; q++) sv[q] = J.in[cell(tid + q * NT, NV, L::kPadLo)];
+  }
+  R* const uc = f + NF * NF * NF;
+  if constexpr (!DOWN) {
+    const int c0 = n0 / 2, c1 = n1 / 2, c2 = n2 / 2;
+#pragma unroll
+    for (int q = 0; q < LC; q++) {
+      const int t = tid + q * NT;
+      const int k = t % NC, j = t / NC % NC, i = min(t / (NC * NC), NC - 1);
+      sc[q] = J.coarse[(wrap_once(x0 / 2 - 3 + i, c0) * c1 + wrap_once(y0 / 2 - 3 + j, c1)) * c2 +
+                       wrap_once(z0 / 2 - 3 + k, c2)];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < LF; q++)
+    if (tid + q * NT < NF * NF * NF) f[tid + q * NT] = sf[q];
+  if (with_v) {
+#pragma unroll
+    for (int q = 0; q < LV; q++)
+      if (tid + q * NT < NV * NV * NV) v[tid + q * NT] = sv[q];
+  }
+  if constexpr (!DOWN) {
+#pragma unroll
+    for (int q = 0; q < LC; q++)
+      if (tid + q * NT < NC * NC * NC) uc[tid + q * NT] = sc[q];
+    __syncthreads();
+#pragma unroll 1
+    for (int t = tid; t < NV * NV * NV; t += NT) {
+      // prolong_value's sums; the tile starts on an even cell, kPadLo = 5 below it an odd one
+      const int k = t % NV + 1, j = t / NV % NV + 1, i = t / (NV * NV) + 1;
+      const R* u = uc + ((i >> 1) * NC + (j >> 1)) * NC + (k >> 1);
+      const bool X = i & 1, Y = j & 1, Z = k & 1;
+      R val = u[0];
+      val = X ? val + u[NC * NC] : val;
+      val = Y ? val + u[NC] : val;
+      val = Z ? val + u[1] : val;
+      val = X && Y ? val + u[NC * NC + NC] : val;
+      val = X && Z ? val + u[NC * NC + 1] : val;
+      val = Y && Z ? val + u[NC + 1] : val;
+      val = X && Y && Z ? val + u[NC * NC + NC + 1] : val;
+      // over 2, 4 or 8: the product with the power of two rounds the same
+      v[t] += val * ((X ? R(0.5) : R(1)) * (Y ? R(0.5) : R(1)) * (Z ? R(0.5) : R(1)));
+    }
+  }
+  __syncthreads();
+  int left = A.niter - 1;
+  if (DOWN && A.zero_start) {
+    leg_pass<R, DOWN, kOpJacobiZero, LOCAL, FAST>(T, v, f, w, L::kLo + left, L::kHi + left, x0, y0, z0, A.omega,
+                                                      A.keep);
+    R* s = v;
+    v = w;
+    w = s;
+    left--;
+  }
+#pragma unroll 1
+  for (; left >= 0; left--) {
+    leg_pass<R, DOWN, kOpJacobi, LOCAL, FAST>(T, v, f, w, L::kLo + left, L::kHi + left, x0, y0, z0, A.omega,
+                                                  A.keep);
+    R* s = v;
+    v = w;
+    w = s;
+  }
+  // the tile's own cells
+  for (int t = tid; t < BT * BT * BT; t += NT) {
+    const int k = t % BT, j = t / BT % BT, i = t / (BT * BT);
+    const int ix = x0 + i, iy = y0 + j, iz = z0 + k;
+    if (ix >= n0 || iy >= n1 || iz >= n2) continue;
+    const R val = v[((i + L::kPadLo) * NV + j + L::kPadLo) * NV + k + L::kPadLo];
+    const int at = (ix * n1 + iy) * n2 + iz;
+    if (!DOWN && T.acc)
+      T.acc[at] += static_cast<double>(val);
+    else
+      J.out[at] = val;
+  }
+  if constexpr (DOWN) {
+    leg_pass<R, DOWN, kOpResidual, LOCAL, FAST>(T, v, f, w, 1, 0, x0, y0, z0, A.omega, A.keep);
+    constexpr int H = BT / 2;
+    for (int t = tid; t < H * H * H; t += NT) {
+      const int k = t % H, j = t / H % H, i = t / (H * H);
+      const int jx = x0 / 2 + i, jy = y0 / 2 + j, jz = z0 / 2 + k;
+      if (2 * jx >= n0 || 2 * jy >= n1 || 2 * jz >= n2) continue;
+      const R* c = w + ((2 * i + L::kPadLo) * NV + 2 * j + L::kPadLo) * NV + 2 * k + L::kPadLo;
+      J.coarse[(jx * (n1 / 2) + jy) * (n2 / 2) + jz] =
+          restrict_sum<R>([&](int a, int b, int e) { return c[((a - 1) * NV + b - 1) * NV + e - 1]; });
+    }
   }
 }
 
@@ -1893,32 +2161,32 @@ static int launch_jacobi(const R* v, const R* f, R* out, const LevelGeom<R>& G, 
                          bool zero_in, hipStream_t s, int timer = -1, bool fast = false,
                          double* acc = nullptr, bool* fused = nullptr) {
   const size_t total = static_cast<size_t>(G.n[0]) * G.n[1] * G.n[2];
-  if (fused) *fused = false;
   // a sweep added into the FP64 iterate is another kernel (kOpJacobiAcc): not in the timer
-  const bool tiled = tiled_ok(G.n);
+  const bool tiled = tiled_ok(G.n), blocks = tiled && !short_tiles(G.n);
   const bool into_acc = acc && !zero_in && (!tiled || fast) && std::is_same<R, float>::value;
   if (into_acc) timer = -1;
   constexpr bool kFast = std::is_same<R, float>::value;
   timer_before(timer, s);
-  if (into_acc) {
-    if (tiled)
-      launch_tiled<R, R, kOpJacobiAcc, kFast>(v, f, out, G, omega, keep, s, acc);
+  // launch_tiled or launch_uneven, with the fast arithmetic or the exact one
+  const auto sweep = [&](auto op) {
+    constexpr int OP = decltype(op)::value;
+    double* into = OP == kOpJacobiAcc ? acc : nullptr;
+    if (blocks && fast)
+      launch_tiled<R, R, OP, kFast>(v, f, out, G, omega, keep, s, into);
+    else if (blocks)
+      launch_tiled<R, R, OP, false>(v, f, out, G, omega, keep, s, into);
+    else if (tiled && fast)
+      launch_uneven<R, R, OP, kFast>(v, f, out, G, omega, keep, s, into);
     else
-      launch_uneven<R, R, kOpJacobiAcc>(v, f, out, G, omega, keep, s, acc);
-    if (fused) *fused = true;
-  } else if (!tiled && zero_in) {
-    launch_uneven<R, R, kOpJacobiZero>(v, f, out, G, omega, keep, s);
-  } else if (!tiled) {
-    launch_uneven<R, R, kOpJacobi>(v, f, out, G, omega, keep, s);
-  } else if (zero_in && fast) {
-    launch_tiled<R, R, kOpJacobiZero, kFast>(v, f, out, G, omega, keep, s);
-  } else if (zero_in) {
-    launch_tiled<R, R, kOpJacobiZero, false>(v, f, out, G, omega, keep, s);
-  } else if (fast) {
-    launch_tiled<R, R, kOpJacobi, kFast>(v, f, out, G, omega, keep, s);
-  } else {
-    launch_tiled<R, R, kOpJacobi, false>(v, f, out, G, omega, keep, s);
-  }
+      launch_uneven<R, R, OP>(v, f, out, G, omega, keep, s, into);
+  };
+  if (into_acc)
+    sweep(std::integral_constant<int, kOpJacobiAcc>());
+  else if (zero_in)
+    sweep(std::integral_constant<int, kOpJacobiZero>());
+  else
+    sweep(std::integral_constant<int, kOpJacobi>());
+  if (fused) *fused = into_acc;
   // algorithmic traffic: read v (unless zero) and f, write the new iterate
   timer_after(timer, s, static_cast<double>(total) * sizeof(R) * (zero_in ? 2 : 3));
   PRH_LAUNCHED();
@@ -1928,14 +2196,16 @@ static int launch_jacobi(const R* v, const R* f, R* out, const LevelGeom<R>& G, 
 template <typename R, typename O>
 static int launch_residual(const R* v, const R* f, O* r, const LevelGeom<R>& G, hipStream_t s,
                            bool fast = false, Centre C = {}) {
-  if (tiled_ok(G.n) && fast) {
-    launch_tiled<R, O, kOpResidual, std::is_same<R, float>::value && std::is_same<O, float>::value>(
-        v, f, r, G, R(0), R(0), s, nullptr, C);
-  } else if (tiled_ok(G.n)) {
+  const bool tiled = tiled_ok(G.n), blocks = tiled && !short_tiles(G.n);
+  constexpr bool kFast = std::is_same<R, float>::value && std::is_same<O, float>::value;
+  if (blocks && fast)
+    launch_tiled<R, O, kOpResidual, kFast>(v, f, r, G, R(0), R(0), s, nullptr, C);
+  else if (blocks)
     launch_tiled<R, O, kOpResidual, false>(v, f, r, G, R(0), R(0), s, nullptr, C);
-  } else {
+  else if (tiled && fast)
+    launch_uneven<R, O, kOpResidual, kFast>(v, f, r, G, R(0), R(0), s, nullptr, C);
+  else
     launch_uneven<R, O, kOpResidual>(v, f, r, G, R(0), R(0), s, nullptr, C);
-  }
   PRH_LAUNCHED();
   return PRH_OK;
 }
@@ -2265,7 +2535,7 @@ struct Solver {
   // first level handled by the single-workgroup coarse kernel
   int coarse_level() const {
     for (int l = 0; l < nlev(); l++)
-      if (size(l) <= kCoarseCells && nlev() - l <= kMaxCoarse) return l;
+      if (size(l) <= (leg_ok(l) ? kCoarseOne : kCoarseCells) && nlev() - l <= kMaxCoarse) return l;
     return nlev();
   }
 
@@ -2302,9 +2572,82 @@ struct Solver {
     return PRH_OK;
   }
 
+  // whether the leg kernels take level l
+  bool leg_ok(int l) const {
+    if (niter < 1 || niter > kLegSweeps || l + 1 >= nlev()) return false;
+    size_t least = n(l)[0];
+    for (int d = 1; d < 3; d++) least = n(l)[d] < least ? n(l)[d] : least;
+    // halo cells wrap once around the level
+    return least >= 12 && size(l) <= kLegCells;
+  }
+
+  // one leg of the V-cycle on level l: the iterate goes from `in` to `out`
+  template <bool DOWN, bool FAST>
+  int leg(int l, const Ptrs<R>& in, const Ptrs<R>& src, const Ptrs<R>& out, const Ptrs<R>& coarse, bool zero_start) {
+    using L = LegTile<R, DOWN>;
+    constexpr int BT = kLegTile;
+    LegArgs<R> A;
+    A.niter = niter;
+    A.zero_start = zero_start ? 1 : 0;
+    A.omega = omega;
+    A.keep = keep;
+    const size_t* m = n(l);
+    A.tx = static_cast<int>(ceil_div(m[0], BT));
+    A.ty = static_cast<int>(ceil_div(m[1], BT));
+    A.tz = static_cast<int>(ceil_div(m[2], BT));
+    const bool local = G[0][l].local;
+    bool same = true;
+    for (int j = 0; j < count; j++) same = same && (G[j][l].local != 0) == local;
+    for (int j0 = 0; j0 < count; j0 += same ? count : 1) {
+      const int nj = same ? count : 1;
+      for (int q = 0; q < nj; q++) {
+        const int j = j0 + q;
+        LegJob<R>& J = A.job[q];
+        J.T = TileCoef<R>();
+        J.T.G = G[j][l];
+        J.T.K = G[j][l].local ? GlobalCoef<R>() : GlobalCoef<R>::make(G[j][l]);
+        J.T.dinv = G[j][l].local ? R(0) : R(1) / J.T.K.d;
+        J.T.acc = !DOWN && l == 0 && fuse_top ? acc_top[j] : nullptr;
+        if (!DOWN && l == 0 && fuse_top) fused[j] = true;
+        J.in = in[j];
+        J.src = src[j];
+        J.out = out[j];
+        J.coarse = coarse[j];
+      }
+      const dim3 grid(A.tx * A.ty * A.tz, nj);
+      const bool loc = G[j0][l].local;
+      auto* k = loc ? &k_vcycle_leg<R, DOWN, true, FAST> : &k_vcycle_leg<R, DOWN, false, FAST>;
+      if (L::lds > 65536)
+        PRH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    static_cast<int>(L::lds)));
+      k<<<grid, kLegThreads, L::lds, s>>>(A);
+      PRH_LAUNCHED();
+    }
+    return PRH_OK;
+  }
+  template <bool DOWN>
+  int leg(int l, const Ptrs<R>& in, const Ptrs<R>& src, const Ptrs<R>& out, const Ptrs<R>& coarse, bool zero_start) {
+    // the fast FP32 forms where the sweeps of this level would take them
+    const int nn[3] = {static_cast<int>(n(l)[0]), static_cast<int>(n(l)[1]), static_cast<int>(n(l)[2])};
+    if constexpr (std::is_same<R, float>::value)
+      if (fast && tiled_ok(nn)) return leg<DOWN, true>(l, in, src, out, coarse, zero_start);
+    return leg<DOWN, false>(l, in, src, out, coarse, zero_start);
+  }
+
   // src/multigrid.c:270-300
   int vcycle(int l, Ptrs<R>& cur, Ptrs<R>& alt, const Ptrs<R>& src, bool zero_start) {
     if (l >= coarse_level()) return vcycle_coarse(l, cur, alt, src, zero_start);
+    if (leg_ok(l)) {
+      const Ptrs<R> fc = f(l + 1);
+      PRH_TRY(leg<true>(l, cur, src, alt, fc, zero_start));
+      swap_all(cur, alt, count);
+      Ptrs<R> cc = v(l + 1);
+      Ptrs<R> ca = tmp(l + 1);
+      PRH_TRY(vcycle(l + 1, cc, ca, fc, true));
+      PRH_TRY(leg<false>(l, cur, src, alt, cc, false));
+      swap_all(cur, alt, count);
+      return PRH_OK;
+    }
     PRH_TRY(smooth(l, cur, alt, src, zero_start));
     if (l + 1 < nlev()) {
       PRH_TRY(residual(l, cur, src, alt));
