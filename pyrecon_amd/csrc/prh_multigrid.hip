@@ -74,7 +74,16 @@ __device__ __forceinline__ R centre_mean(const Centre& C) {
 // (FP32 rows of 512 cells): the first sweep of a zero iterate is pointwise in
 // the source, so the second stages the first's value of each cell, computed
 // from the source as the zero-start sweep computes it, instead of reading it
-enum StencilOp { kOpJacobi = 0, kOpResidual = 1, kOpJacobiZero = 2, kOpJacobiAcc = 3, kOpJacobiAfterZero = 4 };
+// kOpJacobiCorrect: a sweep of the iterate plus the coarser level's correction
+// (src/multigrid.c:293-298), which is added to each value as it is staged from
+// coarse planes in LDS: the corrected iterate is neither stored nor read back,
+// 16 (FP64) or 8 bytes a cell of 41 and 20.5.  The sweep and the pass are bound by
+// memory; with the corrections, 7 LDS reads more a staged cell, a sweep of 512^3
+// takes 0.91 ms in FP64 tiles (0.68 without) and 0.53 ms in FP32 rows (0.30, and
+// 0.25 for the pass that it replaces)
+enum StencilOp {
+  kOpJacobi = 0, kOpResidual = 1, kOpJacobiZero = 2, kOpJacobiAcc = 3, kOpJacobiAfterZero = 4, kOpJacobiCorrect = 5
+};
 constexpr int kTileZ = 64;
 
 // Coefficients of a level passed to the blocked kernels: the geometry for a
@@ -90,6 +99,8 @@ struct TileCoef {
   double* acc = nullptr;
   // kOpResidual: the source's mean to remove (the mixed path's centred source)
   Centre C;
+  // kOpJacobiCorrect: the coarser level's correction (n0 / 2, n1 / 2, n2 / 2)
+  const R* coarse = nullptr;
   // FLEX tiles: tz x ty cells (at most kFlexCells), and their numbers along z and y
   int tz = 0, ty = 0, ztiles = 0, ytiles = 0;
 };
@@ -162,6 +173,33 @@ constexpr int tiled_min_waves() {
   return std::is_same<R, double>::value && std::is_same<O, float>::value ? 4 : PRH_TILED_MIN_WAVES;
 }
 
+// The trilinear prolongation (prolong_value: the same operands and order; the product with 1/2, 1/4 or 1/8
+// rounds as the quotient) of two coarse planes staged in LDS: p holds coarse plane x / 2 and q the next, the
+// cell's coarse value is at p[at], the next ones along y and z at p[at + dy] and p[atz].  X, Y, Z: whether
+// the cell is odd along each axis.  All values are read and the ones not used dropped (branches on the
+// parity of rows that a wavefront has to itself: 32.4 ms for a global FP32 solve of 512^3 against 31.9).
+template <typename R>
+__device__ __forceinline__ R ring_value(const R* p, const R* q, int at, int atz, int dy, bool X, bool Y, bool Z) {
+  const R a = p[at], ay = p[at + dy], az = p[atz], ayz = p[atz + dy];
+  R sum = a, scale = (Y ? R(0.5) : R(1)) * (Z ? R(0.5) : R(1));
+  if (X) {
+    const R ax = q[at], axy = q[at + dy], axz = q[atz], axyz = q[atz + dy];
+    scale *= R(0.5);
+    sum += ax;
+    sum = Y ? sum + ay : sum;
+    sum = Z ? sum + az : sum;
+    sum = Y ? sum + axy : sum;
+    sum = Z ? sum + axz : sum;
+    sum = Y && Z ? sum + ayz : sum;
+    sum = Y && Z ? sum + axyz : sum;
+  } else {
+    sum = Y ? sum + ay : sum;
+    sum = Z ? sum + az : sum;
+    sum = Y && Z ? sum + ayz : sum;
+  }
+  return sum * scale;
+}
+
 // FLEX: tiles of any extent, for levels whose rows are no multiple of 64 cells or
 // whose planes are no multiple of 8 rows: the level's (y, z) plane is cut evenly
 // into tiles of at most kFlexCells cells, the tile's cells are dealt to the
@@ -177,6 +215,14 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
   const int W = FLEX ? T.tz + 2 : kTileZ + 2;
   const int staged_cells = FLEX ? W * (T.ty + 2) : PLANE;
   __shared__ R lds[4 * PLANE];
+  // kOpJacobiCorrect: the correction's cells below the tile and its halo, a ring of 4 coarse planes (two
+  // of them in use); runs start on even planes
+  constexpr bool CORR = OP == kOpJacobiCorrect;
+  constexpr int OPC = CORR ? kOpJacobi : OP;
+  static_assert(!CORR || !FLEX, "correction: the 64-wide tiles");
+  constexpr int CW = kTileZ / 2 + 2, CH = TY / 2 + 2, CPLANE = CORR ? CW * CH : 1;
+  static_assert(CPLANE <= 256, "one coarse value a thread");
+  __shared__ R ring[4 * CPLANE + CW + 2];  // the last cells' neighbours are read and not used
   const LevelGeom<R>& G = T.G;
   const R fmean = OP == kOpResidual ? centre_mean<R>(T.C) : R(0);
   const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
@@ -214,13 +260,40 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
   auto wrapx = [n0](int x) { return x < 0 ? x + n0 : (x >= n0 ? x - n0 : x); };
   // ring slot of plane x, relative to the run start (static inside the unrolled loop)
   auto slot = [xb](int x) { return (x - xb + 4) & 3; };
+  // the coarse value of this thread, in coarse plane J (periodic)
+  int coff = 0;
+  if constexpr (CORR) {
+    const int jy = y0 / 2 - 1 + tid / CW, jz = z0 / 2 - 1 + tid % CW, c1 = n1 / 2, c2 = n2 / 2;
+    coff = (jy < 0 ? jy + c1 : jy >= c1 ? jy - c1 : jy) * c2 + (jz < 0 ? jz + c2 : jz >= c2 ? jz - c2 : jz);
+  }
+  auto coarse_at = [&](int J) {
+    const int c0 = n0 / 2, j = J < 0 ? J + c0 : J >= c0 ? J - c0 : J;
+    return T.coarse[static_cast<size_t>(j) * (s0 / 4) + coff];
+  };
+  // the value staged for cell e of plane xp, with the correction there added (the halo starts on an odd row
+  // and column)
+  auto staged = [&](R val, int xp, int e) -> R {
+    if constexpr (!CORR) {
+      return val;
+    } else {
+      const int row = e / (kTileZ + 2), col = e - row * (kTileZ + 2);
+      const int at = ((row + 1) >> 1) * CW + ((col + 1) >> 1);
+      return val + ring_value<R>(ring + ((xp >> 1) & 3) * CPLANE, ring + (((xp >> 1) + 1) & 3) * CPLANE, at, at + 1, CW,
+                                 xp & 1, !(row & 1), !(col & 1));
+    }
+  };
+  if constexpr (CORR) {
+    if (tid < CPLANE)
+      for (int J = xb / 2 - 1; J <= xb / 2 + 1; J++) ring[(J & 3) * CPLANE + tid] = coarse_at(J);
+    __syncthreads();
+  }
   if (OP != kOpJacobiZero)
   for (int p = -1; p <= 1; p++) {
     const R* src = v + static_cast<size_t>(wrapx(xb + p)) * s0;
     R* dst = lds + slot(xb + p) * PLANE;
 #pragma unroll
     for (int q = 0; q < PER; q++)
-      if (has[q]) dst[tid + 256 * q] = src[off[q]];
+      if (has[q]) dst[tid + 256 * q] = staged(src[off[q]], xb + p, tid + 256 * q);
   }
   // per-thread constants: rows iy_k = y0 + ty + 4k, column iz; FLEX: cells tid and
   // tid + 256 of the tile
@@ -266,11 +339,11 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
     for (int q = 0; q < PER; q++)
       if (has[q]) dst[q] = src[off[q]];
   };
-  auto stash = [&](const R(&src)[PER], int sl) {
+  auto stash = [&](const R(&src)[PER], int sl, int xp) {
     R* dst = lds + sl * PLANE;
 #pragma unroll
     for (int q = 0; q < PER; q++)
-      if (has[q]) dst[tid + 256 * q] = src[q];
+      if (has[q]) dst[tid + 256 * q] = staged(src[q], xp, tid + 256 * q);
   };
   // the source values of plane x, loaded one plane ahead (see k_stencil_rows)
   auto load_f = [&](R(&dst)[KY], int x) {
@@ -312,7 +385,7 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
       h.ypzm = P[o + W - 1];
       }
       const R fv = (OP == kOpResidual && T.C.sum) ? fvs[k] - fmean : fvs[k];
-      const R res = stencil_cell<R, OP, LOCAL, FAST>(T, h, fv, px, A, py[k], B[k], pz[FLEX ? k : 0],
+      const R res = stencil_cell<R, OPC, LOCAL, FAST>(T, h, fv, px, A, py[k], B[k], pz[FLEX ? k : 0],
                                                      C[FLEX ? k : 0], pypz[k],
                                                      omega, keep);
       if constexpr (OP == kOpJacobiAcc)
@@ -338,6 +411,7 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
     }
     if (xb + 1 < xe) fetch(preA, xb + 2);
     __syncthreads();
+    R cnext = R(0);
     for (int x0 = xb; x0 < xe; x0 += 4) {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
@@ -349,14 +423,18 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
             else
               fetch(preA, x + 3);
           }
+          // staging plane x + 2 (even) ends the use of coarse plane x / 2 and the next step's odd plane
+          // needs the one after next
+          if (CORR && !(u & 1) && tid < CPLANE) cnext = coarse_at(x / 2 + 2);
           load_f(fA, x);
           compute(x, fA, lds + ((u + 3) & 3) * PLANE, lds + (u & 3) * PLANE, lds + ((u + 1) & 3) * PLANE);
           if (x + 1 < xe) {
             if ((u + 2) & 1)
-              stash(preB, (u + 2) & 3);
+              stash(preB, (u + 2) & 3, x + 2);
             else
-              stash(preA, (u + 2) & 3);
+              stash(preA, (u + 2) & 3, x + 2);
           }
+          if (CORR && !(u & 1) && tid < CPLANE) ring[((x / 2 + 2) & 3) * CPLANE + tid] = cnext;
           __syncthreads();
         }
       }
@@ -377,6 +455,7 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
   fetch(preA, min(xb + 2, xe));
   load_f(fA, xb);
   __syncthreads();
+  R cnext = R(0);
   for (int x0 = xb; x0 < xe; x0 += 4) {
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -389,16 +468,18 @@ __global__ __launch_bounds__(256, (tiled_min_waves<R, O>())) void k_stencil_tile
         load_f(fB, min(x + 1, xe - 1));
       else
         load_f(fA, min(x + 1, xe - 1));
+      if (CORR && !(u & 1) && tid < CPLANE) cnext = coarse_at(min(x, xe) / 2 + 2);
       __builtin_amdgcn_sched_barrier(0);
       if (x < xe) {
         compute(x, (u & 1) ? fB : fA, lds + ((u + 3) & 3) * PLANE, lds + (u & 3) * PLANE,
                 lds + ((u + 1) & 3) * PLANE);
         if (x + 1 < xe) {
           if ((u + 2) & 1)
-            stash(preB, (u + 2) & 3);
+            stash(preB, (u + 2) & 3, x + 2);
           else
-            stash(preA, (u + 2) & 3);
+            stash(preA, (u + 2) & 3, x + 2);
         }
+        if (CORR && !(u & 1) && tid < CPLANE) ring[((x / 2 + 2) & 3) * CPLANE + tid] = cnext;
         __syncthreads();
       }
     }
@@ -438,9 +519,13 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
   // kOpJacobiAfterZero: v is the source, and the staged value of each cell is
   // the zero-start sweep's; the computation is then a plain sweep
   constexpr bool AZ = OP == kOpJacobiAfterZero;
-  constexpr int OPC = AZ ? kOpJacobi : OP;
+  // kOpJacobiCorrect: the correction's rows below the tile and its halo, as in k_stencil_tiled
+  constexpr bool CORR = OP == kOpJacobiCorrect;
+  constexpr int CW = N2 / 2, CPLANE = CORR ? (RY / 2 + 2) * CW : 1, CPER = (CPLANE + NT - 1) / NT;
+  constexpr int OPC = AZ || CORR ? kOpJacobi : OP;
   static_assert(!AZ || FAST, "two sweeps from zero: the FP32 fast sweeps");
   __shared__ R lds[4 * PLANE];
+  __shared__ R ring[4 * CPLANE + CW];  // the last row's neighbours are read and not used
   const LevelGeom<R>& G = T.G;
   const int n0 = G.n[0], n1 = G.n[1];
   const int tid = threadIdx.x, lane = tid & 63, ty = (tid >> 6) / WPR;
@@ -468,9 +553,30 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
   }
   auto wrapx = [n0](int x) { return x < 0 ? x + n0 : (x >= n0 ? x - n0 : x); };
   auto slot = [xb](int x) { return (x - xb + 4) & 3; };
-  // the value staged for element q of plane xp (a plane index in [0, n0))
+  // the coarse values of this thread, in coarse plane J (periodic)
+  auto coarse_at = [&](R(&dst)[CPER], int J) {
+    const int c0 = n0 / 2, c1 = n1 / 2, j = J < 0 ? J + c0 : J >= c0 ? J - c0 : J;
+#pragma unroll
+    for (int q = 0; q < CPER; q++) {
+      const int e = tid + NT * q, jy = y0 / 2 - 1 + e / CW;
+      if (CPLANE % NT != 0 && e >= CPLANE) break;
+      dst[q] = T.coarse[(static_cast<size_t>(j) * c1 + (jy < 0 ? jy + c1 : jy >= c1 ? jy - c1 : jy)) * CW + e % CW];
+    }
+  };
+  auto coarse_to = [&](const R(&src)[CPER], int J) {
+#pragma unroll
+    for (int q = 0; q < CPER; q++)
+      if (CPLANE % NT == 0 || tid + NT * q < CPLANE) ring[(J & 3) * CPLANE + tid + NT * q] = src[q];
+  };
+  // the value staged for element q of plane xp (a plane index in [0, n0); with a correction, its number in
+  // the run)
   auto staged = [&](R val, int xp, int q) -> R {
-    if constexpr (!AZ) {
+    if constexpr (CORR) {
+      const int e = tid + NT * q, row = e / N2, col = e % N2, jz = col >> 1;
+      const int at = ((row + 1) >> 1) * CW;
+      return val + ring_value<R>(ring + ((xp >> 1) & 3) * CPLANE, ring + (((xp >> 1) + 1) & 3) * CPLANE, at + jz,
+                                 at + (jz + 1 == CW ? 0 : jz + 1), CW, xp & 1, !(row & 1), col & 1);
+    } else if constexpr (!AZ) {
       return val;
     } else {
       // the zero-start sweep at (xp, gy, gz), with the coefficients that
@@ -496,6 +602,14 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
                                                          pypz, omega, keep);
     }
   };
+  R cnext[CPER];
+  if constexpr (CORR) {
+    for (int J = xb / 2 - 1; J <= xb / 2 + 1; J++) {
+      coarse_at(cnext, J);
+      coarse_to(cnext, J);
+    }
+    __syncthreads();
+  }
   if (OP != kOpJacobiZero)
     for (int p = -1; p <= 1; p++) {
       const int xp = wrapx(xb + p);
@@ -503,7 +617,7 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
       R* dst = lds + slot(xb + p) * PLANE;
 #pragma unroll
       for (int q = 0; q < PER; q++)
-        if (has[q]) dst[tid + NT * q] = staged(src[off[q]], xp, q);
+        if (has[q]) dst[tid + NT * q] = staged(src[off[q]], CORR ? xb + p : xp, q);
     }
   // per-thread constants: row iy = y0 + ty, columns iz = zb + 64 WPR c
   const int iy = y0 + ty;
@@ -537,7 +651,7 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
     R* dst = lds + sl * PLANE;
 #pragma unroll
     for (int q = 0; q < PER; q++)
-      if (has[q]) dst[tid + NT * q] = src[q];
+      if (has[q]) dst[tid + NT * q] = CORR ? staged(src[q], xp, q) : src[q];
     if constexpr (AZ) {
       // the thread's own elements, in place, once the loaded values are out of
       // registers (kept apart from the sweep's own code, which holds the rest)
@@ -647,14 +761,16 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
             else
               fetch(preA, x + 3);
           }
+          if (CORR && !(u & 1)) coarse_at(cnext, x / 2 + 2);
           load_f(fA, x);
           compute(x, fA, lds + ((u + 3) & 3) * PLANE, lds + (u & 3) * PLANE, lds + ((u + 1) & 3) * PLANE);
           if (x + 1 < xe) {
             if ((u + 2) & 1)
-              stash(preB, (u + 2) & 3, wrapx(x + 2));
+              stash(preB, (u + 2) & 3, CORR ? x + 2 : wrapx(x + 2));
             else
-              stash(preA, (u + 2) & 3, wrapx(x + 2));
+              stash(preA, (u + 2) & 3, CORR ? x + 2 : wrapx(x + 2));
           }
+          if (CORR && !(u & 1)) coarse_to(cnext, x / 2 + 2);
           __syncthreads();
         }
       }
@@ -676,6 +792,7 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
         load_f(fB, min(x + 1, xe - 1));
       else
         load_f(fA, min(x + 1, xe - 1));
+      if (CORR && !(u & 1)) coarse_at(cnext, min(x, xe) / 2 + 2);
       // keep the loads ahead of the computation (the scheduler would otherwise
       // sink them below the waits for this plane's sources)
       __builtin_amdgcn_sched_barrier(0);
@@ -684,10 +801,11 @@ __global__ __launch_bounds__(64 * RY * WPR, PRH_ROWS_MIN_WAVES) void k_stencil_r
                 lds + ((u + 1) & 3) * PLANE);
         if (x + 1 < xe) {
           if ((u + 2) & 1)
-            stash(preB, (u + 2) & 3, wrapx(x + 2));
+            stash(preB, (u + 2) & 3, CORR ? x + 2 : wrapx(x + 2));
           else
-            stash(preA, (u + 2) & 3, wrapx(x + 2));
+            stash(preA, (u + 2) & 3, CORR ? x + 2 : wrapx(x + 2));
         }
+        if (CORR && !(u & 1)) coarse_to(cnext, x / 2 + 2);
         __syncthreads();
       }
     }
@@ -971,7 +1089,8 @@ inline int tiled_xlen(const int* n) {
 template <typename R, typename O, int OP, bool FAST, int WPR, int CZ, int RY = kRowsY>
 static void launch_rows_cz(const R* v, const R* f, O* out, const TileCoef<R>& T, R omega, R keep,
                            hipStream_t s) {
-  const int xlen = rows_xlen(T.G.n);
+  int xlen = rows_xlen(T.G.n);
+  if (OP == kOpJacobiCorrect) xlen += xlen & 1;
   const unsigned grid =
       static_cast<unsigned>((T.G.n[1] / RY) * ((T.G.n[0] + xlen - 1) / xlen));
   constexpr int nt = 64 * RY * WPR;
@@ -1007,7 +1126,10 @@ static bool launch_rows(const R* v, const R* f, O* out, const TileCoef<R>& T, R 
       // 512-cell rows: two wavefronts per row keep the registers per lane near those of 256
       case 8: launch_rows_cz<R, O, OP, FAST, 2, 4>(v, f, out, T, omega, keep, s); return true;
       // 1024-cell rows: four wavefronts per row, 4 rows per block
-      case 16: launch_rows_cz<R, O, OP, FAST, 4, 4, kRowsY1024>(v, f, out, T, omega, keep, s); return true;
+      case 16:
+        if constexpr (OP != kOpJacobiCorrect)
+          launch_rows_cz<R, O, OP, FAST, 4, 4, kRowsY1024>(v, f, out, T, omega, keep, s);
+        return true;
       default: return false;
     }
   }
@@ -1016,8 +1138,9 @@ static bool launch_rows(const R* v, const R* f, O* out, const TileCoef<R>& T, R 
 
 template <typename R, typename O, int OP, bool FAST>
 static void launch_tiled(const R* v, const R* f, O* out, const LevelGeom<R>& G, R omega, R keep,
-                         hipStream_t s, double* acc = nullptr, Centre C = {}) {
-  const int xlen = tiled_xlen(G.n);
+                         hipStream_t s, double* acc = nullptr, Centre C = {}, const R* correction = nullptr) {
+  int xlen = tiled_xlen(G.n);
+  if (OP == kOpJacobiCorrect) xlen += xlen & 1;
   const unsigned grid = static_cast<unsigned>((G.n[2] / kTileZ) * (G.n[1] / kTileY) *
                                               ((G.n[0] + xlen - 1) / xlen));
   TileCoef<R> T;
@@ -1026,6 +1149,7 @@ static void launch_tiled(const R* v, const R* f, O* out, const LevelGeom<R>& G, 
   T.dinv = G.local ? R(0) : R(1) / T.K.d;
   T.acc = acc;
   T.C = C;
+  T.coarse = correction;
   if constexpr (OP == kOpJacobiAfterZero) {
     // only where after_zero_ok() holds: FP32 fast rows of 512 cells
     launch_rows<R, O, OP, FAST>(v, f, out, T, omega, keep, s);
@@ -2502,16 +2626,51 @@ struct Solver {
     return PRH_ERR_STATE;
   }
 
+  // the correction of a coarser level in the first sweep that follows it (kOpJacobiCorrect): levels in
+  // 64-wide tiles or whole rows, a solve of 512^3 in 67.8 ms against 69.1 (FP64), 38.5 against 39.1 (mixed,
+  // local line of sight) and 35.0 against 36.4 (mixed, global), of 384 x 320 x 448 in 33.7 against 34.4 and
+  // 20.7 against 21.0.  FP32 rows of 1024 cells would spill (256 x 256 x 1024 mixed: 25.8 ms against 23.6),
+  // and so the correction stays a pass of its own there, as it does where its sweep is also the last one,
+  // which may have to be added into the FP64 iterate.
+  bool corrects(int l) const {
+    if (grouped(l) || niter < 2) return false;
+    const int nn[3] = {static_cast<int>(n(l)[0]), static_cast<int>(n(l)[1]), static_cast<int>(n(l)[2])};
+    return tiled_ok(nn) && !short_tiles(nn) && !(std::is_same<R, float>::value && rows_cz(nn) == 16);
+  }
+  int jacobi_correct(int l, const Ptrs<R>& in, const Ptrs<R>& coarse, const Ptrs<R>& src, const Ptrs<R>& out) {
+    for (int j = 0; j < count; j++) {
+      if (fast)
+        launch_tiled<R, R, kOpJacobiCorrect, std::is_same<R, float>::value>(in[j], src[j], out[j], G[j][l], omega, keep, s,
+                                                                            nullptr, {}, coarse[j]);
+      else
+        launch_tiled<R, R, kOpJacobiCorrect, false>(in[j], src[j], out[j], G[j][l], omega, keep, s, nullptr, {}, coarse[j]);
+      PRH_LAUNCHED();
+    }
+    return PRH_OK;
+  }
+
   // niter damped-Jacobi sweeps; the iterate moves between cur and alt.  Where
   // the level allows, the sweeps go in fused pairs (the last one alone when
   // niter is odd), and a zero start's first two sweeps go in one launch.
-  int smooth(int l, Ptrs<R>& cur, Ptrs<R>& alt, const Ptrs<R>& src, bool zero_start, bool post = false) {
+  // correction: the coarser level's, added to the iterate before the first sweep.
+  int smooth(int l, Ptrs<R>& cur, Ptrs<R>& alt, const Ptrs<R>& src, bool zero_start, bool post = false,
+             const Ptrs<R>* correction = nullptr) {
+    if (correction && !corrects(l)) {
+      PRH_TRY(prolong_to(l, *correction, cur, true));
+      correction = nullptr;
+    }
     if (niter <= 0) {
       if (zero_start) PRH_TRY(fill_zero(l, cur));
       return PRH_OK;
     }
     const bool last_fused = post && fuse_top && l == 0;
     for (int it = 0; it < niter;) {
+      if (correction && it == 0) {
+        PRH_TRY(jacobi_correct(l, cur, *correction, src, alt));
+        swap_all(cur, alt, count);
+        it++;
+        continue;
+      }
       if (zero_start && it == 0 && niter >= 2 && !(pairable(l)) && !(last_fused && niter == 2) &&
           after_zero_ok(l)) {
         // two sweeps: the iterate ends in cur, as after two single sweeps (two swaps)
@@ -2656,7 +2815,7 @@ struct Solver {
       Ptrs<R> cc = v(l + 1);
       Ptrs<R> ca = tmp(l + 1);
       PRH_TRY(vcycle(l + 1, cc, ca, fc, true));
-      PRH_TRY(prolong_to(l, cc, cur, true));
+      return smooth(l, cur, alt, src, false, true, &cc);
     }
     return smooth(l, cur, alt, src, false, true);
   }
