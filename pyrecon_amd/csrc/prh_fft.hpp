@@ -357,7 +357,7 @@ struct LineRows {
 };
 // Pairs of rows: as many as 256 threads take.  Blocks of a multiple of four wavefronts share the
 // four SIMDs evenly; five pairs of 384 elements on five wavefronts left half of the slots empty
-// (2.2 against 1.35 ms for the six fields of 384^3).
+// (2.2 against 1.35 ms for six fields of 384^3).
 template <typename R>
 LineRows line_rows(const LinePlan& P) {
   int nl = 256 * LineTile<R>::held / P.n;

@@ -13,15 +13,16 @@
 //     power of a Nyquist component appears only together with another one.
 //   * k_a k_b / k^2 splits into 1 / k^2 and a product of powers of kx, ky and kz.  The x pass
 //     transforms forward, divides by k^2 and goes back with kx^0, kx^1, kx^2 without leaving the
-//     workgroup (1 mesh read, 3 written); the y pass makes six fields of the three; the z pass
-//     transforms all six and adds x_a x_b / |x|^2 times each to the density in registers.
-//   * The six fields between the y and z passes exist for a slab of x planes at a time (kSlabBytes).
+//     workgroup (1 mesh read, 3 written).  x and y are constant along z: the y pass transforms the
+//     six products, times x_a x_b, and adds those of one power of z, three fields written where the
+//     three read were; the z pass transforms those and adds them times 1, z, z^2 in registers.
 // Bound: HBM, with the LDS exchanges and the FP64 butterflies close behind.  One iteration with a
-// local line of sight moves 25 meshes (z and y forward 2 + 2, x pass 1 + 3, y 3 + 6, z 6 + 2); one c2c
-// transform per term with separate operators moved 120.  At 384^3 in FP64 the three iterations and
-// the displacements take 12.9 ms; they took 63.3 ms that way.  Passes there: z and y forward 0.16 and
-// 0.18 ms (5.5 and 5.1 TB/s), x 0.65 ms (2.8 TB/s, four transforms), y 1.19 ms (3.4 TB/s, six), z with
-// the sums 1.4 ms (2.5 TB/s, six).
+// local line of sight moves 19 meshes (z and y forward 2 + 2, x pass 1 + 3, y 3 + 3, z 3 + 2); six
+// fields between y and z (in slabs, for their size) made it 25, one c2c transform per term with separate
+// operators 120.  At 384^3 in FP64 the three iterations and the displacements take 10.8 ms, 12.9 with six
+// fields, 63.3 that way; 512^3 23.6 and 27.9.  Passes at 384^3: z and y forward 0.16 and 0.18 ms (5.5 and
+// 5.1 TB/s), x 0.67 ms (2.7 TB/s, four transforms), y 1.34 ms (six transforms: 0.22 ms each, the FP64
+// arithmetic and LDS of one with two workgroups a CU), z with the sums 0.67 ms (3.4 TB/s; 1.5 for six).
 #include <cmath>
 
 #include "prh_fft.hpp"
@@ -73,11 +74,7 @@ bool line_plan(size_t n, LinePlan& P) {
 
 namespace {
 
-constexpr int kTerms = 6;  // pairs of axes (a <= b): xx xy xz yy yz zz
-// Bytes of the six fields of a slab.  Larger slabs fill the last round of workgroups of a launch
-// better (384^3: 17.1 ms a run with 96 MB, which the last-level cache would hold, 12.9 with 1 GB, 12.6
-// without slabs); smaller ones bound the scratch of large meshes.
-constexpr size_t kSlabBytes = size_t(1) << 30;
+constexpr int kPowers = 3;  // a local line of sight: fields of z^0, z^1 and z^2
 
 // Shape, wavenumbers and line of sight of a call.
 struct SpecShape {
@@ -158,14 +155,13 @@ enum RowsOut { kRowsStore = 0, kRowsMinus = 1, kRowsMinusLocal = 2 };
 // that are their own conjugates are dropped).
 //   kRowsStore: field blockIdx.y of `fields` to out[blockIdx.y].
 //   kRowsMinus: out = base - factor t.
-//   kRowsMinusLocal: out = base - factor sum_ab (2 if a != b) x_a x_b t_ab / |x|^2, the six fields
-//     one after another through the same registers; the powers of kz are applied here.
+//   kRowsMinusLocal: out = base - factor (t_0 + z t_1 + z^2 t_2) / |x|^2, the three fields one after
+//     another through the same registers.
 template <typename R>
 struct RowsArgs {
-  const Cx<R>* field[kTerms];
+  const Cx<R>* field[kPowers];
   R* out[3];
   const R* base;
-  size_t row0;  // row of the meshes that the fields' first row is
   int nrows;
   double factor;
   RealGeom G;
@@ -180,7 +176,7 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
   const int held = (nl * n + 15) & ~15;
   LineFft<R, false> L{buf, stage_twiddles(buf + held, tw, P.ntw), n, nl, 0, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
   const int pair0 = blockIdx.x * nl;
-  constexpr int NF = MODE == kRowsMinusLocal ? kTerms : 1;
+  constexpr int NF = MODE == kRowsMinusLocal ? kPowers : 1;
   constexpr int kSum = MODE == kRowsMinusLocal ? LineTile<R>::held : 1;
   double sum_a[kSum], sum_b[kSum];
 #pragma unroll
@@ -191,7 +187,7 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
     const Cx<R>* __restrict__ field = A.field[MODE == kRowsStore ? blockIdx.y : f];
     L.tid = hidden(threadIdx.x);
     if (f > 0) __syncthreads();
-    // the kept half of a thread's elements; fewer at a time beside the sums of the six fields
+    // the kept half of a thread's elements; fewer at a time beside the sums of the three fields
     constexpr int kBatch = MODE == kRowsMinusLocal ? LineTile<R>::held / 4 + 1 : LineTile<R>::held / 2 + 1;
     for (int t0 = L.tid; t0 < total; t0 += kBatch * L.nt) {
       Cx<R> a[kBatch], b[kBatch];
@@ -210,12 +206,6 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
         const int t = t0 + i * L.nt;
         if (t >= total) continue;
         const int line = quotient(t, div_nzc), k = t - line * S.nzc;
-        if (MODE == kRowsMinusLocal && (f == 2 || f == 4 || f == 5)) {
-          const double kz = wave(k, n, S.val[2]);
-          const double s = f == 5 ? kz * kz : kz;
-          a[i] = scaled(a[i], s);
-          b[i] = scaled(b[i], s);
-        }
         if (k == 0 || 2 * k == n) {
           buf[L.slot(line, k)] = {a[i].re, b[i].re};
         } else {
@@ -231,7 +221,7 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
           P, [](int, int) { return Cx<R>{R(0), R(0)}; },
           [&](int line, int e, Cx<R> v) {
             const int row = 2 * (pair0 + line);
-            const size_t at = (A.row0 + row) * n + e;
+            const size_t at = static_cast<size_t>(row) * n + e;
             if (row < A.nrows) out[at] = v.re;
             if (row + 1 < A.nrows) out[at + n] = v.im;
           });
@@ -240,7 +230,7 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
           P, [](int, int) { return Cx<R>{R(0), R(0)}; },
           [&](int line, int e, Cx<R> v) {
             const int row = 2 * (pair0 + line);
-            const size_t at = (A.row0 + row) * n + e;
+            const size_t at = static_cast<size_t>(row) * n + e;
             if (row < A.nrows)
               A.out[0][at] = static_cast<R>(static_cast<double>(A.base[at]) - A.factor * static_cast<double>(v.re));
             if (row + 1 < A.nrows)
@@ -254,19 +244,10 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
         int line, e;
         L.element(i, div_n, line, e);
         const Cx<R> v = buf[L.slot(line, e)];
-        const unsigned ra = static_cast<unsigned>(A.row0) + 2 * (pair0 + line), rb = ra + 1;
-        const unsigned ia = ra / S.n[1], ib = rb / S.n[1];
-        const double xa = A.G.o[0] + A.G.c[0] * static_cast<double>(ia);
-        const double ya = A.G.o[1] + A.G.c[1] * static_cast<double>(ra - ia * S.n[1]);
-        const double xb = A.G.o[0] + A.G.c[0] * static_cast<double>(ib);
-        const double yb = A.G.o[1] + A.G.c[1] * static_cast<double>(rb - ib * S.n[1]);
         const double z = A.G.o[2] + A.G.c[2] * static_cast<double>(e);
-        // x_a x_b, twice for a != b
-        const double pa = f <= 2 ? xa : f <= 4 ? ya : z, pb = f <= 2 ? xb : f <= 4 ? yb : z;
-        const double qa = f == 0 ? xa : f == 1 || f == 3 ? ya : z, qb = f == 0 ? xb : f == 1 || f == 3 ? yb : z;
-        const double twice = f == 0 || f == 3 || f == 5 ? 1. : 2.;
-        sum_a[i] += twice * (pa * qa) * static_cast<double>(v.re);
-        sum_b[i] += twice * (pb * qb) * static_cast<double>(v.im);
+        const double w = f == 0 ? 1. : f == 1 ? z : z * z;
+        sum_a[i] += w * static_cast<double>(v.re);
+        sum_b[i] += w * static_cast<double>(v.im);
       }
     }
   }
@@ -277,14 +258,14 @@ __global__ __launch_bounds__(1024) void k_rows_inverse(RowsArgs<R> A, LinePlan P
       if (!L.element(i, div_n, line, e)) continue;
       const int row = 2 * (pair0 + line);
       if (row >= A.nrows) continue;
-      const unsigned ra = static_cast<unsigned>(A.row0) + row, rb = ra + 1;
+      const unsigned ra = row, rb = ra + 1;
       const unsigned ia = ra / S.n[1], ib = rb / S.n[1];
       const double xa = A.G.o[0] + A.G.c[0] * static_cast<double>(ia);
       const double ya = A.G.o[1] + A.G.c[1] * static_cast<double>(ra - ia * S.n[1]);
       const double xb = A.G.o[0] + A.G.c[0] * static_cast<double>(ib);
       const double yb = A.G.o[1] + A.G.c[1] * static_cast<double>(rb - ib * S.n[1]);
       const double z = A.G.o[2] + A.G.c[2] * static_cast<double>(e);
-      const size_t at = (A.row0 + row) * n + e;
+      const size_t at = static_cast<size_t>(row) * n + e;
       A.out[0][at] = static_cast<R>(static_cast<double>(A.base[at]) -
                                     A.factor * (sum_a[i] / (xa * xa + ya * ya + z * z)));
       if (row + 1 < A.nrows)
@@ -313,69 +294,87 @@ __global__ __launch_bounds__(1024) void k_columns(Cx<R>* s0, Cx<R>* s1, Cx<R>* s
       [&](int line, int e, Cx<R> v) { base[static_cast<size_t>(e) * pitch + line] = v; });
 }
 
-// The six fields of the local line of sight, from X_p = IFFT_x(kx^p d), p = blockIdx.y: along y with
-// ky^0, ky^1, ky^2.  Elements with a Nyquist component (the header's half-sum):
+// A local line of sight: the sum over the pairs of axes of x_a x_b t_ab, grouped by its power of z, from
+// X_p = IFFT_x(kx^p d).  With t_ab along z still to be transformed,
+//   u = 0: x^2 t_xx + 2 x y t_xy + y^2 t_yy    from X2, ky X1, ky^2 X0, to where X2 was
+//   u = 1: kz (2 x t_xz + 2 y t_yz)            from X1, ky X0, to where X1 was
+//   u = 2: kz^2 t_zz                           from X0, in place
+// Elements with a Nyquist component (the header's half-sum):
 //   xy at ky Nyquist and xz at kz Nyquist keep the kx Nyquist term alone, whose transform along x is
 //   (-1)^x times its value; the x pass leaves those values in edge_y[kz] and edge_z[ky].
 //   yz at kz Nyquist keeps the ky Nyquist term alone.
+// A block owns its lines of the three arrays: the later outputs read them again, from L2.
 template <typename R>
-__global__ __launch_bounds__(1024) void k_columns_local(const Cx<R>* __restrict__ x0, const Cx<R>* __restrict__ x1,
-                                                       const Cx<R>* __restrict__ x2, Cx<R>* __restrict__ slab,
-                                                       size_t slab_field, const Cx<R>* __restrict__ edge_y,
+__global__ __launch_bounds__(1024) void k_columns_local(Cx<R>* x0, Cx<R>* x1, Cx<R>* x2, const Cx<R>* __restrict__ edge_y,
                                                        const Cx<R>* __restrict__ edge_z, LinePlan P,
-                                                       const Cx<R>* __restrict__ tw, int lw, SpecShape S, int plane0) {
+                                                       const Cx<R>* __restrict__ tw, int lw, SpecShape S, RealGeom G) {
   extern __shared__ double smem[];
   Cx<R>* buf = reinterpret_cast<Cx<R>*>(smem);
   const int n = P.n;
   const int W = 1 << lw;
   LineFft<R, true> L{buf, stage_twiddles(buf + (n + 1) * W, tw, P.ntw), n, W, lw, static_cast<int>(blockDim.x), static_cast<int>(threadIdx.x)};
-  const int power = blockIdx.y, ix = plane0 + blockIdx.z, kz0 = blockIdx.x * W;
-  const size_t row = static_cast<size_t>(S.pitch);
-  const Cx<R>* in = (power == 0 ? x0 : power == 1 ? x1 : x2) + static_cast<size_t>(ix) * n * row + kz0;
-  Cx<R>* out = slab + static_cast<size_t>(blockIdx.z) * n * row + kz0;
+  const int ix = blockIdx.y, kz0 = blockIdx.x * W;
+  const size_t row = static_cast<size_t>(S.pitch), first = static_cast<size_t>(ix) * n * row + kz0;
+  const double x = G.o[0] + G.c[0] * static_cast<double>(ix);
   const double sign = ix & 1 ? -1. : 1.;
   const double knx = S.n[0] % 2 ? 0. : sign * wave(S.n[0] / 2, S.n[0], S.val[0]);
-  const int outputs = 3 - power;
+  constexpr int kBatch = LineTile<R>::held / 2;
+  double sum_re[LineTile<R>::held], sum_im[LineTile<R>::held];
 #pragma unroll 1
-  for (int o = 0; o < outputs; o++) {
-    // ky power and field of output o: X0 -> zz yz yy, X1 -> xz xy, X2 -> xx
-    const int field = power == 0 ? 5 - o : power == 1 ? 2 - o : 0;
-    Cx<R>* dst = out + field * slab_field;
+  for (int t = 0; t < 6; t++) {
+    // output u, power o of y (and of ky), power p of x (and of kx)
+    const int u = t < 3 ? 0 : t < 5 ? 1 : 2, o = t < 3 ? t : t < 5 ? t - 3 : 0, p = 2 - u - o;
+    const Cx<R>* in = (p == 0 ? x0 : p == 1 ? x1 : x2) + first;
     L.tid = hidden(threadIdx.x);
-    Cx<R> d[LineTile<R>::held];  // read again for every output, from L2
+    // a few elements at a time beside the sums
+#pragma unroll 1
+    for (int i0 = 0; i0 < LineTile<R>::held; i0 += kBatch) {
+      Cx<R> d[kBatch];
 #pragma unroll
-    for (int i = 0; i < LineTile<R>::held; i++) {
-      int line, e;
-      L.element(i, 0, line, e);
-      d[i] = in[e * row + line];
-    }
-    __syncthreads();
+      for (int i = 0; i < kBatch; i++) {
+        int line, e;
+        L.element(i0 + i, 0, line, e);
+        d[i] = in[e * row + line];
+      }
+      if (i0 == 0) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < LineTile<R>::held; i++) {
-      int line, e;
-      if (!L.element(i, 0, line, e)) continue;
-      const bool nyz = nyquist(kz0 + line, S.n[2]), nyy = nyquist(e, n);
-      const double ky = wave(e, n, S.val[1]);
-      Cx<R> v = d[i];
-      double s = 1.;
-      if (power == 0) {
-        s = o == 0 ? 1. : o == 2 ? ky * ky : nyz == nyy ? ky : 0.;
-      } else if (power == 1 && o == 0 && nyz) {
-        s = knx;
-        if (knx != 0.) v = edge_z[e];
-      } else if (power == 1 && o == 1) {
-        s = ky;
-        if (nyy) {
+      for (int i = 0; i < kBatch; i++) {
+        int line, e;
+        if (!L.element(i0 + i, 0, line, e)) continue;
+        const bool nyz = nyquist(kz0 + line, S.n[2]), nyy = nyquist(e, n);
+        const double ky = wave(e, n, S.val[1]), kz = wave(kz0 + line, S.n[2], S.val[2]);
+        Cx<R> v = d[i];
+        double s = o == 0 ? 1. : o == 1 ? ky : ky * ky;
+        if (u == 1 && o == 1 && nyz != nyy) s = 0.;
+        if (u == 1 && o == 0 && nyz) {
+          s = knx;
+          if (knx != 0.) v = edge_z[e];
+        }
+        if (u == 0 && o == 1 && nyy) {
           s = kz0 + line < S.nzc ? knx * ky : 0.;
           if (s != 0.) v = edge_y[kz0 + line];
         }
+        if (u > 0) s *= u == 1 ? kz : kz * kz;
+        buf[L.slot(line, e)] = s == 0. ? Cx<R>{R(0), R(0)} : scaled(v, s);
       }
-      buf[L.slot(line, e)] = s == 0. ? Cx<R>{R(0), R(0)} : scaled(v, s);
     }
     __syncthreads();
-    L.template run<true, true, false>(
-        P, [](int, int) { return Cx<R>{R(0), R(0)}; },
-        [&](int line, int e, Cx<R> v) { dst[e * row + line] = v; });
+    L.template run<true, true, true>(P, [](int, int) { return Cx<R>{R(0), R(0)}; }, [](int, int, Cx<R>) {});
+    const double xs = p == 0 ? 1. : p == 1 ? x : x * x;
+    const double twice = t == 0 || t == 2 || t == 5 ? 1. : 2.;
+    Cx<R>* out = (u == 0 ? x2 : u == 1 ? x1 : x0) + first;
+#pragma unroll
+    for (int i = 0; i < LineTile<R>::held; i++) {
+      int line, e;
+      const bool ok = L.element(i, 0, line, e);
+      const double y = G.o[1] + G.c[1] * static_cast<double>(e);
+      const double w = twice * xs * (o == 0 ? 1. : o == 1 ? y : y * y);
+      const Cx<R> v = buf[L.slot(line, e)];
+      const double re = w * static_cast<double>(v.re), im = w * static_cast<double>(v.im);
+      sum_re[i] = o == 0 ? re : sum_re[i] + re;
+      sum_im[i] = o == 0 ? im : sum_im[i] + im;
+      if (ok && p == 0) out[e * row + line] = {static_cast<R>(sum_re[i]), static_cast<R>(sum_im[i])};
+    }
   }
 }
 
@@ -480,8 +479,6 @@ struct Layout {
   LinePlan P[3];
   int nzc = 0, pitch = 0;
   size_t elems = 0;     // one half spectrum
-  size_t plane = 0;     // one x plane of it
-  int slab = 0;         // x planes of a slab
 };
 
 template <typename R>
@@ -491,20 +488,15 @@ bool layout(const size_t* n, Layout& L) {
   constexpr int W = LineTile<R>::lines;
   L.nzc = static_cast<int>(n[2]) / 2 + 1;
   L.pitch = (L.nzc + W - 1) / W * W;
-  L.plane = n[1] * L.pitch;
-  L.elems = n[0] * L.plane;
-  const size_t per = L.plane * sizeof(Cx<R>) * kTerms;
-  const size_t fit = kSlabBytes / per;
-  L.slab = static_cast<int>(fit < 2 ? 2 : fit > n[0] ? n[0] : fit);
-  if (L.slab > static_cast<int>(n[0])) L.slab = static_cast<int>(n[0]);
+  L.elems = n[0] * n[1] * L.pitch;
   return true;
 }
 
 size_t edge_elems(const Layout& L, const size_t* n) { return (L.nzc + n[1] + 15) / 16 * 16; }
 
-// Complex elements of scratch: spectra, and for a local line of sight the slab and edge values.
+// Complex elements of scratch: spectra, and for a local line of sight the edge values.
 size_t scratch_elems(const Layout& L, const size_t* n, int spectra, bool local) {
-  return spectra * L.elems + (local ? kTerms * L.slab * L.plane + edge_elems(L, n) : 0);
+  return spectra * L.elems + (local ? edge_elems(L, n) : 0);
 }
 
 template <typename R>
@@ -596,7 +588,7 @@ struct Call {
   template <int MODE>
   int rows(const RowsArgs<R>& A, int fields) const {
     const double part = static_cast<double>(A.nrows) / (static_cast<double>(S.n[0]) * S.n[1]);
-    const double meshes = MODE == kRowsStore ? 2. * fields : MODE == kRowsMinus ? 3. : kTerms + 2.;
+    const double meshes = MODE == kRowsStore ? 2. * fields : MODE == kRowsMinus ? 3. : kPowers + 2.;
     return timed(meshes * part, [&]() {
       const LineRows B = line_rows<R>(L.P[2]);
       auto* k = &k_rows_inverse<R, MODE>;
@@ -676,26 +668,21 @@ int do_iterate(prh_workspace* ws, const R* src, const R* delta, R* out, const si
     A.nrows = S.n[0] * S.n[1];
     return C.template rows<kRowsMinus>(A, 1);
   }
-  Cx<R>*x1 = spec + L.elems, *x2 = x1 + L.elems, *slab = x2 + L.elems;
-  const size_t slab_field = L.slab * L.plane;
-  Cx<R>*edge_y = slab + kTerms * slab_field, *edge_z = edge_y + L.nzc;
+  Cx<R>*x1 = spec + L.elems, *x2 = x1 + L.elems, *edge_y = x2 + L.elems, *edge_z = edge_y + L.nzc;
   PRH_TRY((C.template pencils<kXLocal>(spec, spec, x1, x2, edge_y, edge_z)));
-  for (int f = 0; f < kTerms; f++) A.field[f] = slab + f * slab_field;
-  for (int x0 = 0; x0 < S.n[0]; x0 += L.slab) {
-    const int px = S.n[0] - x0 < L.slab ? S.n[0] - x0 : L.slab;
-    PRH_TRY(C.timed((3. + kTerms) * px / S.n[0], [&]() {
-      const LineCols B = line_cols<R>(L.P[1]);
-      const dim3 grid(S.pitch >> B.lw, 3, px);
-      auto* k = &k_columns_local<R>;
-      PRH_TRY(allow_lds(k, B.lds));
-      k<<<grid, B.threads, B.lds, C.s>>>(spec, x1, x2, slab, slab_field, edge_y, edge_z, L.P[1], C.tw(1), B.lw, S, x0);
-      return PRH_OK;
-    }));
-    A.row0 = static_cast<size_t>(x0) * S.n[1];
-    A.nrows = px * S.n[1];
-    PRH_TRY((C.template rows<kRowsMinusLocal>(A, kTerms)));
-  }
-  return PRH_OK;
+  PRH_TRY(C.timed(6, [&]() {
+    const LineCols B = line_cols<R>(L.P[1]);
+    const dim3 grid(S.pitch >> B.lw, S.n[0]);
+    auto* k = &k_columns_local<R>;
+    PRH_TRY(allow_lds(k, B.lds));
+    k<<<grid, B.threads, B.lds, C.s>>>(spec, x1, x2, edge_y, edge_z, L.P[1], C.tw(1), B.lw, S, A.G);
+    return PRH_OK;
+  }));
+  A.field[0] = x2;
+  A.field[1] = x1;
+  A.field[2] = spec;
+  A.nrows = S.n[0] * S.n[1];
+  return C.template rows<kRowsMinusLocal>(A, kPowers);
 }
 
 template <typename R>
