@@ -2071,6 +2071,15 @@ constexpr int kLegSweeps = 5;
 // solve of 64^3 2.17 ms against 1.98), and in one workgroup below kCoarseOne.
 constexpr size_t kLegCells = 20000, kCoarseOne = 1024;
 constexpr int kLegTile = 4;
+// Larger levels, up to kPartCells cells: the ends of the legs where two levels meet on tiles of kPartTile^3
+// cells, the last sweep with the residual and its restriction and the correction with the first sweep; the
+// other sweeps are launches of their own (two of them in one on these tiles take 10.5 us on 64^3 and 6.6 on
+// 32^3 in FP64, more than two apart).  In FP64 on 64^3 the ends take 12.6 us (down) and 8.3 (up), on 32^3 8.0
+// and 5.4.  Solves with and without: 192^3 FP64 6.23 and 6.37 ms, 256^3 FP32 meshes 7.10 and 7.47, 128^3 mixed
+// 2.83 and 2.89, 64^3 FP64 1.79 and 1.81.  Above 64^3 the halos cost what the launches do: with 128^3 too,
+// 256^3 takes 12.8 ms against 12.3, and 112^3 and 160^3 are the same either way.
+constexpr size_t kPartCells = size_t(64) * 64 * 64;
+constexpr int kPartTile = 8;
 
 template <typename R>
 struct LegJob {
@@ -2088,36 +2097,35 @@ struct LegArgs {
   LegJob<R> job[kMaxGroup];
 };
 
-template <typename R, bool DOWN>
+template <typename R, bool DOWN, int BT, int SW>
 struct LegTile {
-  static constexpr int BT = kLegTile;
   // cells around the tile: the residual's restriction looks one cell below the tile, the residual one
   // further on both sides, and each sweep one more
   static constexpr int kLo = DOWN ? 2 : 0, kHi = DOWN ? 1 : 0;
-  static constexpr int kPadLo = kLo + kLegSweeps, kPadHi = kHi + kLegSweeps;
+  static constexpr int kPadLo = kLo + SW, kPadHi = kHi + SW;
   static constexpr int kV = BT + kPadLo + kPadHi;  // staged extent of the iterate
   static constexpr int kF = kV - 2;                // and of the source
-  static constexpr int kC = DOWN ? 0 : BT / 2 + 7;  // and of the correction on the coarser level
+  static constexpr int kCLo = (SW + 1) / 2;        // and of the correction on the coarser level, from kCLo below
+  static constexpr int kC = DOWN ? 0 : BT / 2 + 2 * kCLo + 1;
+  static constexpr int kThreads = BT == kPartTile ? 512 : 1024;
   static constexpr size_t lds = sizeof(R) * (2 * static_cast<size_t>(kV) * kV * kV + static_cast<size_t>(kF) * kF * kF +
                                              static_cast<size_t>(kC) * kC * kC);
 };
-constexpr int kLegThreads = 1024;
 
 __device__ __forceinline__ int wrap_once(int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; }
 
 // One sweep (OP kOpJacobi, kOpJacobiZero) or the residual from v to w, over the tile and lo cells below,
 // hi above: two cells along x a thread and round.
-template <typename R, bool DOWN, int OP, bool LOCAL, bool FAST>
+template <typename R, typename L, int BT, int OP, bool LOCAL, bool FAST>
 __device__ __forceinline__ void leg_pass(const TileCoef<R>& T, const R* v, const R* f, R* w, int lo, int hi, int x0,
                                          int y0, int z0, R omega, R keep) {
-  using L = LegTile<R, DOWN>;
-  constexpr int BT = kLegTile, NV = L::kV, NF = L::kF;
+  constexpr int NV = L::kV, NF = L::kF;
   const LevelGeom<R>& G = T.G;
   const int E = BT + lo + hi, dv = L::kPadLo - lo;
   const int columns = E * E * ((E + 1) / 2);
   const float inv = 1.f / static_cast<float>(E);
 #pragma unroll 1
-  for (int t = threadIdx.x; t < columns; t += kLegThreads) {
+  for (int t = threadIdx.x; t < columns; t += L::kThreads) {
     // t / E and its quotient by E, exact below 2^22 with the half added
     const int tj = static_cast<int>((static_cast<float>(t) + 0.5f) * inv), k = t - tj * E;
     const int ti = static_cast<int>((static_cast<float>(tj) + 0.5f) * inv), j = tj - ti * E, i = 2 * ti;
@@ -2156,10 +2164,10 @@ __device__ __forceinline__ void leg_pass(const TileCoef<R>& T, const R* v, const
   __syncthreads();
 }
 
-template <typename R, bool DOWN, bool LOCAL, bool FAST>
-__global__ __launch_bounds__(kLegThreads) void k_vcycle_leg(LegArgs<R> A) {
-  using L = LegTile<R, DOWN>;
-  constexpr int BT = kLegTile, NV = L::kV, NF = L::kF, NT = kLegThreads;
+template <typename R, bool DOWN, int BT, int SW, bool LOCAL, bool FAST>
+__global__ __launch_bounds__((LegTile<R, DOWN, BT, SW>::kThreads)) void k_vcycle_leg(LegArgs<R> A) {
+  using L = LegTile<R, DOWN, BT, SW>;
+  constexpr int NV = L::kV, NF = L::kF, NT = L::kThreads;
   extern __shared__ double smem[];
   R* v = reinterpret_cast<R*>(smem);
   R* w = v + NV * NV * NV;
@@ -2193,8 +2201,8 @@ __global__ __launch_bounds__(kLegThreads) void k_vcycle_leg(LegArgs<R> A) {
     for (int q = 0; q < LC; q++) {
       const int t = tid + q * NT;
       const int k = t % NC, j = t / NC % NC, i = min(t / (NC * NC), NC - 1);
-      sc[q] = J.coarse[(wrap_once(x0 / 2 - 3 + i, c0) * c1 + wrap_once(y0 / 2 - 3 + j, c1)) * c2 +
-                       wrap_once(z0 / 2 - 3 + k, c2)];
+      sc[q] = J.coarse[(wrap_once(x0 / 2 - L::kCLo + i, c0) * c1 + wrap_once(y0 / 2 - L::kCLo + j, c1)) * c2 +
+                       wrap_once(z0 / 2 - L::kCLo + k, c2)];
     }
   }
 #pragma unroll
@@ -2212,8 +2220,9 @@ __global__ __launch_bounds__(kLegThreads) void k_vcycle_leg(LegArgs<R> A) {
     __syncthreads();
 #pragma unroll 1
     for (int t = tid; t < NV * NV * NV; t += NT) {
-      // prolong_value's sums; the tile starts on an even cell, kPadLo = 5 below it an odd one
-      const int k = t % NV + 1, j = t / NV % NV + 1, i = t / (NV * NV) + 1;
+      // prolong_value's sums; the tile starts on an even cell, kPadLo below it an odd one where that is odd
+      constexpr int ODD = 2 * L::kCLo - L::kPadLo;
+      const int k = t % NV + ODD, j = t / NV % NV + ODD, i = t / (NV * NV) + ODD;
       const R* u = uc + ((i >> 1) * NC + (j >> 1)) * NC + (k >> 1);
       const bool X = i & 1, Y = j & 1, Z = k & 1;
       R val = u[0];
@@ -2231,7 +2240,7 @@ __global__ __launch_bounds__(kLegThreads) void k_vcycle_leg(LegArgs<R> A) {
   __syncthreads();
   int left = A.niter - 1;
   if (DOWN && A.zero_start) {
-    leg_pass<R, DOWN, kOpJacobiZero, LOCAL, FAST>(T, v, f, w, L::kLo + left, L::kHi + left, x0, y0, z0, A.omega,
+    leg_pass<R, L, BT, kOpJacobiZero, LOCAL, FAST>(T, v, f, w, L::kLo + left, L::kHi + left, x0, y0, z0, A.omega,
                                                       A.keep);
     R* s = v;
     v = w;
@@ -2240,7 +2249,7 @@ __global__ __launch_bounds__(kLegThreads) void k_vcycle_leg(LegArgs<R> A) {
   }
 #pragma unroll 1
   for (; left >= 0; left--) {
-    leg_pass<R, DOWN, kOpJacobi, LOCAL, FAST>(T, v, f, w, L::kLo + left, L::kHi + left, x0, y0, z0, A.omega,
+    leg_pass<R, L, BT, kOpJacobi, LOCAL, FAST>(T, v, f, w, L::kLo + left, L::kHi + left, x0, y0, z0, A.omega,
                                                   A.keep);
     R* s = v;
     v = w;
@@ -2259,7 +2268,7 @@ __global__ __launch_bounds__(kLegThreads) void k_vcycle_leg(LegArgs<R> A) {
       J.out[at] = val;
   }
   if constexpr (DOWN) {
-    leg_pass<R, DOWN, kOpResidual, LOCAL, FAST>(T, v, f, w, 1, 0, x0, y0, z0, A.omega, A.keep);
+    leg_pass<R, L, BT, kOpResidual, LOCAL, FAST>(T, v, f, w, 1, 0, x0, y0, z0, A.omega, A.keep);
     constexpr int H = BT / 2;
     for (int t = tid; t < H * H * H; t += NT) {
       const int k = t % H, j = t / H % H, i = t / (H * H);
@@ -2652,39 +2661,40 @@ struct Solver {
   // niter damped-Jacobi sweeps; the iterate moves between cur and alt.  Where
   // the level allows, the sweeps go in fused pairs (the last one alone when
   // niter is odd), and a zero start's first two sweeps go in one launch.
-  // correction: the coarser level's, added to the iterate before the first sweep.
+  // correction: the coarser level's, added to the iterate before the first sweep.  sweeps: another number.
   int smooth(int l, Ptrs<R>& cur, Ptrs<R>& alt, const Ptrs<R>& src, bool zero_start, bool post = false,
-             const Ptrs<R>* correction = nullptr) {
+             const Ptrs<R>* correction = nullptr, int sweeps = -1) {
+    if (sweeps < 0) sweeps = niter;
     if (correction && !corrects(l)) {
       PRH_TRY(prolong_to(l, *correction, cur, true));
       correction = nullptr;
     }
-    if (niter <= 0) {
+    if (sweeps <= 0) {
       if (zero_start) PRH_TRY(fill_zero(l, cur));
       return PRH_OK;
     }
     const bool last_fused = post && fuse_top && l == 0;
-    for (int it = 0; it < niter;) {
+    for (int it = 0; it < sweeps;) {
       if (correction && it == 0) {
         PRH_TRY(jacobi_correct(l, cur, *correction, src, alt));
         swap_all(cur, alt, count);
         it++;
         continue;
       }
-      if (zero_start && it == 0 && niter >= 2 && !(pairable(l)) && !(last_fused && niter == 2) &&
+      if (zero_start && it == 0 && sweeps >= 2 && !(pairable(l)) && !(last_fused && sweeps == 2) &&
           after_zero_ok(l)) {
         // two sweeps: the iterate ends in cur, as after two single sweeps (two swaps)
         PRH_TRY(jacobi_after_zero(l, src, cur));
         it += 2;
         continue;
       }
-      if (pairable(l) && niter - it >= 2) {
-        PRH_TRY(jacobi_pair(l, cur, src, alt, zero_start && it == 0, last_fused && it + 2 == niter));
+      if (pairable(l) && sweeps - it >= 2) {
+        PRH_TRY(jacobi_pair(l, cur, src, alt, zero_start && it == 0, last_fused && it + 2 == sweeps));
         swap_all(cur, alt, count);
         it += 2;
         continue;
       }
-      PRH_TRY(jacobi(l, cur, src, alt, zero_start && it == 0, last_fused && it == niter - 1));
+      PRH_TRY(jacobi(l, cur, src, alt, zero_start && it == 0, last_fused && it == sweeps - 1));
       swap_all(cur, alt, count);
       it++;
     }
@@ -2740,13 +2750,22 @@ struct Solver {
     return least >= 12 && size(l) <= kLegCells;
   }
 
-  // one leg of the V-cycle on level l: the iterate goes from `in` to `out`
-  template <bool DOWN, bool FAST>
-  int leg(int l, const Ptrs<R>& in, const Ptrs<R>& src, const Ptrs<R>& out, const Ptrs<R>& coarse, bool zero_start) {
-    using L = LegTile<R, DOWN>;
-    constexpr int BT = kLegTile;
+  // whether level l goes in parts of a leg
+  bool parts_ok(int l) const {
+    if (niter < 1 || l + 1 >= nlev() || leg_ok(l) || size(l) > kPartCells) return false;
+    size_t least = n(l)[0];
+    for (int d = 1; d < 3; d++) least = n(l)[d] < least ? n(l)[d] : least;
+    return least >= 12;
+  }
+
+  // one leg of the V-cycle on level l, or part of one: `sweeps` sweeps take the iterate from `in` to `out`;
+  // acc: the result is added into the FP64 iterate where that is wanted (fuse_top)
+  template <bool DOWN, int BT, int SW, bool FAST>
+  int leg(int l, const Ptrs<R>& in, const Ptrs<R>& src, const Ptrs<R>& out, const Ptrs<R>& coarse, int sweeps,
+          bool zero_start, bool acc) {
+    using L = LegTile<R, DOWN, BT, SW>;
     LegArgs<R> A;
-    A.niter = niter;
+    A.niter = sweeps;
     A.zero_start = zero_start ? 1 : 0;
     A.omega = omega;
     A.keep = keep;
@@ -2754,6 +2773,7 @@ struct Solver {
     A.tx = static_cast<int>(ceil_div(m[0], BT));
     A.ty = static_cast<int>(ceil_div(m[1], BT));
     A.tz = static_cast<int>(ceil_div(m[2], BT));
+    acc = acc && l == 0 && fuse_top;
     const bool local = G[0][l].local;
     bool same = true;
     for (int j = 0; j < count; j++) same = same && (G[j][l].local != 0) == local;
@@ -2766,8 +2786,8 @@ struct Solver {
         J.T.G = G[j][l];
         J.T.K = G[j][l].local ? GlobalCoef<R>() : GlobalCoef<R>::make(G[j][l]);
         J.T.dinv = G[j][l].local ? R(0) : R(1) / J.T.K.d;
-        J.T.acc = !DOWN && l == 0 && fuse_top ? acc_top[j] : nullptr;
-        if (!DOWN && l == 0 && fuse_top) fused[j] = true;
+        J.T.acc = acc ? acc_top[j] : nullptr;
+        if (acc) fused[j] = true;
         J.in = in[j];
         J.src = src[j];
         J.out = out[j];
@@ -2775,22 +2795,23 @@ struct Solver {
       }
       const dim3 grid(A.tx * A.ty * A.tz, nj);
       const bool loc = G[j0][l].local;
-      auto* k = loc ? &k_vcycle_leg<R, DOWN, true, FAST> : &k_vcycle_leg<R, DOWN, false, FAST>;
+      auto* k = loc ? &k_vcycle_leg<R, DOWN, BT, SW, true, FAST> : &k_vcycle_leg<R, DOWN, BT, SW, false, FAST>;
       if (L::lds > 65536)
         PRH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                     static_cast<int>(L::lds)));
-      k<<<grid, kLegThreads, L::lds, s>>>(A);
+      k<<<grid, L::kThreads, L::lds, s>>>(A);
       PRH_LAUNCHED();
     }
     return PRH_OK;
   }
-  template <bool DOWN>
-  int leg(int l, const Ptrs<R>& in, const Ptrs<R>& src, const Ptrs<R>& out, const Ptrs<R>& coarse, bool zero_start) {
+  template <bool DOWN, int BT = kLegTile, int SW = kLegSweeps>
+  int leg(int l, const Ptrs<R>& in, const Ptrs<R>& src, const Ptrs<R>& out, const Ptrs<R>& coarse, int sweeps,
+          bool zero_start = false, bool acc = false) {
     // the fast FP32 forms where the sweeps of this level would take them
     const int nn[3] = {static_cast<int>(n(l)[0]), static_cast<int>(n(l)[1]), static_cast<int>(n(l)[2])};
     if constexpr (std::is_same<R, float>::value)
-      if (fast && tiled_ok(nn)) return leg<DOWN, true>(l, in, src, out, coarse, zero_start);
-    return leg<DOWN, false>(l, in, src, out, coarse, zero_start);
+      if (fast && tiled_ok(nn)) return leg<DOWN, BT, SW, true>(l, in, src, out, coarse, sweeps, zero_start, acc);
+    return leg<DOWN, BT, SW, false>(l, in, src, out, coarse, sweeps, zero_start, acc);
   }
 
   // src/multigrid.c:270-300
@@ -2798,14 +2819,26 @@ struct Solver {
     if (l >= coarse_level()) return vcycle_coarse(l, cur, alt, src, zero_start);
     if (leg_ok(l)) {
       const Ptrs<R> fc = f(l + 1);
-      PRH_TRY(leg<true>(l, cur, src, alt, fc, zero_start));
+      PRH_TRY(leg<true>(l, cur, src, alt, fc, niter, zero_start));
       swap_all(cur, alt, count);
       Ptrs<R> cc = v(l + 1);
       Ptrs<R> ca = tmp(l + 1);
       PRH_TRY(vcycle(l + 1, cc, ca, fc, true));
-      PRH_TRY(leg<false>(l, cur, src, alt, cc, false));
+      PRH_TRY(leg<false>(l, cur, src, alt, cc, niter, false, true));
       swap_all(cur, alt, count);
       return PRH_OK;
+    }
+    if (parts_ok(l)) {
+      const Ptrs<R> fc = f(l + 1);
+      if (niter > 1) PRH_TRY(smooth(l, cur, alt, src, zero_start, false, nullptr, niter - 1));
+      PRH_TRY((leg<true, kPartTile, 1>(l, cur, src, alt, fc, 1, zero_start && niter == 1)));
+      swap_all(cur, alt, count);
+      Ptrs<R> cc = v(l + 1);
+      Ptrs<R> ca = tmp(l + 1);
+      PRH_TRY(vcycle(l + 1, cc, ca, fc, true));
+      PRH_TRY((leg<false, kPartTile, 1>(l, cur, src, alt, cc, 1, false, niter == 1)));
+      swap_all(cur, alt, count);
+      return niter > 1 ? smooth(l, cur, alt, src, false, true, nullptr, niter - 1) : PRH_OK;
     }
     PRH_TRY(smooth(l, cur, alt, src, zero_start));
     if (l + 1 < nlev()) {
