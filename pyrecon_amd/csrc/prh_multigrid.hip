@@ -48,6 +48,8 @@ __device__ __forceinline__ void unflatten(I i, int n1, int n2, int& ix, int& iy,
   }
 }
 
+__device__ __forceinline__ int wrap_once(int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; }
+
 // A source read with its mean removed: each value f becomes f - sum[0] / n
 // (sum on the device, n the number of cells), the same FP64 subtraction as a
 // centred copy of f would hold.  sum == nullptr: the source as it is.
@@ -1504,6 +1506,130 @@ __global__ __launch_bounds__(kThreads) void k_restrict_quads(const float* __rest
   }
 }
 
+// The residual and its restriction in one launch, on levels whose planes are cut into tiles of 64 x 16
+// cells.  A block of 512 threads walks a run of x planes: the iterate's planes with two cells around the
+// tile's low sides and one beyond its high ones in a ring of 4 in LDS (two more in flight in registers), the
+// residual's with one cell below the tile in another ring of 4, one barrier a plane, and every second plane
+// 16 / 2 x 64 / 2 coarse cells from the residual's last three.  The residual is neither stored nor read back:
+// 16 of 33 bytes a cell in FP64, for 8% more cells of it.  16 rows, because 8 of them would make that 14% and
+// leave half of a round of threads idle.  512^3 in FP64: 0.82 ms, the two launches 0.67 and 0.28; 256^3 0.097
+// ms, 0.095 and 0.040.  Bound by the FP64 arithmetic behind a barrier a plane, two blocks a CU.  Same
+// expressions and order as the two launches, same bits.
+constexpr int kRestrictY = 16, kRestrictThreads = 512;
+template <typename R, bool LOCAL, bool FAST>
+__global__ __launch_bounds__(kRestrictThreads, 4) void k_residual_restrict(const R* __restrict__ v,
+                                                                          const R* __restrict__ f,
+                                                                          R* __restrict__ coarse, TileCoef<R> T,
+                                                                          int xlen) {
+  constexpr int TY = kRestrictY, NT = kRestrictThreads;
+  // the iterate on rows y0 - 2 .. y0 + 16 and columns z0 - 2 .. z0 + 64, the residual on rows y0 - 1 ..
+  // y0 + 15 and columns z0 - 1 .. z0 + 63
+  constexpr int W = kTileZ + 3, VP = W * (TY + 3), RW = kTileZ + 1, RP = RW * (TY + 1);
+  constexpr int PER = (VP + NT - 1) / NT, CELLS = (RP + NT - 1) / NT;
+  __shared__ R sv[4 * VP];
+  __shared__ R sr[4 * RP];
+  const LevelGeom<R>& G = T.G;
+  const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
+  const int tid = threadIdx.x;
+  // XCD-aware order (see k_stencil_tiled)
+  const int ztiles = n2 / kTileZ, ytiles = n1 / TY;
+  const unsigned nb = gridDim.x, bid = blockIdx.x, per = nb / 8;
+  const unsigned L = bid < per * 8 ? (bid % 8) * per + bid / 8 : bid;
+  const int zt = static_cast<int>(L % ztiles), yt = static_cast<int>((L / ztiles) % ytiles);
+  const int xr = static_cast<int>(L / (static_cast<unsigned>(ztiles) * ytiles));
+  const int z0 = zt * kTileZ, y0 = yt * TY, xb = xr * xlen;
+  const int xe = xb + xlen < n0 ? xb + xlen : n0;
+  const size_t s0 = static_cast<size_t>(n1) * n2;
+  int off[PER];
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    const int e = min(tid + NT * q, VP - 1);
+    off[q] = wrap_once(y0 - 2 + e / W, n1) * n2 + wrap_once(z0 - 2 + e % W, n2);
+  }
+  // residual cells of this thread; the last, partial round goes to the last wavefronts, the restriction to
+  // the first
+  int at[CELLS], fo[CELLS];
+  R py[CELLS], pz[CELLS];
+  bool has[CELLS];
+#pragma unroll
+  for (int q = 0; q < CELLS; q++) {
+    const int e = q + 1 < CELLS ? tid + NT * q : NT * q + NT - 1 - tid;
+    has[q] = e < RP;
+    const int i = has[q] ? e / RW : 0, j = has[q] ? e % RW : 0;
+    const int gy = wrap_once(y0 - 1 + i, n1), gz = wrap_once(z0 - 1 + j, n2);
+    at[q] = (i + 1) * W + j + 1;
+    fo[q] = gy * n2 + gz;
+    py[q] = LOCAL ? static_cast<R>(gy) + G.org[1] : R(0);
+    pz[q] = LOCAL ? static_cast<R>(gz) + G.org[2] : R(0);
+  }
+  R preA[PER], preB[PER];
+  auto fetch = [&](R(&dst)[PER], int xp) {
+    const R* src = v + static_cast<size_t>(wrap_once(xp, n0)) * s0;
+#pragma unroll
+    for (int q = 0; q < PER; q++) dst[q] = src[off[q]];
+  };
+  auto stash = [&](const R(&src)[PER], int slot) {
+#pragma unroll
+    for (int q = 0; q < PER; q++)
+      if (tid + NT * q < VP) sv[(slot & 3) * VP + tid + NT * q] = src[q];
+  };
+  // step t: the residual of plane xb - 1 + t; iterate plane xb - 2 + s lies in slot s & 3
+  const int steps = xe - xb + 1;
+  auto step = [&](int t, R(&cur)[PER], R(&next)[PER]) {
+    const int x = wrap_once(xb - 1 + t, n0);
+    if (t + 2 < steps) fetch(next, xb + 2 + t);
+    const R* fx = f + static_cast<size_t>(x) * s0;
+    const R *M = sv + (t & 3) * VP, *P = sv + ((t + 1) & 3) * VP, *N = sv + ((t + 2) & 3) * VP;
+    R px = R(0), A = R(0);
+    if (LOCAL) {
+      px = static_cast<R>(x) + G.org[0];
+      A = G.h2[0] * px * px;
+    }
+    R fv[CELLS];
+#pragma unroll
+    for (int q = 0; q < CELLS; q++) fv[q] = fx[fo[q]];
+#pragma unroll
+    for (int q = 0; q < CELLS; q++) {
+      if (q + 1 == CELLS && !has[q]) continue;
+      const int o = at[q];
+      R B = R(0), C = R(0), pypz = T.K.pypz;
+      if (LOCAL) {
+        B = G.h2[1] * py[q] * py[q];
+        C = G.h2[2] * pz[q] * pz[q];
+        pypz = py[q] * pz[q];
+      }
+      Hood<R> h;
+      h.c = P[o];
+      h.xp = N[o], h.xm = M[o], h.yp = P[o + W], h.ym = P[o - W], h.zp = P[o + 1], h.zm = P[o - 1];
+      h.xpyp = N[o + W], h.xmym = M[o - W], h.xmyp = M[o + W], h.xpym = N[o - W];
+      h.xpzp = N[o + 1], h.xmzm = M[o - 1], h.xmzp = M[o + 1], h.xpzm = N[o - 1];
+      h.ypzp = P[o + W + 1], h.ymzm = P[o - W - 1], h.ymzp = P[o - W + 1], h.ypzm = P[o + W - 1];
+      const int e = q + 1 < CELLS ? tid + NT * q : NT * q + NT - 1 - tid;
+      sr[(t & 3) * RP + e] =
+          stencil_cell<R, kOpResidual, LOCAL, FAST>(T, h, fv[q], px, A, py[q], B, pz[q], C, pypz, R(0), R(0));
+    }
+    if (t + 1 < steps) stash(cur, t + 3);
+    __syncthreads();
+    // planes t - 2, t - 1, t around an even one; the next step writes the fourth slot
+    if (t >= 2 && !(t & 1) && tid < (TY / 2) * (kTileZ / 2)) {
+      const int jy = tid / (kTileZ / 2), jz = tid % (kTileZ / 2);
+      const R* c = sr + 2 * jy * RW + 2 * jz;
+      coarse[(static_cast<size_t>((xb + t - 2) / 2) * (n1 / 2) + y0 / 2 + jy) * (n2 / 2) + z0 / 2 + jz] =
+          restrict_sum<R>([&](int a, int b, int k) { return c[((t - 2 + a) & 3) * RP + b * RW + k]; });
+    }
+  };
+  for (int k = 0; k < 3; k++) {
+    fetch(preA, xb - 2 + k);
+    stash(preA, k);
+  }
+  if (steps > 1) fetch(preA, xb + 1);
+  __syncthreads();
+  for (int t = 0; t < steps; t += 2) {
+    step(t, preA, preB);
+    if (t + 1 < steps) step(t + 1, preB, preA);
+  }
+}
+
 // Trilinear prolongation from the coarse mesh (c0, c1, c2) to the fine mesh,
 // one thread per fine cell (src/multigrid.c:177-205), either overwriting the
 // fine value or adding to it (the V-cycle correction, src/multigrid.c:296).
@@ -2112,8 +2238,6 @@ struct LegTile {
                                              static_cast<size_t>(kC) * kC * kC);
 };
 
-__device__ __forceinline__ int wrap_once(int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; }
-
 // One sweep (OP kOpJacobi, kOpJacobiZero) or the residual from v to w, over the tile and lo cells below,
 // hi above: two cells along x a thread and round.
 template <typename R, typename L, int BT, int OP, bool LOCAL, bool FAST>
@@ -2339,6 +2463,36 @@ static int launch_residual(const R* v, const R* f, O* r, const LevelGeom<R>& G, 
     launch_uneven<R, O, kOpResidual, kFast>(v, f, r, G, R(0), R(0), s, nullptr, C);
   else
     launch_uneven<R, O, kOpResidual>(v, f, r, G, R(0), R(0), s, nullptr, C);
+  PRH_LAUNCHED();
+  return PRH_OK;
+}
+
+// Whether the residual of a level and its restriction go in one launch: the levels in 64-wide tiles (FP64
+// solves of 512^3 66.0 ms against 67.3, with a global line of sight 61.4 against 63.6, of 256^3 11.85 against
+// 12.2, of 384 x 320 x 448 33.0 against 33.4, mixed 20.4 against 20.7).  FP32 whole rows do with a global line
+// of sight (mixed 512^3 34.6 against 34.9) and lose with a local one (38.2 against 38.0): their own residual
+// reads less of the neighbouring tiles.
+template <typename R>
+inline bool restricts_at_once(const LevelGeom<R>& G) {
+  if (std::is_same<R, float>::value && G.local && rows_cz(G.n) != 0) return false;
+  return tiled_ok(G.n) && !short_tiles(G.n) && G.n[1] % kRestrictY == 0 && G.n[0] % 2 == 0;
+}
+template <typename R, bool FAST>
+static int launch_residual_restrict(const R* v, const R* f, R* coarse, const LevelGeom<R>& G, hipStream_t s) {
+  TileCoef<R> T;
+  T.G = G;
+  T.K = G.local ? GlobalCoef<R>() : GlobalCoef<R>::make(G);
+  T.dinv = G.local ? R(0) : R(1) / T.K.d;
+  const int tiles = (G.n[2] / kTileZ) * (G.n[1] / kRestrictY);
+  // about 1024 blocks (two a CU at a time), runs of at least 8 planes (one more residual each)
+  const int chunks = (1024 + tiles - 1) / tiles;
+  int xlen = (G.n[0] + chunks - 1) / chunks;
+  xlen = xlen < 8 ? 8 : xlen + (xlen & 1);
+  const unsigned grid = static_cast<unsigned>(tiles) * ((G.n[0] + xlen - 1) / xlen);
+  if (G.local)
+    k_residual_restrict<R, true, FAST><<<grid, kRestrictThreads, 0, s>>>(v, f, coarse, T, xlen);
+  else
+    k_residual_restrict<R, false, FAST><<<grid, kRestrictThreads, 0, s>>>(v, f, coarse, T, xlen);
   PRH_LAUNCHED();
   return PRH_OK;
 }
@@ -2635,6 +2789,24 @@ struct Solver {
     return PRH_ERR_STATE;
   }
 
+  // the residual's restriction to fc; `r` holds the residual where that is a launch of its own
+  int residual_restrict(int l, const Ptrs<R>& in, const Ptrs<R>& src, const Ptrs<R>& r, const Ptrs<R>& fc) {
+    bool once = !grouped(l);
+    for (int j = 0; j < count; j++) once = once && restricts_at_once(G[j][l]);
+    if (!once) {
+      PRH_TRY(residual(l, in, src, r));
+      return restrict_to(l, r, fc);
+    }
+    constexpr bool kFast = std::is_same<R, float>::value;
+    for (int j = 0; j < count; j++) {
+      if (fast)
+        PRH_TRY((launch_residual_restrict<R, kFast>(in[j], src[j], fc[j], G[j][l], s)));
+      else
+        PRH_TRY((launch_residual_restrict<R, false>(in[j], src[j], fc[j], G[j][l], s)));
+    }
+    return PRH_OK;
+  }
+
   // the correction of a coarser level in the first sweep that follows it (kOpJacobiCorrect): levels in
   // 64-wide tiles or whole rows, a solve of 512^3 in 67.8 ms against 69.1 (FP64), 38.5 against 39.1 (mixed,
   // local line of sight) and 35.0 against 36.4 (mixed, global), of 384 x 320 x 448 in 33.7 against 34.4 and
@@ -2842,9 +3014,8 @@ struct Solver {
     }
     PRH_TRY(smooth(l, cur, alt, src, zero_start));
     if (l + 1 < nlev()) {
-      PRH_TRY(residual(l, cur, src, alt));
       const Ptrs<R> fc = f(l + 1);
-      PRH_TRY(restrict_to(l, alt, fc));
+      PRH_TRY(residual_restrict(l, cur, src, alt, fc));
       Ptrs<R> cc = v(l + 1);
       Ptrs<R> ca = tmp(l + 1);
       PRH_TRY(vcycle(l + 1, cc, ca, fc, true));
