@@ -495,9 +495,8 @@ def run_fft(args):
     """The FFT reconstructions on the workload's catalogs (FP64 meshes): IterativeFFTReconstruction
     (niterations=3, the value), PlaneParallelFFTReconstruction (global line of sight along z) and
     IterativeFFTParticleReconstruction (niterations=3).  A step: paint, smoothing and density contrast,
-    run, and the shifted positions of data and randoms.  Their shifts take and return host arrays
-    (the particle variant also keeps the data on the host), so a step includes those transfers; the
-    paint reads the device-resident catalogs.  The roofline is that of the 3-D transform passes."""
+    run, and the shifted positions of data and randoms.  Their shifts take and return host arrays,
+    so a step includes those transfers; the paint reads the device-resident catalogs.  The roofline is that of the 3-D transform passes."""
     import pyrecon_amd as P
     from pyrecon_amd import _lib
     from pyrecon_amd.device import device_name
@@ -544,13 +543,15 @@ def run_fft(args):
     achieved = main['fft_pass_gbs']
     roofline = dict(bound='hbm', achieved=achieved, peak=HBM_PEAK_GBS, unit='GB/s',
                     frac=round(achieved / HBM_PEAK_GBS, 4) if achieved else None, traffic=None,
-                    kernel='k_fft_axis: one axis pass of a 3-D c2c transform, 512^3 FP64, LDS Stockham passes; '
-                           'achieved = algorithmic bytes (4 n^3 x 8 B per complex pass, 3 n^3 x 8 B for the real-in '
-                           'and real-out passes) / average pass time (HIP events) over the IterativeFFTReconstruction '
+                    kernel='the half-spectrum passes (k_rows_forward, k_columns, k_pencils, k_columns_local, '
+                           'k_rows_inverse), 512^3 FP64; achieved = the spectra and meshes that each reads and '
+                           'writes (n^3 x 8 B each) / pass time (HIP events) over the IterativeFFTReconstruction '
                            'steps', avg_launch_ms=main['fft_pass_avg_ms'])
     cpu = None
     if not args.no_cpu_baseline:
-        ntrans = main['fft_passes_per_step'] // 3
+        # the reference's 3-D transforms: each of 3 iterations one forward and six inverse, the displacements
+        # one and three
+        ntrans = 3 * (1 + 6) + 1 + 3
         log('cpu baseline ({:d} transforms per step)'.format(ntrans))
         cpu = fft_cpu_baseline(cat, threads=args.workers, transforms=ntrans)
         log('cpu baseline', cpu)

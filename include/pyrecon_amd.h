@@ -487,11 +487,11 @@ int prh_fmg_mixed(prh_workspace *ws, const double *f1h, double *v1h, const size_
  * synchronizes and returns the summed device time, the number of launches
  * and the algorithmic bytes they moved (e.g. 3 n^3 words per Jacobi sweep).
  * Process-wide; not for concurrent use from several threads.              */
-#define PRH_TIMER_JACOBI_FINEST 0 /* damped-Jacobi sweeps on the finest level */
+#define PRH_TIMER_JACOBI_FINEST 0 /* damped-Jacobi sweeps on the finest level, in launches of their own */
 #define PRH_TIMER_PAINT_GATHER 1  /* CIC paint merge-gather kernel */
 #define PRH_TIMER_READ_SHIFTS 2   /* fused finite-difference read + shift kernel */
 #define PRH_TIMER_PAIR_FINEST 3   /* two fused FP32 sweeps on the finest level (mixed path) */
-#define PRH_TIMER_FFT_PASS 4      /* one axis pass of a 3-D transform (prh_fft3d_*) */
+#define PRH_TIMER_FFT_PASS 4      /* one axis pass of a 3-D transform (prh_fft3d_*, prh_spectral_*) */
 #define PRH_TIMER_COUNT 5
 int prh_timer_enable(int which, int enable);
 int prh_timer_reset(int which);
