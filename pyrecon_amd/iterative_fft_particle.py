@@ -6,7 +6,8 @@ density contrast, transforms, divides by k^2 and reads the displacement at the d
 of the displacement (reduced by beta / (1 + beta) in the first iteration) is then removed from the
 original positions.  All of it runs in the HIP library, the per-point algebra with numpy's expressions
 in the positions dtype; where numpy would promote beyond that dtype (f4 positions with a f8 mesh and a
-global line of sight or wrap), or for other dtypes, the algebra is the reference's numpy on the host.
+global line of sight or wrap, or with a growth rate or bias that is a numpy f8), or for other dtypes, the
+algebra is the reference's numpy on the host.
 """
 import numpy as np
 
@@ -14,7 +15,8 @@ from . import _lib
 from ._lib import lib, check
 from .device import DeviceArray, as_device, stream_handle
 from .mesh import RealMesh
-from .recon import BaseReconstruction, SpectralReconstruction, ReconstructionError, _suffix, distance, numpy_mean
+from .recon import BaseReconstruction, SpectralReconstruction, ReconstructionError, _suffix, distance, keeps_dtype, \
+    numpy_mean
 
 
 class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
@@ -83,7 +85,7 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
         self.mesh_data.smooth_gaussian(self.smoothing_radius)
         if self.has_randoms: self.mesh_randoms.smooth_gaussian(self.smoothing_radius)
         dtype = self._positions_data.dtype
-        if self._on_device(dtype):
+        if self._on_device(dtype) and keeps_dtype(dtype, self.f, self.bias):
             self._data, _ = as_device(self._positions_data, stream=self.stream)
             self._rec_data = self._data
             self._data_weights, _ = as_device(self._weights_data, stream=self.stream)
@@ -183,7 +185,8 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
         data = isinstance(positions, str) and positions == 'data'
         if not data and not isinstance(positions, DeviceArray): positions = np.asarray(positions)
         if self._data is not None if data else \
-                positions.ndim == 2 and positions.shape[1] == 3 and self._on_device(positions.dtype):
+                positions.ndim == 2 and positions.shape[1] == 3 and self._on_device(positions.dtype) \
+                and (field == 'disp' or keeps_dtype(positions.dtype, self.f)):
             return self._device_shifts(None if data else positions, field, shifted).numpy(stream=self.stream)
         if not data and isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
         shifts = self._host_shifts(positions, field)

@@ -32,6 +32,16 @@ def distance(position):
     return np.sqrt((position**2).sum(axis=-1))
 
 
+def keeps_dtype(dtype, *scalars):
+    """Whether numpy's products of an array of ``dtype`` with ``scalars`` stay in ``dtype``: Python's numbers take
+    it on, numpy's bring their own (an FP64 growth rate makes FP64 of FP32 displacements)."""
+    for scalar in scalars:
+        if type(scalar) in (int, float): continue
+        scalar = np.asarray(scalar)
+        if scalar.ndim or np.promote_types(dtype, scalar.dtype) != dtype: return False
+    return True
+
+
 def _suffix(dtype):
     return 'f32' if np.dtype(dtype) == np.float32 else 'f64'
 
@@ -391,7 +401,8 @@ class SpectralReconstruction(BaseReconstruction):
     def _wrapped_shifts(self, positions, field, shifted):
         """The same with the positions wrapped first, on the device; host arrays out."""
         if not isinstance(positions, DeviceArray): positions = np.asarray(positions)
-        if positions.ndim != 2 or positions.shape[1] != 3 or not self._device_dtype(positions.dtype):
+        if positions.ndim != 2 or positions.shape[1] != 3 or not self._device_dtype(positions.dtype) \
+                or (field != 'disp' and not keeps_dtype(positions.dtype, self.f)):
             # other dtypes take numpy's promotions on the host
             if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
             shifts = self._host_shifts(positions, field)
