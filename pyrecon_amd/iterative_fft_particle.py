@@ -184,9 +184,10 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
         """Shifts or shifted positions (host arrays out)."""
         data = isinstance(positions, str) and positions == 'data'
         if not data and not isinstance(positions, DeviceArray): positions = np.asarray(positions)
-        if self._data is not None if data else \
-                positions.ndim == 2 and positions.shape[1] == 3 and self._on_device(positions.dtype) \
-                and (field == 'disp' or keeps_dtype(positions.dtype, self.f)):
+        on_device = self._data is not None if data else \
+            positions.ndim == 2 and positions.shape[1] == 3 and self._on_device(positions.dtype) \
+            and (field == 'disp' or keeps_dtype(positions.dtype, self.f))
+        if on_device and self._psi_on_mesh():
             return self._device_shifts(None if data else positions, field, shifted).numpy(stream=self.stream)
         if not data and isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
         shifts = self._host_shifts(positions, field)
@@ -218,10 +219,11 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
     def _host_shifts(self, positions, field):
         """The shifts with the reference's numpy algebra on the host."""
         if isinstance(positions, str):
-            shifts = self._read_psi(self._rec_data, wrap=True)
+            positions = self._positions_rec_data
+            shifts = self._read_psi(positions, wrap=True)
             if field == 'disp':
                 return shifts
-            rsd = self._positions_data - self._rec_data
+            rsd = self._positions_data - positions
             if field == 'rsd':
                 return rsd
             shifts += rsd

@@ -337,6 +337,16 @@ class SpectralReconstruction(BaseReconstruction):
             raise ReconstructionError('run the reconstruction before reading shifts')
         return field
 
+    def _psi_on_mesh(self):
+        """Whether :attr:`mesh_psi` are three meshes of this reconstruction's shape, box, dtype and stream, as one
+        pass over them takes them (a program may put its own in their place; those are read one by one)."""
+        def same(psi):
+            a, b = psi.info, self.info
+            return stream_handle(psi.stream) == stream_handle(self.stream) and (a is b or (
+                a.dtype == b.dtype and all(np.array_equal(getattr(a, name), getattr(b, name))
+                                           for name in ('nmesh', 'boxsize', 'boxcenter'))))
+        return len(self.mesh_psi) == 3 and all(isinstance(psi, RealMesh) and same(psi) for psi in self.mesh_psi)
+
     def _read_psi_device(self, pos, field=_lib.FIELD_VALUE, wrap=False, shifted=False, odtype=None, psis=None):
         """:attr:`mesh_psi` (or ``psis``) read by CIC at the device positions: the (N, 3) displacements, or the
         shifts or shifted positions they give (pyrecon/recon.py:255-325, without wrap)."""
@@ -395,14 +405,23 @@ class SpectralReconstruction(BaseReconstruction):
             pos, is_host = as_device(np.asarray(positions, dtype='f8'), stream=self.stream)
         odt = pos.dtype
         if field == 'rsd' and self.los is not None: odt = np.promote_types(pos.dtype, self.info.dtype)
-        out = self._read_psi_device(pos, field=self._FIELDS[field], shifted=shifted, odtype=odt)
+        if self._psi_on_mesh():
+            out = self._read_psi_device(pos, field=self._FIELDS[field], shifted=shifted, odtype=odt)
+        else:
+            comps = [psi.read_cic(pos, wrap=False) for psi in self.mesh_psi]
+            los = None if self.los is None else np.ascontiguousarray(self.los, dtype=self.info.dtype)
+            out = DeviceArray((len(pos), 3), odt, stream=self.stream)
+            fn = getattr(lib, 'prh_shift_algebra_' + _suffix(self.info.dtype))
+            check(fn(pos.ptr, _lib.dtype_code(pos.dtype), comps[0].ptr, comps[1].ptr, comps[2].ptr, len(pos),
+                     float(self.f), los.ctypes.data if los is not None else None, self._FIELDS[field],
+                     int(bool(shifted)), out.ptr, _lib.dtype_code(odt), stream_handle(self.stream)), 'shift algebra')
         return out.numpy(stream=self.stream) if is_host else out
 
     def _wrapped_shifts(self, positions, field, shifted):
         """The same with the positions wrapped first, on the device; host arrays out."""
         if not isinstance(positions, DeviceArray): positions = np.asarray(positions)
         if positions.ndim != 2 or positions.shape[1] != 3 or not self._device_dtype(positions.dtype) \
-                or (field != 'disp' and not keeps_dtype(positions.dtype, self.f)):
+                or (field != 'disp' and not keeps_dtype(positions.dtype, self.f)) or not self._psi_on_mesh():
             # other dtypes take numpy's promotions on the host
             if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
             shifts = self._host_shifts(positions, field)
