@@ -243,16 +243,21 @@ class DeviceArray(object):
             pass
 
 
+def device_view(obj):
+    """A device object (a :class:`DeviceArray`, a device tensor) as a DeviceArray, without a copy; None for others."""
+    if isinstance(obj, DeviceArray): return obj
+    data_ptr = getattr(obj, 'data_ptr', None)
+    if data_ptr is None or not getattr(obj, 'is_cuda', False): return None
+    if not obj.is_contiguous():
+        raise ValueError('device tensors must be contiguous')
+    np_dtype = np.dtype(str(obj.dtype).replace('torch.', ''))
+    return DeviceArray(tuple(obj.shape), np_dtype, ptr=data_ptr(), owner=False, base=obj)
+
+
 def as_device(obj, dtype=None, stream=None):
     """Return ``(device_array, is_host)``: wrap a device object or upload a host array."""
-    if isinstance(obj, DeviceArray):
-        return obj, False
-    data_ptr = getattr(obj, 'data_ptr', None)
-    if data_ptr is not None and getattr(obj, 'is_cuda', False):
-        if not obj.is_contiguous():
-            raise ValueError('device tensors must be contiguous')
-        np_dtype = np.dtype(str(obj.dtype).replace('torch.', ''))
-        return DeviceArray(tuple(obj.shape), np_dtype, ptr=data_ptr(), owner=False, base=obj), False
+    view = device_view(obj)
+    if view is not None: return view, False
     array = np.asarray(obj)
     if dtype is not None: array = array.astype(dtype, copy=False)
     return DeviceArray.from_numpy(array, stream=stream), True

@@ -13,7 +13,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import lib, check
-from .device import DeviceArray, as_device, stream_handle
+from .device import DeviceArray, as_device, device_view, stream_handle
 from .mesh import RealMesh
 from .recon import BaseReconstruction, SpectralReconstruction, ReconstructionError, _suffix, distance, keeps_dtype, \
     numpy_mean
@@ -24,9 +24,10 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
 
     def assign_data(self, positions, weights=None):
         """Paint the data and keep their positions (for :meth:`run`) and weights (iterative_fft_particle.py:16-31)."""
-        if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
-        if isinstance(weights, DeviceArray): weights = weights.numpy(stream=self.stream)
-        positions = np.asarray(positions)
+        view = device_view(positions)
+        positions = view.numpy(stream=self.stream) if view is not None else np.asarray(positions)
+        view = device_view(weights)
+        if view is not None: weights = view.numpy(stream=self.stream)
         if weights is None:
             weights = np.ones_like(positions, shape=(len(positions),))
         if self.wrap: positions = self.info.wrap(positions)
@@ -183,13 +184,14 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
     def _shifts(self, positions, field, shifted):
         """Shifts or shifted positions (host arrays out)."""
         data = isinstance(positions, str) and positions == 'data'
-        if not data and not isinstance(positions, DeviceArray): positions = np.asarray(positions)
+        view = device_view(positions)
+        if not data: positions = view if view is not None else np.asarray(positions)
         on_device = self._data is not None if data else \
             positions.ndim == 2 and positions.shape[1] == 3 and self._on_device(positions.dtype) \
             and (field == 'disp' or keeps_dtype(positions.dtype, self.f))
         if on_device and self._psi_on_mesh():
             return self._device_shifts(None if data else positions, field, shifted).numpy(stream=self.stream)
-        if not data and isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
+        if view is not None: positions = view.numpy(stream=self.stream)
         shifts = self._host_shifts(positions, field)
         if not shifted: return shifts
         positions = (self._positions_data if data else positions) - shifts

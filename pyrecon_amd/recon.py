@@ -13,7 +13,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import lib, check, MeshError
-from .device import DeviceArray, as_device, stream_handle
+from .device import DeviceArray, as_device, device_view, stream_handle
 from .mesh import MeshInfo, RealMesh, Workspace
 
 
@@ -419,11 +419,12 @@ class SpectralReconstruction(BaseReconstruction):
 
     def _wrapped_shifts(self, positions, field, shifted):
         """The same with the positions wrapped first, on the device; host arrays out."""
-        if not isinstance(positions, DeviceArray): positions = np.asarray(positions)
+        view = device_view(positions)
+        positions = view if view is not None else np.asarray(positions)
         if positions.ndim != 2 or positions.shape[1] != 3 or not self._device_dtype(positions.dtype) \
                 or (field != 'disp' and not keeps_dtype(positions.dtype, self.f)) or not self._psi_on_mesh():
             # other dtypes take numpy's promotions on the host
-            if isinstance(positions, DeviceArray): positions = positions.numpy(stream=self.stream)
+            if view is not None: positions = view.numpy(stream=self.stream)
             shifts = self._host_shifts(positions, field)
             return self.info.wrap(positions - shifts) if shifted else shifts
         pos, _ = as_device(positions, stream=self.stream)
