@@ -372,10 +372,12 @@ class SpectralReconstruction(BaseReconstruction):
         return out
 
     def _device_dtype(self, dtype):
-        """Whether numpy's promotions of positions of ``dtype`` with the box and a global line of sight (both in
-        the mesh dtype) all stay in ``dtype``, as the device's per-point algebra has it."""
+        """Whether numpy's promotions of positions of ``dtype`` with the box (in the mesh dtype) and a global line of
+        sight (in that too, unless a program put its own in place) all stay in ``dtype``, as the device's per-point
+        algebra has it."""
         dtype = np.dtype(dtype)
-        return dtype in (np.dtype('f4'), np.dtype('f8')) and np.promote_types(dtype, self.info.dtype) == dtype
+        if dtype not in (np.dtype('f4'), np.dtype('f8')) or np.promote_types(dtype, self.info.dtype) != dtype: return False
+        return self.los is None or np.promote_types(dtype, np.asarray(self.los).dtype) == dtype
 
     def _point_algebra(self, op, x, a=None, s=None, t=None, out=None, field=_lib.FIELD_DISP_RSD, first=0., shifted=False,
                        skip=0, outside=False):

@@ -55,3 +55,22 @@ def test_particle(f, bias, dtype, wrap, los):
     out = run(True)
     assert out[0].dtype == promoted(f)
     for a, b in zip(out, run(False)): assert_same(a, b)
+
+
+@pytest.mark.parametrize('algorithm', ['IterativeFFT', 'IterativeFFTParticle'])
+def test_own_line_of_sight(algorithm):
+    """A line of sight in f8 that a program put in the place of an f4 reconstruction's: f8 shifts, as numpy has them."""
+    import pyrecon_amd
+    recon = getattr(pyrecon_amd, algorithm + 'Reconstruction')(f=0.8, bias=2., los='x', nmesh=(32, 24, 40), boxsize=BOX,
+                                                               boxcenter=CENTER, dtype='f4', wrap=True)
+    recon.los = np.array([0.3, 0.4, np.sqrt(0.75)])
+    recon.assign_data(points(20000, 'f4', True, 1))
+    recon.set_density_contrast(smoothing_radius=30.)
+    recon.run()
+    x = points(1000, 'f4', True, 2)
+    for field in ('rsd', 'disp+rsd'):
+        expect = recon._host_shifts(x, field)
+        if field == 'rsd' or algorithm == 'IterativeFFTParticle': assert expect.dtype == np.float64
+        assert_same(recon.read_shifts(x, field), expect)
+        assert_same(recon.read_shifted_positions(x, field), recon.info.wrap(x - expect))
+    if algorithm == 'IterativeFFTParticle': assert recon._positions_rec_data.dtype == np.float64
