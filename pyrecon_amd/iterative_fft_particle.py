@@ -15,8 +15,8 @@ from . import _lib
 from ._lib import lib, check
 from .device import DeviceArray, as_device, device_view, stream_handle
 from .mesh import RealMesh
-from .recon import BaseReconstruction, SpectralReconstruction, ReconstructionError, _suffix, distance, keeps_dtype, \
-    numpy_mean
+from .recon import BaseReconstruction, SpectralReconstruction, ReconstructionError, _suffix, distance, keeps_class, \
+    keeps_dtype, numpy_mean
 
 
 class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
@@ -179,6 +179,9 @@ class OriginalIterativeFFTParticleReconstruction(SpectralReconstruction):
     def read_shifted_positions(self, positions, field='disp+rsd'):
         """``positions - read_shifts(positions)`` (``'data'``: the data given to :meth:`assign_data`), wrapped
         if :attr:`wrap` (iterative_fft_particle.py:214-239)."""
+        if not isinstance(positions, str) and keeps_class(positions):
+            positions = positions - self._shifts(positions, self._check_field(field), False)
+            return self.info.wrap(positions) if self.wrap else positions
         return self._shifts(positions, self._check_field(field), True)
 
     def _shifts(self, positions, field, shifted):

@@ -42,6 +42,12 @@ def keeps_dtype(dtype, *scalars):
     return True
 
 
+def keeps_class(positions):
+    """Whether numpy's difference with ``positions`` is of their own class: other host arrays than numpy's plain ones
+    (masked arrays, host tensors)."""
+    return device_view(positions) is None and type(positions) not in (np.ndarray, list, tuple)
+
+
 def _suffix(dtype):
     return 'f32' if np.dtype(dtype) == np.float32 else 'f64'
 
@@ -465,4 +471,6 @@ class SpectralReconstruction(BaseReconstruction):
     def read_shifted_positions(self, positions, field='disp+rsd'):
         """``positions - read_shifts(positions)``, wrapped if :attr:`wrap` (pyrecon/recon.py:304-325)."""
         field = self._check_field(field)
+        if self.wrap and keeps_class(positions):
+            return self.info.wrap(positions - self._wrapped_shifts(positions, field, False))
         return self._wrapped_shifts(positions, field, True) if self.wrap else self._device_shifts(positions, field, True)
