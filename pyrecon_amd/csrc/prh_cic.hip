@@ -2238,7 +2238,8 @@ static int read_psi_all(prh_workspace* ws, const R* const* psi, const ReadArgs<R
 }
 
 // Shifts of the FFT reconstructions (recon.py:255-325 without wrap): the displacement of point i
-// is (s0[i], s1[i], s2[i]), read by CIC from the three displacement meshes in the positions dtype.
+// is (s0[i], s1[i], s2[i]), read by CIC from the three displacement meshes in the positions dtype.  For meshes that are not alike, which
+// one pass (k_read_psi) does not take.
 template <typename R, typename P, typename O>
 __global__ __launch_bounds__(kCicThreads) void k_shift_algebra(const P* __restrict__ pos, const P* __restrict__ s0,
                                                                const P* __restrict__ s1, const P* __restrict__ s2,

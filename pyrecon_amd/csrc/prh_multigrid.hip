@@ -2412,8 +2412,9 @@ __global__ __launch_bounds__((LegTile<R, DOWN, BT, SW>::kThreads)) void k_vcycle
 static size_t ncells(const size_t* n) { return n[0] * n[1] * n[2]; }
 
 template <typename R>
-// acc (FP32 fast sweeps on blocked levels only): add the result into this FP64
-// mesh instead of storing it; *fused tells whether that was done.
+// acc (FP32 sweeps of an iterate, fast ones where the level is in 64-wide tiles):
+// add the result into this FP64 mesh instead of storing it; *fused tells whether
+// that was done.
 static int launch_jacobi(const R* v, const R* f, R* out, const LevelGeom<R>& G, R omega, R keep,
                          bool zero_in, hipStream_t s, int timer = -1, bool fast = false,
                          double* acc = nullptr, bool* fused = nullptr) {
@@ -2589,10 +2590,10 @@ static void swap_all(Ptrs<R>& a, Ptrs<R>& b, int count) {
 
 // State of one solve over `count` hierarchies of the same shape (count = 1
 // for the reference-shaped entry points).  Every level runs the schedule of
-// src/multigrid.c:270-328 for all jobs in lock step.  Levels that the blocked
-// kernels cover are launched once per job (they fill the device alone); the
-// smaller levels, which the generic kernels handle and whose launches are
-// latency-bound, are launched once for the whole group.
+// src/multigrid.c:270-328 for all jobs in lock step.  Sweeps of levels in 64-wide
+// tiles, and of others of kFlexMin cells, are launched once per job (they fill
+// the device alone, or nearly); those of the other levels, the legs and their
+// ends, whose launches are latency-bound, once for the whole group.
 template <typename R>
 struct Solver {
   int count = 1;
@@ -2604,7 +2605,7 @@ struct Solver {
   bool fast = false;  // fast FP32 kernels on the blocked levels (mixed-precision corrections)
   bool pair_enabled = true;  // with fast: two sweeps per launch where the level allows
   // When fuse_top is set, the last post-smoothing sweep of level 0 adds its result into the FP64
-  // mesh acc_top[j] instead of storing it; fused[j] tells whether it could (blocked levels).
+  // mesh acc_top[j] instead of storing it; fused[j] tells whether it could (launch_jacobi, leg).
   bool fuse_top = false;
   double* acc_top[kMaxGroup] = {};
   bool fused[kMaxGroup] = {};

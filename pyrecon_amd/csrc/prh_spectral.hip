@@ -587,9 +587,8 @@ struct Call {
 
   template <int MODE>
   int rows(const RowsArgs<R>& A, int fields) const {
-    const double part = static_cast<double>(A.nrows) / (static_cast<double>(S.n[0]) * S.n[1]);
     const double meshes = MODE == kRowsStore ? 2. * fields : MODE == kRowsMinus ? 3. : kPowers + 2.;
-    return timed(meshes * part, [&]() {
+    return timed(meshes, [&]() {
       const LineRows B = line_rows<R>(L.P[2]);
       auto* k = &k_rows_inverse<R, MODE>;
       PRH_TRY(allow_lds(k, B.lds));

@@ -27,26 +27,6 @@ struct Coef {
   R px, py, pz, g, cx, cy, cz;
 };
 
-// cell_coef() with g given (the same expressions after g).
-template <typename R>
-__device__ __forceinline__ Coef<R> cell_coef_g(const LevelGeom<R>& G, int ix, int iy, int iz, R g) {
-  Coef<R> k;
-  if (G.local) {
-    k.px = static_cast<R>(ix) + G.org[0];
-    k.py = static_cast<R>(iy) + G.org[1];
-    k.pz = static_cast<R>(iz) + G.org[2];
-  } else {
-    k.px = G.losc[0];
-    k.py = G.losc[1];
-    k.pz = G.losc[2];
-  }
-  k.g = g;
-  k.cx = G.ih2[0] + k.g * k.px * k.px;
-  k.cy = G.ih2[1] + k.g * k.py * k.py;
-  k.cz = G.ih2[2] + k.g * k.pz * k.pz;
-  return k;
-}
-
 template <typename R>
 __device__ __forceinline__ Coef<R> cell_coef(const LevelGeom<R>& G, int ix, int iy, int iz) {
   Coef<R> k;
