@@ -2920,7 +2920,24 @@ struct Solver {
     size_t least = n(l)[0];
     for (int d = 1; d < 3; d++) least = n(l)[d] < least ? n(l)[d] : least;
     // halo cells wrap once around the level
-    return least >= 12 && size(l) <= kLegCells;
+    return least >= 12 && size(l) <= kLegCells && (count == 1 || group_leg(l));
+  }
+
+  // Whether a group's legs pay on level l.  A leg of one problem is bound by latency, those of several by
+  // the halos that their workgroups repeat once these no longer run at the same time: one FP64 tile or two
+  // FP32 ones a CU.  The one-workgroup kernel takes kCoarseGroup problems a launch, in a time that grows
+  // with the level (a V-cycle's two legs about 29 us), so a second launch leaves the legs a second round.
+  // Solves of 8 meshes of 48^3 in FP64: 4.40 ms with legs as for one, 3.15 so (2: 2.15 and 1.95), of 4 of
+  // 80 x 96 x 112 6.62 and 5.75, of 8 of 20 x 24 x 28 2.04 and 1.32; 8 of 32^3, whose 16^3 keeps its legs,
+  // 1.86, 2.30 without.
+  bool group_leg(int l) const {
+    const size_t launches =
+        size(l) <= kCoarseCells && nlev() - l <= kMaxCoarse ? (count + kCoarseGroup - 1) / kCoarseGroup : 0;
+    constexpr size_t kOneLaunch = sizeof(R) == 8 ? 2048 : 3072, kAtOnce = sizeof(R) == 8 ? 256 : 512;
+    if (launches > 0 && launches * size(l) <= kOneLaunch) return false;
+    const size_t* m = n(l);
+    const size_t tiles = static_cast<size_t>(ceil_div(m[0], kLegTile)) * ceil_div(m[1], kLegTile) * ceil_div(m[2], kLegTile);
+    return count * tiles <= kAtOnce * (launches > 0 ? launches : 1);
   }
 
   // whether level l goes in parts of a leg
