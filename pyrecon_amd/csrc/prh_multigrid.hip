@@ -1016,8 +1016,14 @@ inline bool short_tiles(const int* n) { return static_cast<size_t>(n[0]) * n[1] 
 // 224 takes 24.4 ms (29.5 with the columns below, 35.1 with a cell a thread).  FP32 ones, half the size
 // and mostly in cache, go through the columns: 21.4 ms for 384 x 320 x 448 against 22.9 with FLEX tiles.
 constexpr size_t kFlexMin = 500000;
-inline bool fills_alone(const int* n) {
-  return !tiled_ok(n) && static_cast<size_t>(n[0]) * n[1] * n[2] >= kFlexMin;
+// Of those levels, the ones whose sweeps a group launches mesh by mesh; smaller ones go in one launch for
+// the group, a cell a thread.  FP32: 8 meshes of 80 x 96 x 112 mesh by mesh 6.42 ms, together 5.70, of 112^3
+// 7.76 and 7.47, of 160 x 160 x 96 12.2 and 12.9.  FP64: 8 of 80 x 96 x 112 10.00 and 9.62, of 128 x 112 x
+// 96 15.9 and 16.7, of 160 x 160 x 96 25.8 and 30.1.
+template <typename R>
+constexpr size_t kGroupAlone = sizeof(R) == 8 ? 1250000 : 1500000;
+inline bool fills_alone(const int* n, size_t least = kFlexMin) {
+  return !tiled_ok(n) && static_cast<size_t>(n[0]) * n[1] * n[2] >= least;
 }
 // The plane cut evenly: tiles along z of at most 64 cells, and along y of as many rows as two cells a
 // thread take.
@@ -2591,9 +2597,9 @@ static void swap_all(Ptrs<R>& a, Ptrs<R>& b, int count) {
 // State of one solve over `count` hierarchies of the same shape (count = 1
 // for the reference-shaped entry points).  Every level runs the schedule of
 // src/multigrid.c:270-328 for all jobs in lock step.  Sweeps of levels in 64-wide
-// tiles, and of others of kFlexMin cells, are launched once per job (they fill
-// the device alone, or nearly); those of the other levels, the legs and their
-// ends, whose launches are latency-bound, once for the whole group.
+// tiles, and of others of kGroupAlone cells, are launched once per job (they
+// fill the device alone, or nearly); those of the other levels, the legs and
+// their ends, whose launches are latency-bound, once for the whole group.
 template <typename R>
 struct Solver {
   int count = 1;
@@ -2623,7 +2629,7 @@ struct Solver {
   }
   bool grouped(int l) const {
     int nn[3] = {static_cast<int>(n(l)[0]), static_cast<int>(n(l)[1]), static_cast<int>(n(l)[2])};
-    return count > 1 && !tiled_ok(nn) && !fills_alone(nn);
+    return count > 1 && !tiled_ok(nn) && !fills_alone(nn, kGroupAlone<R>);
   }
 
   void setup(Hierarchy* h, const R* boxsize, const R* boxcenter, R beta, R damping, int nit,

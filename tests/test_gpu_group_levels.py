@@ -23,3 +23,11 @@ def check_group(shape, count, dtype, mixed):
 @pytest.mark.parametrize('shape,count', [(shape, count) for shape, counts in SHAPES for count in counts])
 def test_equals_alone(shape, count, dtype, mixed):
     check_group(shape, count, dtype, mixed)
+
+
+@pytest.mark.parametrize('dtype,mixed', [('f4', False), ('f8', False), ('f8', True)])
+@pytest.mark.parametrize('shape', [(80, 96, 112), (96, 112, 116), (96, 112, 120), (96, 128, 120), (96, 128, 124)])
+def test_finest_level_equals_alone(shape, dtype, mixed):
+    """Meshes of 860 160 cells to 1 523 712, on both sides of where the finest level of a group is no longer relaxed in
+    one launch for it (1.25 million cells in FP64, 1.5 in FP32)."""
+    check_group(shape, 2, dtype, mixed)
