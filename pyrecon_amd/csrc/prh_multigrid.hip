@@ -1967,37 +1967,45 @@ __device__ __forceinline__ float divided(float a, float d, float y) {
   return fmaf(fmaf(-q1, d, a), y, q1);
 }
 
-// XL consecutive x of one (y, z) of a level in LDS, for one thread: offsets of the neighbours and the
+// XL consecutive cells along an axis of a level in LDS, for one thread: offsets of the neighbours and the
 // operator's coefficients, worked out once per visit of the level (five sweeps, and the residual on the
-// way down).  The x neighbourhood moves through registers, 11.5 LDS reads a cell for XL = 4.
-template <typename R, int XL>
+// way down).  The neighbourhood along the axis moves through registers, 11.5 LDS reads a cell for XL = 4.
+// A: the axis of the column; the other two in their order are its y and z here (for A = 0 they are those).
+template <typename R, int XL, int A>
 struct CoarseColumn {
+  static constexpr int P = A == 0 ? 1 : 0, Q = A == 2 ? 1 : 2;
   int live;                  // cells of this column, 0 for a thread without one
-  int c, yp, ym, zp, zm, s0; // (y, z) offset in a plane, those of its neighbours, plane size
+  int c, yp, ym, zp, zm, s0; // (y, z) offset in a plane, those of its neighbours, distance of the planes
   int ix, x0, xm, xp;        // first x; offsets of its plane, the one before it and the one after the last
   R py, pz, pypz, px0;
   R g[XL], y[XL];            // g and 1 / d: the divisions; the rest is a few products
 
   __device__ __forceinline__ void set(const LevelGeom<R>& G, int t) {
-    const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
-    s0 = n1 * n2;
+    const int stride[3] = {G.n[1] * G.n[2], G.n[2], 1};
+    const int n0 = G.n[A], n1 = G.n[P], n2 = G.n[Q], s1 = stride[P], s2 = stride[Q];
+    s0 = stride[A];
     int group, iy, iz;
     unflatten(t, n1, n2, group, iy, iz);
     x0 = group * XL;
     live = x0 < n0 ? min(XL, n0 - x0) : 0;
     if (!live) return;
-    c = iy * n2 + iz;
-    yp = (iy + 1 == n1 ? 0 : iy + 1) * n2 + iz;
-    ym = (iy == 0 ? n1 - 1 : iy - 1) * n2 + iz;
-    zp = (iz + 1 == n2 ? 0 : iz + 1) - iz;
-    zm = (iz == 0 ? n2 - 1 : iz - 1) - iz;
+    c = iy * s1 + iz * s2;
+    yp = (iy + 1 == n1 ? 0 : iy + 1) * s1 + iz * s2;
+    ym = (iy == 0 ? n1 - 1 : iy - 1) * s1 + iz * s2;
+    zp = ((iz + 1 == n2 ? 0 : iz + 1) - iz) * s2;
+    zm = ((iz == 0 ? n2 - 1 : iz - 1) - iz) * s2;
     xm = (x0 == 0 ? n0 - 1 : x0 - 1) * s0;
     xp = (x0 + live == n0 ? 0 : x0 + live) * s0;
     x0 *= s0;
 #pragma unroll
     for (int u = 0; u < XL; u++) {
-      const Coef<R> k = cell_coef(G, group * XL + u, iy, iz);
-      if (u == 0) px0 = k.px, py = k.py, pz = k.pz;
+      const int at = group * XL + u;
+      const Coef<R> k = cell_coef(G, A == 0 ? at : iy, A == 1 ? at : A == 0 ? iy : iz, A == 2 ? at : iz);
+      if (u == 0) {
+        px0 = A == 0 ? k.px : A == 1 ? k.py : k.pz;
+        py = A == 0 ? k.py : k.px;
+        pz = A == 2 ? k.py : k.pz;
+      }
       g[u] = k.g;
       y[u] = reciprocal(R(2) * (k.cx + k.cy + k.cz));
     }
@@ -2041,17 +2049,38 @@ struct CoarseColumn {
     for (int u = 0; u < XL; u++) {
       if (u >= live) break;
       if (!zero_in) n = plane(in + (u + 1 == live ? xp : x0 + (u + 1) * s0), u + 1 < XL);
-      const R px = local ? static_cast<R>(ix + u) + G.org[0] : px0;
-      const R cx = G.ih2[0] + g[u] * px * px, cy = G.ih2[1] + g[u] * py * py, cz = G.ih2[2] + g[u] * pz * pz;
+      // the mesh's x, y and z of the column's own: h's neighbours and the position
+      const R pr = local ? static_cast<R>(ix + u) + G.org[A] : px0;
+      const R px = A == 0 ? pr : py, pY = A == 1 ? pr : A == 0 ? py : pz, pZ = A == 2 ? pr : pz;
+      const R pYZ = A == 0 ? pypz : pY * pZ;
+      Hood<R> h;
+      h.c = b.c;
+      if constexpr (A == 0) {
+        h.xp = n.c, h.xm = a.c, h.yp = b.yp, h.ym = b.ym, h.zp = b.zp, h.zm = b.zm;
+        h.xpyp = n.yp, h.xmym = a.ym, h.xmyp = a.yp, h.xpym = n.ym;
+        h.xpzp = n.zp, h.xmzm = a.zm, h.xmzp = a.zp, h.xpzm = n.zm;
+        h.ypzp = b.pp, h.ymzm = b.mm, h.ymzp = b.mp, h.ypzm = b.pm;
+      } else if constexpr (A == 1) {
+        h.yp = n.c, h.ym = a.c, h.xp = b.yp, h.xm = b.ym, h.zp = b.zp, h.zm = b.zm;
+        h.xpyp = n.yp, h.xmym = a.ym, h.xmyp = n.ym, h.xpym = a.yp;
+        h.xpzp = b.pp, h.xmzm = b.mm, h.xmzp = b.mp, h.xpzm = b.pm;
+        h.ypzp = n.zp, h.ymzm = a.zm, h.ymzp = a.zp, h.ypzm = n.zm;
+      } else {
+        h.zp = n.c, h.zm = a.c, h.xp = b.yp, h.xm = b.ym, h.yp = b.zp, h.ym = b.zm;
+        h.xpyp = b.pp, h.xmym = b.mm, h.xmyp = b.mp, h.xpym = b.pm;
+        h.xpzp = n.yp, h.xmzm = a.ym, h.xmzp = n.ym, h.xpzm = a.yp;
+        h.ypzp = n.zp, h.ymzm = a.zm, h.ymzp = n.zm, h.ypzm = a.zp;
+      }
+      const R cx = G.ih2[0] + g[u] * px * px, cy = G.ih2[1] + g[u] * pY * pY, cz = G.ih2[2] + g[u] * pZ * pZ;
       const R d = R(2) * (cx + cy + cz);
-      const R t0 = cx * (n.c + a.c);
-      const R t1 = cy * (b.yp + b.ym);
-      const R t2 = cz * (b.zp + b.zm);
+      const R t0 = cx * (h.xp + h.xm);
+      const R t1 = cy * (h.yp + h.ym);
+      const R t2 = cz * (h.zp + h.zm);
       const R t3 = g[u] / R(2) *
-                   (px * py * (n.yp + a.ym - a.yp - n.ym) + px * pz * (n.zp + a.zm - a.zp - n.zm) +
-                    pypz * (b.pp + b.mm - b.mp - b.pm));
+                   (px * pY * (h.xpyp + h.xmym - h.xmyp - h.xpym) + px * pZ * (h.xpzp + h.xmzm - h.xmzp - h.xpzm) +
+                    pYZ * (h.ypzp + h.ymzm - h.ymzp - h.ypzm));
       R drift = R(0);
-      if (local) drift = g[u] * (px * (n.c - a.c) + py * (b.yp - b.ym) + pz * (b.zp - b.zm));
+      if (local) drift = g[u] * (px * (h.xp - h.xm) + pY * (h.yp - h.ym) + pZ * (h.zp - h.zm));
       const int at = x0 + u * s0 + c;
       const R fv = src[at];
       if constexpr (RESIDUAL) {
@@ -2073,11 +2102,12 @@ struct CoarseColumn {
 // One visit of a level: `niter` sweeps, the iterate moving between cur and alt, then the residual into
 // the spare of the two if `residual`.  HELD: every column has a thread of its own, which keeps the
 // coefficients; otherwise the threads go round and work them out again.
-template <typename R, int XL, bool HELD>
+template <typename R, int XL, bool HELD, int A = 0>
 __device__ void coarse_visit(const LevelGeom<R>& G, R* cur, R* alt, const R* src, int niter, R omega, R keep,
                              bool zero_start, bool residual) {
-  CoarseColumn<R, XL> C;
-  const int columns = G.n[1] * G.n[2] * ((G.n[0] + XL - 1) / XL);
+  using Column = CoarseColumn<R, XL, A>;
+  Column C;
+  const int columns = G.n[Column::P] * G.n[Column::Q] * ((G.n[A] + XL - 1) / XL);
   if (HELD) C.set(G, threadIdx.x);
   for (int it = 0; it < niter; it++) {
     for (int t = threadIdx.x; t < columns; t += kCoarseThreads) {
@@ -2098,7 +2128,10 @@ __device__ void coarse_visit(const LevelGeom<R>& G, R* cur, R* alt, const R* src
   }
 }
 
-// The longest columns that still give every thread its own: small levels take one cell a thread.
+// The shortest columns that give every column a thread: small levels take one cell a thread.  Four cells
+// along x leave some columns without a thread where planes are a large share of the threads; along y or z
+// they fit (10 x 80 x 5, the last level of 40 x 320 x 20: a solve takes 1.85 ms in FP64, 2.11 with the
+// coefficients worked out in every sweep; 3 x 32 x 40 of 24 x 256 x 320 3.66 and 4.28).
 template <typename R>
 __device__ __forceinline__ void coarse_level(const LevelGeom<R>& G, R* cur, R* alt, const R* src, int niter,
                                              R omega, R keep, bool zero_start, bool residual) {
@@ -2109,6 +2142,10 @@ __device__ __forceinline__ void coarse_level(const LevelGeom<R>& G, R* cur, R* a
     coarse_visit<R, 2, true>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
   else if (plane * ((G.n[0] + 3) / 4) <= kCoarseThreads)
     coarse_visit<R, 4, true>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
+  else if (G.n[0] * G.n[2] * ((G.n[1] + 3) / 4) <= kCoarseThreads)
+    coarse_visit<R, 4, true, 1>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
+  else if (G.n[0] * G.n[1] * ((G.n[2] + 3) / 4) <= kCoarseThreads)
+    coarse_visit<R, 4, true, 2>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
   else
     coarse_visit<R, 2, false>(G, cur, alt, src, niter, omega, keep, zero_start, residual);
 }
