@@ -1984,10 +1984,15 @@ struct CoarseColumn {
     const int stride[3] = {G.n[1] * G.n[2], G.n[2], 1};
     const int n0 = G.n[A], n1 = G.n[P], n2 = G.n[Q], s1 = stride[P], s2 = stride[Q];
     s0 = stride[A];
+    // columns in the order of memory, neighbouring threads on neighbouring banks (40 x 320 x 20 in FP32 1.26 ms
+    // a solve, 1.45 with group the slowest along every axis)
+    const int groups = (n0 + XL - 1) / XL;
     int group, iy, iz;
-    unflatten(t, n1, n2, group, iy, iz);
+    if constexpr (A == 0) unflatten(t, n1, n2, group, iy, iz);
+    if constexpr (A == 1) unflatten(t, groups, n2, iy, group, iz);
+    if constexpr (A == 2) unflatten(t, n2, groups, iy, iz, group);
     x0 = group * XL;
-    live = x0 < n0 ? min(XL, n0 - x0) : 0;
+    live = t < groups * n1 * n2 ? min(XL, n0 - x0) : 0;
     if (!live) return;
     c = iy * s1 + iz * s2;
     yp = (iy + 1 == n1 ? 0 : iy + 1) * s1 + iz * s2;
@@ -2130,8 +2135,9 @@ __device__ void coarse_visit(const LevelGeom<R>& G, R* cur, R* alt, const R* src
 
 // The shortest columns that give every column a thread: small levels take one cell a thread.  Four cells
 // along x leave some columns without a thread where planes are a large share of the threads; along y or z
-// they fit (10 x 80 x 5, the last level of 40 x 320 x 20: a solve takes 1.85 ms in FP64, 2.11 with the
-// coefficients worked out in every sweep; 3 x 32 x 40 of 24 x 256 x 320 3.66 and 4.28).
+// they fit (10 x 80 x 5, the last level of 40 x 320 x 20: a solve takes 1.74 ms in FP64, 2.11 with the
+// coefficients worked out in every sweep; 3 x 32 x 40 of 24 x 256 x 320 3.65 and 4.28).  Not five cells along
+// x: coarse_visit is inlined no more with another form beside these.
 template <typename R>
 __device__ __forceinline__ void coarse_level(const LevelGeom<R>& G, R* cur, R* alt, const R* src, int niter,
                                              R omega, R keep, bool zero_start, bool residual) {
