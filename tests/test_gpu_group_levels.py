@@ -31,3 +31,10 @@ def test_finest_level_equals_alone(shape, dtype, mixed):
     """Meshes of 860 160 cells to 1 523 712, on both sides of where the finest level of a group is no longer relaxed in
     one launch for it (1.25 million cells in FP64, 1.5 in FP32)."""
     check_group(shape, 2, dtype, mixed)
+
+
+@pytest.mark.parametrize('dtype,mixed', [('f4', False), ('f8', False), ('f8', True)])
+@pytest.mark.parametrize('shape', [(16, 96, 192), (32, 128, 120), (32, 128, 128)])
+def test_residual_restriction_equals_alone(shape, dtype, mixed):
+    """Levels in 64-wide tiles and not, below and above the size from which a group's residuals are restricted at once."""
+    check_group(shape, 2, dtype, mixed)
